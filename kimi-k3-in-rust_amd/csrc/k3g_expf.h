@@ -1,4 +1,5 @@
-/* k3g_expf.h - the engine's float expf, bit for bit, for device and host code.
+/* k3g_expf.h - the engine's float expf, bit for bit, and a float tanh, for device and host
+ * code.
  *
  * The engine's router and SiTU/SwiGLU call the C library's expf (src/core/k3_ops.c:105,
  * :446-458): glibc 2.35 on the x86-64 hosts it runs on. That expf is not correctly rounded
@@ -114,6 +115,51 @@ K3X_FN float k3x_expf(float x)
     y = fma(z, r2, y);
     y = y * s;
     return (float)y;
+}
+
+/* tanhf, correctly rounded but for a vanishing set of inputs next to a midpoint of two floats:
+ * tanh x = E / (E + 2) with E = e^(2 x) - 1 in double,
+ *
+ *   2 x = n ln 2 + r, |r| <= ln 2 / 2 (two-part reduction),  E = 2^n (e^r - 1) + (2^n - 1)
+ *
+ * e^r - 1 from its Taylor series to r^12 (the next term is below 2^-53 of it), so small
+ * arguments lose nothing to cancellation, and the quotient from a reciprocal seed of at least
+ * 20 bits, one Newton step and one correction of the quotient. In all within 2^-50 of tanh x:
+ * about one input in 2^25 can round to the other neighbour. From |x| = 20 on the float is 1. */
+K3X_FN float k3x_tanhf(float x)
+{
+    double a = fabs((double)x);
+    a = a > 20.0 ? 20.0 : a;                          /* NaN stays */
+    const double y = a + a;
+    const double shift = 0x1.8p+52;
+    const double nd = fma(y, 0x1.71547652b82fep+0, shift) - shift;
+    double r = fma(nd, -0x1.62e42fefa39efp-1, y);
+    r = fma(nd, -0x1.abc9e3b39803fp-56, r);
+    double p = 1.0 / 479001600.0;
+    p = fma(p, r, 1.0 / 39916800.0);
+    p = fma(p, r, 1.0 / 3628800.0);
+    p = fma(p, r, 1.0 / 362880.0);
+    p = fma(p, r, 1.0 / 40320.0);
+    p = fma(p, r, 1.0 / 5040.0);
+    p = fma(p, r, 1.0 / 720.0);
+    p = fma(p, r, 1.0 / 120.0);
+    p = fma(p, r, 1.0 / 24.0);
+    p = fma(p, r, 1.0 / 6.0);
+    p = fma(p, r, 0.5);
+    p = fma(p * r, r, r);                             /* e^r - 1 */
+    /* nd is 0 .. 58 (NaN: any n, p is NaN) */
+    const double s = k3x_asdouble((uint64_t)(1023 + (int)(nd == nd ? nd : 0.0)) << 52);
+    const double e = fma(s, p, s - 1.0), d = e + 2.0;
+#if defined(__HIP_DEVICE_COMPILE__)
+    double q = __builtin_amdgcn_rcp(d);
+#else
+    double q = (double)(1.0f / (float)d);
+#endif
+    q = fma(q, fma(-d, q, 1.0), q);
+    double t = e * q;
+    t = fma(fma(-t, d, e), q, t);
+    const float f = (float)t;
+    return __builtin_copysignf(f, x);
 }
 
 #endif

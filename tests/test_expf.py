@@ -60,3 +60,19 @@ def test_correct_rounding_is_not_the_engine():
     xs = np.random.default_rng(5).standard_normal(20000).astype(np.float32)
     diff = sum(np.float32(libm.expf(C.c_float(v))) != np.float32(math.exp(float(v))) for v in xs)
     assert diff > 0
+
+
+def test_tanhf_is_correctly_rounded(tmp_path):
+    """The device's float tanh (the SiTU caps, src/core/k3_ops.c:110-123) compiled for the host:
+    over a 2^-8 sample of all floats and every float of the ranges where its parts change
+    over, no result more than a float step from the rounded double tanh. Its error bound,
+    2^-50, lets about one input in 2^25 round the other way: at most 32 of the 54 million."""
+    if not shutil.which("gcc"):
+        pytest.skip("no host compiler")
+    exe = tmp_path / "tanhf_audit"
+    subprocess.run(["gcc", "-O2", "-std=gnu99", "-fopenmp", "-ffp-contract=off", "-I", CSRC,
+                    os.path.join(HOST, "tanhf_audit.c"), "-o", str(exe), "-lm"], check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout
+    n, diff = (int(r.stdout.split()[i]) for i in (1, 3))
+    assert n > 50_000_000 and diff <= 32, r.stdout
