@@ -403,8 +403,8 @@ int  k3g_ctx_paths(K3gCtx *ctx, int clear);
 
 /* Routed experts of calls beyond the fused decode kernel on the FP4 x FP8 matrix cores
  * (v_mfma_scale_f32_16x16x128_f8f6f4): MXFP4 weights as stored, x and the activation h
- * quantised to MXFP8 (OCP MX: E4M3, an E8M0 scale per 32 values). Off by default (the
- * bf16 matrix cores, activations exact to 2^-17). The shared expert stays bf16. No
+ * quantised to MXFP8 (OCP MX: E4M3, an E8M0 scale per 32 values). Off by default
+ * (activations in pieces that hold about 20 bits). The shared expert stays bf16. No
  * reference counterpart. */
 void k3g_ctx_set_fp8(K3gCtx *ctx, int on);
 
@@ -413,7 +413,8 @@ void k3g_ctx_set_fp8(K3gCtx *ctx, int on);
  * (100 MHz counter), then the top-k ticket's stamps after its wait, after its selection
  * and inside the selection. Calls on the grouped GEMMs write 4 uint64 per workgroup of
  * the routed gate/up launch (8 * 4 ceil(tiles / 32) * ceil(inter / 128) workgroups, tiles =
- * ceil(T topk / 128) + min(n_experts, T topk)), then of the routed down launch: wave 0's
+ * ceil(T topk / 128) + min(n_experts, T topk); of a tile of more than 64 pairs the first
+ * 64), then of every second workgroup of the routed down launch (one per 512 rows): wave 0's
  * start and end, column tile << 32 | feature tile, XCC << 32 | HW_ID. NULL turns it off.
  * No reference counterpart. */
 void k3g_ctx_set_trace(K3gCtx *ctx, void *dev_buf);
@@ -458,9 +459,9 @@ int  k3g_expert_gemv(K3gCtx *ctx, const K3gLayer *L, const float *x, int T,
                      const int32_t *idx, float *contrib, void *stream);
 
 /* The same contrib rows as grouped GEMMs over 128-pair column tiles: gate/up with the
- * activation fused, then down, bf16 matrix cores (weights decoded from MXFP4 exactly,
- * x as two bf16 pieces, h as a bf16 piece plus its MXFP8 remainder on the scaled FP8
- * matrix cores, fp32 accumulation; rel-L2 about 4e-5) or, for _f8f6f4, the
+ * activation fused, then down (weights exact, x and h as four FP6 pieces each on the scaled
+ * FP4 x FP6 matrix cores, or x as it is on the bf16 ones when every value is a bf16 value;
+ * fp32 accumulation; rel-L2 about 1.5e-6) or, for _f8f6f4, the
  * scaled FP4 x FP8 ones with x and h quantised to MXFP8. Experts in the tiled layout
  * (K3G_EXPERT_MXFP4_TILED), hidden and inter multiples of 32. */
 int  k3g_grouped_gemm_bf16(K3gCtx *ctx, const K3gLayer *L, const float *x, int T,

@@ -135,10 +135,10 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     const size_t o_daq16 = carve(&at, lat ? (L / 32 + 1) * 1024 : 16);
     const size_t o_dupart = carve(&at, lat ? (size_t)K3G_KS_LU * T4 * d * 4 : 16);
     /* the grouped GEMMs' activation pieces and column tiles */
-    const size_t d128 = (d + 127) / 128 * 128, I128 = (I + 127) / 128 * 128;
+    const size_t d128 = (d + 127) / 128 * 128;
     const size_t SI128 = (SI + 127) / 128 * 128;
     const size_t maxt = (P + 127) / 128 + E;
-    const size_t o_xb = carve(&at, 2 * T * d128 * 2), o_hb = carve(&at, 2 * P * I128 * 2);
+    const size_t o_xb = carve(&at, 2 * T * d128 * 2);
     const size_t o_hsb = carve(&at, 2 * T * (SI128 ? SI128 : 128) * 2);
     /* the dense GEMMs' K-slice sums when few columns leave the GPU idle: the shared
      * expert's gate/up and down, the latent down and up projections */
@@ -175,6 +175,9 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     const size_t L512 = (L + 511) / 512 * 512, q512 = d512 > L512 ? d512 : L512;
     const size_t o_xq8b = carve(&at, T * q512 + T * q512 / 32);
     const size_t o_hq8b = carve(&at, P * I512 + P * I512 / 32);
+    /* the routed experts' input and h as FP6 pieces (k3g_gemm6.hip) */
+    const size_t o_xr = carve(&at, T * (nQd > nQL ? nQd : nQL) * K3G_P6_QUAD);
+    const size_t o_hr = carve(&at, P * nQi * K3G_P6_QUAD);
     /* two banks of counters, one per call in turn; each a multiple of 256 bytes */
     /* the larger of the latent layer's geometry and the plain one (a layer without the
      * latent projections may run on a context sized for them) */
@@ -224,7 +227,6 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     c->dupart = (float *)(b + o_dupart);
     c->sync = (int *)(b + o_sync);
     c->xb = (uint16_t *)(b + o_xb);
-    c->hb = (uint16_t *)(b + o_hb);
     c->hsb = (uint16_t *)(b + o_hsb);
     c->zb = (uint16_t *)(b + o_zb);
     c->zflag = (int32_t *)(b + o_zflag);
@@ -240,6 +242,8 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     c->max_tiles = (int)maxt;
     c->xq8b = (uint8_t *)(b + o_xq8b);
     c->hq8b = (uint8_t *)(b + o_hq8b);
+    c->xr = (uint8_t *)(b + o_xr);
+    c->hr = (uint8_t *)(b + o_hr);
     c->fused = 1;
     if (hipMemset(c->ws, 0, at) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
         hipFree(c->ws);
@@ -403,7 +407,6 @@ static int dense_gemm(K3gCtx *c, const void *W, int rows, int K, const uint16_t 
     K3kGemm s;
     memset(&s, 0, sizeof s);
     s.mode = 1;
-    s.afmt = 1;
     s.rows = rows;
     s.K = K;
     s.ldb = ldb;
@@ -427,7 +430,7 @@ static int dense_gemm(K3gCtx *c, const void *W, int rows, int K, const uint16_t 
  * the routed experts' per-pair rows in contrib. */
 static int gemm_body(K3gCtx *c, const K3gLayer *L, const float *x, int T,
                      const int32_t *idx, const float *wt, float *out, float *contrib, int fp8,
-                     int full, int shared_side, hipStream_t st);
+                     int full, int routed, hipStream_t st);
 
 static int experts_gemm(K3gCtx *c, const K3gLayer *L, const float *x, int T,
                         const int32_t *idx, const float *wt, float *out, float *contrib,
@@ -451,7 +454,6 @@ static int shared_expert(K3gCtx *c, const K3gLayer *L, int T, float *part, hipSt
     K3kGemm s;
     memset(&s, 0, sizeof s);
     s.mode = 0;
-    s.afmt = 1;
     s.rows = SI;
     s.K = d;
     s.ldb = d128;
@@ -493,137 +495,161 @@ static int shared_expert(K3gCtx *c, const K3gLayer *L, int T, float *part, hipSt
     return rc;
 }
 
-/* x's two bf16 pieces (the piece-1 flag cleared before) and, for the FP4 x FP8 routed
- * experts on x itself, its MXFP8 copy. */
+/* the routed experts' input z [T][n] as FP6 pieces (only when *run_flag, if given, is set), or
+ * MXFP8 for the FP4 x FP8 ones */
+static int routed_input(K3gCtx *c, const float *z, int T, int n, int fp8,
+                        const int32_t *run_flag, hipStream_t st)
+{
+    return fp8 ? k3k_xq8(z, T, n, r512(n), c->xq8b, c->xq8b + (size_t)T * r512(n), st)
+               : k3k_x6(z, T, n, c->xr, run_flag, st);
+}
+
+/* x's two bf16 pieces (the piece-1 flag cleared before; the shared expert, the latent down and
+ * the router's flag) and, for routed experts on x itself, their input: FP6 pieces or MXFP8. */
 static int gemm_pieces(K3gCtx *c, const K3gLayer *L, const float *x, int T, int fp8,
                        hipStream_t st)
 {
-    const int d = L->hidden, d128 = r128(d), d512 = r512(d);
+    const int d = L->hidden, d128 = r128(d);
     int rc = 0;
     k3g_stage_begin(c, K3G_ST_PIECES, st);
     rc |= k3k_xpieces(x, T, d, d128, c->xb, (long long)T * d128, c->xflag, st);
-    if (fp8 && !L->down)
-        rc |= k3k_xq8(x, T, d, d512, c->xq8b, c->xq8b + (size_t)T * d512, st);
+    if (!L->down) rc |= routed_input(c, x, T, d, fp8, c->xflag, st);
     k3g_stage_end(c, K3G_ST_PIECES, st);
+    return rc;
+}
+
+/* The routed experts on the column tiles, x or z -> h -> contrib rows (k3g_gemm6.h). max_np:
+ * no expert has more pairs than this */
+static int routed_f6(K3gCtx *c, const K3gLayer *L, int lat, int max_tiles, int max_np,
+                     float *contrib, hipStream_t st)
+{
+    const int I = L->inter;
+    int rc = 0;
+    K3kGemm6 g;
+    memset(&g, 0, sizeof g);
+    g.mode = 0;
+    g.rows = I;
+    g.K = lat;
+    g.eq = L->experts;
+    g.b = c->xr;
+    if (!L->down) {                      /* routed experts on x itself */
+        g.xb = c->xb;
+        g.ldb = r128(L->hidden);
+        g.lo_flag = c->xflag;
+    }
+    g.perm = c->perm;
+    g.topk = L->topk;
+    g.tiles = c->tiles;
+    g.ntiles = c->ntiles;
+    g.max_tiles = max_tiles;
+    g.halves = max_np > 64;
+    g.h = c->hr;
+    g.b1 = L->act_b1;
+    g.b2 = L->act_b2;
+    g.trace = c->trace;
+    g.trace_step = 1;
+    k3g_stage_begin(c, K3G_ST_GATEUP, st);
+    rc |= k3k_gemm6(&g, st);
+    k3g_stage_end(c, K3G_ST_GATEUP, st);
+    /* the down launch's stamps follow the gate/up launch's */
+    if (g.trace)
+        g.trace += 4 * 8 * (size_t)K3G_TILE_ROUNDS(max_tiles) * (size_t)((I + 127) / 128);
+    g.mode = 1;
+    g.rows = lat;
+    g.K = I;
+    g.b = c->hr;
+    g.xb = NULL;
+    g.h = NULL;
+    g.out = contrib;
+    g.ldo = lat;
+    g.trace_step = 2;
+    k3g_stage_begin(c, K3G_ST_DOWN, st);
+    rc |= k3k_gemm6(&g, st);
+    k3g_stage_end(c, K3G_ST_DOWN, st);
+    return rc;
+}
+
+/* the same with x and h in MXFP8 on the FP4 x FP8 ones */
+static int routed_f8(K3gCtx *c, const K3gLayer *L, int T, int lat, int max_tiles,
+                     float *contrib, hipStream_t st)
+{
+    const int I = L->inter, P = T * L->topk, l512 = r512(lat), I512 = r512(c->inter);
+    int rc = 0;
+    K3kGemm g;
+    memset(&g, 0, sizeof g);
+    g.mode = 0;
+    g.rows = I;
+    g.K = lat;
+    g.ldb = l512;
+    g.eq = L->experts;
+    g.perm = c->perm;
+    g.topk = L->topk;
+    g.tiles = c->tiles;
+    g.ntiles = c->ntiles;
+    g.max_tiles = max_tiles;
+    g.b1 = L->act_b1;
+    g.b2 = L->act_b2;
+    g.nft = (I + 255) / 256;
+    g.bq = c->xq8b;
+    g.bs = c->xq8b + (size_t)T * l512;
+    g.hq = c->hq8b;
+    g.hs = c->hq8b + (size_t)P * I512;
+    g.ldhq = I512;
+    k3g_stage_begin(c, K3G_ST_GATEUP, st);
+    rc |= k3k_gemm_f8(&g, st);
+    k3g_stage_end(c, K3G_ST_GATEUP, st);
+    g.mode = 1;
+    g.rows = lat;
+    g.K = I;
+    g.ldb = I512;
+    g.bq = c->hq8b;
+    g.bs = c->hq8b + (size_t)P * I512;
+    g.hq = NULL;
+    g.hs = NULL;
+    g.out = contrib;
+    g.ldo = lat;
+    g.scatter = 1;
+    g.nft = (lat + 511) / 512;
+    k3g_stage_begin(c, K3G_ST_DOWN, st);
+    rc |= k3k_gemm_f8(&g, st);
+    k3g_stage_end(c, K3G_ST_DOWN, st);
     return rc;
 }
 
 /* The grouped GEMMs after the dispatch (column tiles built, x's piece-1 flag cleared):
  * x pieces, [latent down], the shared expert, the routed gate/up and down, [combine,
- * latent up, + shared]. shared_side: x's pieces are already made and the shared expert
+ * latent up, + shared]. routed: called by k3g_moe after its own router (no token has an expert
+ * twice, so no expert has more than T pairs); x's pieces are already made and the shared expert
  * runs on the side stream (ev_shared marks its end; the combine waits for it). */
 static int gemm_body(K3gCtx *c, const K3gLayer *L, const float *x, int T,
                      const int32_t *idx, const float *wt, float *out, float *contrib, int fp8,
-                     int full, int shared_side, hipStream_t st)
+                     int full, int routed, hipStream_t st)
 {
-    const int d = L->hidden, E = L->n_experts, k = L->topk, I = L->inter;
+    const int d = L->hidden, E = L->n_experts, k = L->topk;
     const int SI = full ? L->shared_inter : 0, P = T * k;
-    const int d128 = r128(d), I128 = r128(c->inter);
     const int lat = L->latent > 0 ? L->latent : d, lat128 = r128(lat);
     const int projected = L->down != NULL;
     int rc = 0;
-    const int I512 = r512(c->inter);
-    if (!shared_side) rc |= gemm_pieces(c, L, x, T, fp8, st);
-    /* the routed experts' input: x, or its latent projection z = down x as two bf16
-     * pieces (piece 1 always taken) */
-    const uint16_t *rb = c->xb;
-    int ldr = d128;
-    const int32_t *rflag = c->xflag;
+    if (!routed) rc |= gemm_pieces(c, L, x, T, fp8, st);
+    /* the routed experts' input: x, or its latent projection z = down x */
     if (projected) {
         k3g_stage_begin(c, K3G_ST_LATENT, st);
-        rc |= dense_gemm(c, L->down, lat, d, c->xb, d128, c->xflag, T, c->z, lat, st);
-        rc |= k3k_xpieces(c->z, T, lat, lat128, c->zb, (long long)T * lat128, c->zflag, st);
-        if (fp8) {
-            const int l512 = r512(lat);
-            rc |= k3k_xq8(c->z, T, lat, l512, c->xq8b, c->xq8b + (size_t)T * l512, st);
-        }
+        rc |= dense_gemm(c, L->down, lat, d, c->xb, r128(d), c->xflag, T, c->z, lat, st);
+        rc |= routed_input(c, c->z, T, lat, fp8, NULL, st);
         k3g_stage_end(c, K3G_ST_LATENT, st);
-        rb = c->zb;
-        ldr = lat128;
-        rflag = NULL;
     }
-
-    K3kGemm g;
-    memset(&g, 0, sizeof g);
-    g.mode = 0;
-    g.afmt = 0;
-    g.rows = I;
-    g.K = lat;
-    g.ldb = ldr;
-    g.eq = L->experts;
-    g.b = rb;
-    g.bpiece = (long long)T * ldr;
-    g.perm = c->perm;
-    g.topk = k;
-    g.tiles = c->tiles;
-    g.ntiles = c->ntiles;
-    g.max_tiles = (P + 127) / 128 + (E < P ? E : P);
-    g.npieces = 2;
-    g.lo_flag = rflag;
-    g.h = c->hb;
-    g.hpiece = (long long)P * I128;
-    g.ldh = I128;
-    g.b1 = L->act_b1;
-    g.b2 = L->act_b2;
-    g.nft = (I + 255) / 256;
-
-    if (SI > 0 && !shared_side) rc |= shared_expert(c, L, T, c->kpart, st);
+    const int max_tiles = (P + 127) / 128 + (E < P ? E : P);
+    if (SI > 0 && !routed) rc |= shared_expert(c, L, T, c->kpart, st);
     /* routed experts last, after any copies they wait for (the shared expert above
      * overlaps them) */
     if (c->routed_wait) {
         if (hipStreamWaitEvent(st, c->routed_wait, 0) != hipSuccess) rc = -1;
         c->routed_wait = NULL;
     }
-    if (fp8) {
-        const int l512 = r512(lat);
-        g.bq = c->xq8b;
-        g.bs = c->xq8b + (size_t)T * l512;
-        g.ldb = l512;
-        g.hq = c->hq8b;
-        g.hs = c->hq8b + (size_t)P * I512;
-        g.ldhq = I512;
-    } else {
-        /* h leaves gate/up as bf16 plus its MXFP8 remainder */
-        g.hmix = 1;
-        g.hq = c->hq8b;
-        g.hs = c->hq8b + (size_t)P * I512;
-        g.ldhq = I512;
-    }
-    k3g_stage_begin(c, K3G_ST_GATEUP, st);
-    g.trace = fp8 ? NULL : c->trace;
-    rc |= fp8 ? k3k_gemm_f8(&g, st) : k3k_gemm(&g, st);
-    k3g_stage_end(c, K3G_ST_GATEUP, st);
-    /* the down launch's stamps follow the widest gate/up launch's (4-wave workgroups) */
-    if (g.trace) g.trace += 4 * 8 * (size_t)K3G_TILE_ROUNDS(g.max_tiles) * (size_t)((I + 127) / 128);
+    rc |= fp8 ? routed_f8(c, L, T, lat, max_tiles, contrib, st)
+              : routed_f6(c, L, lat, max_tiles, routed ? T : P, contrib, st);
 
-    g.mode = 1;
-    g.rows = lat;
-    g.K = I;
-    g.ldb = I128;
-    g.b = c->hb;
-    g.bpiece = (long long)P * I128;
-    g.lo_flag = NULL;
-    g.h = NULL;
-    g.out = contrib;
-    g.ldo = lat;
-    g.scatter = 1;
-    g.nft = (lat + 511) / 512;
-    if (fp8) {
-        g.bq = c->hq8b;
-        g.bs = c->hq8b + (size_t)P * I512;
-        g.ldb = I512;
-        g.hq = NULL;
-        g.hs = NULL;
-    } else {
-        g.npieces = 1;
-        g.bq = c->hq8b;
-        g.bs = c->hq8b + (size_t)P * I512;
-    }
-    k3g_stage_begin(c, K3G_ST_DOWN, st);
-    rc |= fp8 ? k3k_gemm_f8(&g, st) : k3k_gemm(&g, st);
-    k3g_stage_end(c, K3G_ST_DOWN, st);
-
-    if (SI > 0 && shared_side && hipStreamWaitEvent(st, c->ev_shared, 0) != hipSuccess) rc = -1;
+    if (SI > 0 && routed && hipStreamWaitEvent(st, c->ev_shared, 0) != hipSuccess) rc = -1;
     if (full && !projected && !L->up && !L->latent_norm) {
         k3g_stage_begin(c, K3G_ST_COMBINE, st);
         rc |= k3k_combine(contrib, idx, wt, T, k, d, SI > 0 ? c->sh_out : NULL, out, st);

@@ -1,5 +1,7 @@
-/* k3g_gemm.hip - the expert products for many tokens (prefill, batched decode) as grouped
- * GEMMs on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16, fp32 accumulation).
+/* k3g_gemm.hip - the GEMMs for many tokens (prefill, batched decode): the routed experts as
+ * grouped GEMMs (k3g_gemm6.h on FP6 pieces; gate/up of bf16-valued x and the FP4 x FP8 variant
+ * here), and the dense ones (shared expert, latent projections) on the bf16 matrix cores
+ * (v_mfma_f32_16x16x32_bf16, fp32 accumulation).
  *
  * The engine computes, per (token, slot) pair, three MXFP4 GEMVs per expert in its
  * moe_prefill_chunk loop (src/core/k3_ops.c:668-808); here the pairs are grouped by
@@ -11,14 +13,13 @@
  *
  * The shared expert is the same GEMM over all tokens with a dense column list.
  *
- * Work unit: one workgroup = one (column tile of up to 128 pairs, feature tile) of one
- * expert. Wave w owns 4 row groups of 16 weight rows (mode 0: 32 gate rows and the 32 up
- * rows of the same features, so the activation is lane-local; mode 1: 64 output rows)
- * and all the tile's columns: 4 x 8 accumulators of 16x16. Gate/up with one-piece
- * activations runs 4-wave workgroups (128 features), two per CU, so that one
- * workgroup's matrix work covers the other's barrier and load waits; two-piece
- * activations and the down GEMM run 8-wave workgroups (256 features / 512 rows), one per
- * CU (their stages need 128 KB of LDS).
+ * Work unit of the bf16 GEMMs: one workgroup = (column tile of up to 128 pairs, feature tile).
+ * Wave w owns 4 row groups of 16 weight rows (mode 0: 32 gate rows and the 32 up rows of the
+ * same features, so the activation is lane-local; mode 1: 64 output rows) and all the tile's
+ * columns: 4 x 8 accumulators of 16x16. The routed gate/up runs 4-wave workgroups (128
+ * features), two per CU, so that one workgroup's matrix work covers the other's barrier and
+ * load waits; the dense GEMMs run 8-wave workgroups (256 features / 512 rows), one per CU
+ * (their stages need 128 KB of LDS).
  *
  * Weights (A operand) go from HBM straight to registers in the tiled layouts of
  * k3g_tile.hip: one 16-byte load per lane and row group gives a 16-row x 128-column block
@@ -26,16 +27,15 @@
  * times a power-of-two scale is a 3-bit significand: bf16 holds it exactly). Tiled bf16
  * weights (the shared expert) load as A operands directly.
  *
- * Activations (B operand) are bf16 PIECES: x (or h) = piece0 + piece1 with piece0 =
- * bf16(v) and piece1 = bf16(v - piece0), 16 significant bits, so the products see the
- * activations to 2^-17 relative. A single bf16 piece of h would cost ~1.7e-3 rel-L2 on
- * the layer output; two cost ~2e-6. When every x is already a bf16 value (piece1 = 0
- * everywhere, recorded in a flag) the gate/up GEMMs skip piece 1: the result is the
- * same. The column tile's activations are staged in LDS, 128 columns x 128 K per piece
- * per stage, two stages, written by global_load_lds_dwordx4 (no register round trip) in a
- * row-XOR-swizzled layout that the B-operand reads (ds_read_b128) hit without bank
- * conflicts. K advances 128 per step: one barrier per step, the next step's weights and
- * activations in flight during the current step's matrix work.
+ * Activations (B operand) are bf16 PIECES: v = piece0 + piece1 with piece0 = bf16(v) and
+ * piece1 = bf16(v - piece0), 16 significant bits. When every x is already a bf16 value
+ * (piece1 = 0 everywhere, recorded in a flag) the products skip piece 1: the result is the
+ * same; the routed gate/up runs here only then. The column tile's activations are staged in
+ * LDS, 128 columns x 128 K per piece per stage, two stages, written by
+ * global_load_lds_dwordx4 (no register round trip) in a row-XOR-swizzled layout that the
+ * B-operand reads (ds_read_b128) hit without bank conflicts. K advances 128 per step: one
+ * barrier per step, the next step's weights and activations in flight during the current
+ * step's matrix work.
  *
  * Workgroup order: column tiles are sorted largest first (an expert's full tiles next to
  * each other) and dealt to the 8 XCDs in groups of K3G_TILE_GROUP consecutive tiles, the
@@ -45,13 +45,8 @@
  * XCD's L2; the feature tiles of one column tile run back to back on one XCD and share
  * the tile's activations there.
  */
-#include "k3g_dev.h"
-#include "k3g_kernels.h"
-
-typedef float k3v4f __attribute__((ext_vector_type(4)));
-typedef __bf16 k3v8bf __attribute__((ext_vector_type(8)));
-typedef __bf16 k3v2bf __attribute__((ext_vector_type(2)));
-typedef __attribute__((address_space(3))) void *k3lds;
+#include "k3g_gemm.h"
+#include "k3g_gemm6.h"
 
 #define GM_WAVES 8
 #define GM_COLS 128                       /* pair columns per tile */
@@ -59,8 +54,6 @@ typedef __attribute__((address_space(3))) void *k3lds;
 #define GM_PIECE (GM_COLS * GM_KC * 2)    /* bytes of one piece of one stage: 32 KB */
 #define GM_STAGE (2 * GM_PIECE)
 #define GM_QT 4352                        /* tiled MXFP4 quad tile */
-
-__device__ __forceinline__ int gm_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 /* E8M0 byte -> 2^(b-127) as fp32 without branches (the tiled layout holds no 255) */
 __device__ __forceinline__ float gm_scale(uint32_t b)
@@ -93,25 +86,6 @@ __device__ __forceinline__ uint16_t gm_bf16_rn(float f)
 
 __device__ __forceinline__ float gm_bf16_f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
 
-/* Loads through pointers the compiler cannot prove global (they come from the expert
- * table) would be flat loads, which also count against the LDS counter and make every
- * ds_read wait for outstanding HBM loads: address them as global memory explicitly. */
-typedef unsigned int gm_v4u __attribute__((ext_vector_type(4)));
-#ifdef __HIP_DEVICE_COMPILE__
-typedef const __attribute__((address_space(1))) gm_v4u *gm_g4;
-typedef const __attribute__((address_space(1))) uint32_t *gm_g1;
-#else
-typedef const gm_v4u *gm_g4;       /* the host pass only parses device code */
-typedef const uint32_t *gm_g1;
-#endif
-
-__device__ __forceinline__ uint4 gm_ld16(const void *p)
-{
-    const gm_v4u v = *(gm_g4)p;
-    return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ uint32_t gm_ld4(const void *p) { return *(gm_g1)p; }
-
 /* h = act(gate, up) for 4 consecutive features of one column, stored as two bf16 pieces
  * (piece 1 at o + piece) */
 __device__ __noinline__ void gm_act_store(k3v4f gt, k3v4f up, float b1, float b2, uint16_t *o,
@@ -131,90 +105,8 @@ __device__ __noinline__ void gm_act_store(k3v4f gt, k3v4f up, float b1, float b2
     *(uint2 *)(o + piece) = vl;
 }
 
-/* One DMA instruction: 64 lanes x 16 bytes from their own global addresses to 1 KB of LDS
- * at byte address `lds` (lane l at lds + 16 l). Issued as inline assembly so the
- * compiler does not treat every later LDS read as waiting on it (it would drain all
- * outstanding loads before each ds_read); completion is awaited explicitly with
- * s_waitcnt vmcnt before the barrier that publishes the stage. M0 is saved and restored
- * around the instruction. */
-__device__ __forceinline__ void gm_dma16(const void *src, uint32_t lds)
-{
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\t"
-                 "s_mov_b32 m0, %2\n\t"
-                 "global_load_lds_dwordx4 %1, off\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(src), "s"(lds) : "memory");
-}
-
-/* The same DMA with a wave-uniform base in scalar registers and this lane's 32-bit byte
- * offset in one vector register: no per-lane 64-bit address to build or keep. */
-__device__ __forceinline__ void gm_dma16s(const void *sbase, uint32_t voff, uint32_t lds)
-{
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\t"
-                 "s_mov_b32 m0, %3\n\t"
-                 "global_load_lds_dwordx4 %1, %2\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds) : "memory");
-}
-
-__device__ __forceinline__ void gm_dma4s(const void *sbase, uint32_t voff, uint32_t lds)
-{
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\t"
-                 "s_mov_b32 m0, %3\n\t"
-                 "global_load_lds_dword %1, %2\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds) : "memory");
-}
-
-/* a wave-uniform pointer, in scalar registers */
-template <typename P>
-__device__ __forceinline__ P *gm_uniform_ptr(P *p)
-{
-    const uint64_t v = (uint64_t)(uintptr_t)p;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (P *)(uintptr_t)(((uint64_t)hi << 32) | lo);
-}
-
-/* raw buffer descriptor over `bytes` at p (p wave-uniform): loads take a scalar offset
- * and this lane's vector offset */
-typedef __amdgpu_buffer_rsrc_t gm_rsrc;
-__device__ __forceinline__ gm_rsrc gm_make_rsrc(const void *p, size_t bytes)
-{
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0,
-                                             (int)(bytes < 0x7fffffffu ? bytes : 0x7fffffffu),
-                                             0x00020000);
-}
-
-/* s_waitcnt vmcnt(N) (expcnt, lgkmcnt not waited on) */
-template <int N>
-__device__ __forceinline__ void gm_wait_vm()
-{
-    static_assert(N >= 0 && N < 16, "vmcnt");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | N);
-}
-
-/* s_waitcnt vmcnt(n) for a wave-uniform n in 8..16 */
-__device__ __forceinline__ void gm_wait_vm_n(int n)
-{
-    switch (n) {
-        case 8: gm_wait_vm<8>(); break;
-        case 9: gm_wait_vm<9>(); break;
-        case 10: gm_wait_vm<10>(); break;
-        case 11: gm_wait_vm<11>(); break;
-        case 12: gm_wait_vm<12>(); break;
-        case 13: gm_wait_vm<13>(); break;
-        case 14: gm_wait_vm<14>(); break;
-        case 15: gm_wait_vm<15>(); break;
-        default: gm_wait_vm<8>(); break;
-    }
-}
-
 /* ============================================================ scaled FP8 MFMA ====== */
-/* Used by the FP4 x FP8 variant and by the remainder piece of h in the bf16 path.
+/* Used by the FP4 x FP8 variant.
  * v_mfma_scale_f32_16x16x128_f8f6f4 with cbsz 4 (A: FP4) and blgp 0 (B: FP8 E4M3), each
  * 32-column block carrying its E8M0 scale. One instruction covers a whole 128-column
  * step: the tiled MXFP4 chunk is its A operand unchanged (lane L: row L % 16, block
@@ -226,16 +118,6 @@ __device__ __forceinline__ void gm_wait_vm_n(int n)
  * distinct bank groups); then 128 x 4 scale bytes. */
 #define GM_F8_DATA (GM_COLS * GM_KC)
 #define GM_F8_STAGE (GM_F8_DATA + GM_COLS * 4)
-
-__device__ __forceinline__ void gm_dma4(const void *src, uint32_t lds)
-{
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\t"
-                 "s_mov_b32 m0, %2\n\t"
-                 "global_load_lds_dword %1, off\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(src), "s"(lds) : "memory");
-}
 
 typedef int gm_v8i __attribute__((ext_vector_type(8)));
 
@@ -268,46 +150,6 @@ __device__ __forceinline__ uint32_t gm_e4m3x4(float a, float b, float c, float d
     int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
     w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
     return (uint32_t)w;
-}
-
-/* h = act(gate, up) for the wave's 32 features of one column (this lane's features
- * 4 g + i and 16 + 4 g + i, g = g4): bf16(h) at o (piece 0, bf16 row at o) and the
- * remainder h - bf16(h) as one MX block: E4M3 bytes at oq, E8M0 scale at *os. The block
- * exponent puts the largest remainder in [128, 256), under E4M3's 448, so nothing clamps;
- * the remainder keeps 4 significant bits, h about 12. */
-__device__ __noinline__ void gm_act_store_mix(k3v4f g0, k3v4f g1, k3v4f u0, k3v4f u1, float b1,
-                                              float b2, uint16_t *o, uint8_t *oq, uint8_t *os,
-                                              int g4)
-{
-    uint16_t hi[8];
-    float rr[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float y0 = k3d_act(g0[i], u0[i], b1, b2), y1 = k3d_act(g1[i], u1[i], b1, b2);
-        hi[i] = gm_bf16_rn(y0);
-        hi[4 + i] = gm_bf16_rn(y1);
-        rr[i] = y0 - gm_bf16_f(hi[i]);
-        rr[4 + i] = y1 - gm_bf16_f(hi[4 + i]);
-    }
-    float m = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(rr[i]));
-    m = fmaxf(m, __shfl_xor(m, 16, K3G_WAVE));
-    m = fmaxf(m, __shfl_xor(m, 32, K3G_WAVE));
-    int sx = -127;
-    if (m > 0.0f) {
-        int e;
-        frexpf(m, &e);
-        sx = e - 8 < -127 ? -127 : (e - 8 > 127 ? 127 : e - 8);
-    }
-    uint2 v0, v1;
-    v0.x = hi[0] | ((uint32_t)hi[1] << 16); v0.y = hi[2] | ((uint32_t)hi[3] << 16);
-    v1.x = hi[4] | ((uint32_t)hi[5] << 16); v1.y = hi[6] | ((uint32_t)hi[7] << 16);
-    *(uint2 *)(o + 4 * g4) = v0;
-    *(uint2 *)(o + 16 + 4 * g4) = v1;
-    *(uint32_t *)(oq + 4 * g4) = gm_e4m3x4(rr[0], rr[1], rr[2], rr[3], sx);
-    *(uint32_t *)(oq + 16 + 4 * g4) = gm_e4m3x4(rr[4], rr[5], rr[6], rr[7], sx);
-    if (g4 == 0) *os = (uint8_t)(sx + 127);
 }
 
 /* Instruction order of one step's matrix work (NR B-operand reads from LDS, 4 MFMAs
@@ -408,14 +250,11 @@ __device__ __forceinline__ void gm_tile(const K3kGemm &g, const GmTile &t)
          * loads in flight), and every step issues the same loads (clamped to the last step;
          * the padding steps past nK only skip their matrix work), so the compiler's load
          * counters agree on every path and its waits stay on the step that is due. */
-        /* loads after the ones step c needs: SN == 3: DMA(c + 1) then weights(c + 1);
-         * SN == 2: weights(c + 1) only (DMA(c) came after them) */
-        const int after = SN == 3 ? 8 + NP * t.ndma : 8;
         auto step = [&](int c, const uint4 (&cur)[4], const uint32_t (&scl)[4], uint4 (&nxt)[4],
                         uint32_t (&nsc)[4]) {
-            gm_wait_vm_n(after);
+            gm_wait_vm<8>();             /* all but the loads of weights(c + 1) */
             __syncthreads();
-            dma(min(c + SN - 1, t.nK - 1));
+            dma(min(c + 1, t.nK - 1));
             aload(min(c + 2, t.nK - 1), nxt, nsc);
             __builtin_amdgcn_sched_barrier(0);
             if (c < t.nK) {
@@ -442,7 +281,6 @@ __device__ __forceinline__ void gm_tile(const K3kGemm &g, const GmTile &t)
         aload(0, ab[0], sb[0]);
         dma(0);
         aload(min(1, t.nK - 1), ab[1], sb[1]);
-        if (SN == 3) dma(min(1, t.nK - 1));
         for (int c = 0; c < t.nK; c += 3) {
             step(c, ab[0], sb[0], ab[2], sb[2]);
             step(c + 1, ab[1], sb[1], ab[0], sb[0]);
@@ -514,6 +352,12 @@ __device__ __forceinline__ void gm_tile(const K3kGemm &g, const GmTile &t)
         }
         return;
     }
+    if constexpr (AF == 0) {
+        __syncthreads();                 /* every wave is done with the LDS */
+        gm_store_h<4, NB>(acc, (float *)(t.ldsp + t.w * GM_HLDS), lane, t.orow0, g.rows, t.p0, t.np,
+                          g.b1, g.b2, g.h6);
+        return;
+    }
     if (g.mode == 0) {
         if (!t.rv[0]) return;
         const int n = t.orow0 + 4 * t.g4;
@@ -522,15 +366,9 @@ __device__ __forceinline__ void gm_tile(const K3kGemm &g, const GmTile &t)
             const int col = 16 * cb + col0;
             if (col < t.np) {
                 const size_t row = (size_t)(t.p0 + col);
-                if (AF == 0 && g.hmix) {
-                    gm_act_store_mix(acc[0][cb], acc[1][cb], acc[2][cb], acc[3][cb], g.b1, g.b2,
-                                     g.h + row * g.ldh + t.orow0, g.hq + row * g.ldhq + t.orow0,
-                                     g.hs + row * (g.ldhq / 32) + t.orow0 / 32, t.g4);
-                } else {
-                    uint16_t *o = g.h + row * g.ldh + n;
-                    gm_act_store(acc[0][cb], acc[2][cb], g.b1, g.b2, o, g.hpiece);
-                    gm_act_store(acc[1][cb], acc[3][cb], g.b1, g.b2, o + 16, g.hpiece);
-                }
+                uint16_t *o = g.h + row * g.ldh + n;
+                gm_act_store(acc[0][cb], acc[2][cb], g.b1, g.b2, o, g.hpiece);
+                gm_act_store(acc[1][cb], acc[3][cb], g.b1, g.b2, o + 16, g.hpiece);
             }
         }
     } else {
@@ -544,155 +382,6 @@ __device__ __forceinline__ void gm_tile(const K3kGemm &g, const GmTile &t)
                 for (int r = 0; r < 4; ++r)
                     if (t.rv[r]) *(k3v4f *)(o + 16 * r) = acc[r][cb];
             }
-        }
-    }
-}
-
-/* Instruction order of one step of the down GEMM's matrix work: NB FP8 groups (the
- * remainder: 3 LDS reads, 4 scaled MFMAs each), then 4 NB bf16 groups (piece 0: 1 LDS
- * read, 4 MFMAs each), the reads AH groups ahead of the MFMAs that use them. */
-template <int NB, int AH>
-__device__ __forceinline__ void gm_pipeline_mix()
-{
-    constexpr int NG = 5 * NB;
-    constexpr int PRO = AH <= NB ? 3 * AH : 3 * NB + (AH - NB);
-    __builtin_amdgcn_sched_group_barrier(0x100, PRO, 0);     /* DS read */
-#pragma unroll
-    for (int j = 0; j < NG; ++j) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);   /* MFMA */
-        if (j + AH < NB) __builtin_amdgcn_sched_group_barrier(0x100, 3, 0);
-        else if (j + AH < NG) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-    }
-}
-
-/* The down GEMM of MXFP4 experts with h as bf16 piece 0 (bf16 matrix cores, as gm_tile)
- * plus its MX remainder (scaled FP8 matrix cores, one 16x16x128 instruction per step
- * on the same weight registers, at twice the bf16 rate): three quarters of the matrix
- * time of two bf16 pieces. Stage c % 2: piece 0 (GM_PIECE, gm_tile's layout), then the
- * remainder's bytes and scales (GM_F8_STAGE, k_gemm_f8's layout). The weight and DMA
- * pipeline is gm_tile's with two stages: a step waits for all but the 8 weight loads
- * issued after its stage's DMA.
- *
- * The tile's B rows are sorted positions p0 .. p0 + 127, contiguous: every DMA takes a
- * uniform base in scalar registers (the tile's first row, advanced per step) and a
- * loop-invariant byte offset per lane (bofb: piece 0, doff: remainder bytes, soff:
- * remainder scales, all relative to row p0); the weights load through one buffer
- * descriptor per row group with the step in the scalar offset. No per-lane 64-bit
- * address is kept, which leaves the registers for the LDS read-ahead. */
-template <int NB>
-__device__ __forceinline__ void gm_tile_mix(const K3kGemm &g, const GmTile &t,
-                                            const uint32_t (&bofb)[4], const uint32_t (&doff)[2],
-                                            uint32_t soff, int nd, int ns)
-{
-    k3v4f acc[4][NB];
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-        for (int cb = 0; cb < NB; ++cb) acc[r][cb] = k3v4f{0.f, 0.f, 0.f, 0.f};
-    const int lane = t.lane;
-    constexpr uint32_t ST = GM_PIECE + GM_F8_STAGE;
-    const uint8_t *b0 = gm_uniform_ptr((const uint8_t *)(g.b + (size_t)t.p0 * g.ldb));
-    const uint8_t *q0 = gm_uniform_ptr(g.bq + (size_t)t.p0 * g.ldhq);
-    const uint8_t *s0 = gm_uniform_ptr(g.bs + (size_t)t.p0 * (g.ldhq / 32));
-    auto dma = [&](int c) {
-        const uint32_t st = t.lds + (c & 1) * ST;
-        const uint8_t *b = b0 + (size_t)c * (2 * GM_KC);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            if (i < t.ndma) gm_dma16s(b, bofb[i], st + t.w * 1024 + i * 8 * 1024);
-        const uint8_t *q = q0 + (size_t)c * GM_KC;
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            if (i < nd) gm_dma16s(q, doff[i], st + GM_PIECE + (8 * i + t.w) * 1024);
-        if (t.w < ns) gm_dma4s(s0 + 4 * c, soff, st + GM_PIECE + GM_F8_DATA + t.w * 256);
-    };
-    const uint8_t *brow = t.ldsp + (lane & 15) * 256;
-    const int q4 = lane >> 4, c0 = lane & 15;
-    gm_rsrc ar[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ar[r] = gm_make_rsrc(t.abase[r], t.rbb);
-    const int v16 = 16 * lane, v4 = 4 * lane;
-    uint4 ab[3][4];
-    uint32_t sbuf[3][4];
-    auto aload = [&](int c, uint4 (&dst)[4], uint32_t (&sdst)[4]) {
-        const int so = (c >> 2) * GM_QT;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            dst[r] = __builtin_bit_cast(
-                uint4, __builtin_amdgcn_raw_buffer_load_b128(ar[r], v16, so + 1024 * (c & 3), 0));
-            sdst[r] = __builtin_amdgcn_raw_buffer_load_b32(ar[r], v4, so + 4096, 0);
-        }
-    };
-    auto step = [&](int c, const uint4 (&cur)[4], const uint32_t (&scl)[4], uint4 (&nxt)[4],
-                    uint32_t (&nsc)[4]) {
-        gm_wait_vm<8>();
-        __syncthreads();
-        dma(min(c + 1, t.nK - 1));
-        aload(min(c + 2, t.nK - 1), nxt, nsc);
-        __builtin_amdgcn_sched_barrier(0);
-        if (c < t.nK) {
-            /* rows outside the matrix read row block 0 and are never stored */
-            const int j = c & 3;
-            const uint32_t so = (c & 1) * ST;
-            /* the remainder first: the weight words then die sub-step by sub-step */
-#pragma unroll
-            for (int cb = 0; cb < NB; ++cb) {
-                const int row = 16 * cb + c0;
-                const int hsw = (row >> 1) & 7;
-                const uint8_t *base = t.ldsp + so + GM_PIECE + row * 128;
-                const uint4 lo = *(const uint4 *)(base + 16 * ((2 * q4) ^ hsw));
-                const uint4 hi = *(const uint4 *)(base + 16 * ((2 * q4 + 1) ^ hsw));
-                const gm_v8i bv = {(int)lo.x, (int)lo.y, (int)lo.z, (int)lo.w,
-                                   (int)hi.x, (int)hi.y, (int)hi.z, (int)hi.w};
-                const uint32_t sb = t.ldsp[so + GM_PIECE + GM_F8_DATA + row * 4 + q4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    acc[r][cb] = gm_mma_f8(cur[r], (scl[r] >> (8 * j)) & 0xffu, bv, sb, acc[r][cb]);
-            }
-            float sc[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sc[r] = gm_scale((scl[r] >> (8 * j)) & 0xffu);
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                k3v8bf a[4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const uint32_t wd = s == 0 ? cur[r].x : s == 1 ? cur[r].y
-                                      : s == 2 ? cur[r].z : cur[r].w;
-                    a[r] = gm_deq8(wd, sc[r]);
-                }
-                const int qs = 4 * s + t.g4;
-#pragma unroll
-                for (int cb = 0; cb < NB; ++cb) {
-                    const uint4 bv = *(const uint4 *)(brow + so + cb * 16 * 256 + 16 * (qs ^ c0));
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) acc[r][cb] = gm_mma(a[r], bv, acc[r][cb]);
-                }
-            }
-            /* the reads three groups ahead (where the registers allow it: a full tile of 8
-             * column blocks keeps the compiler's own order, without spilling) */
-            gm_pipeline_mix<NB, 3>();
-        }
-    };
-    aload(0, ab[0], sbuf[0]);
-    dma(0);
-    aload(min(1, t.nK - 1), ab[1], sbuf[1]);
-    for (int c = 0; c < t.nK; c += 3) {
-        step(c, ab[0], sbuf[0], ab[2], sbuf[2]);
-        step(c + 1, ab[1], sbuf[1], ab[0], sbuf[0]);
-        step(c + 2, ab[2], sbuf[2], ab[1], sbuf[1]);
-    }
-    gm_wait_vm<0>();
-
-#pragma unroll
-    for (int cb = 0; cb < NB; ++cb) {
-        const int col = 16 * cb + c0;
-        if (col < t.np) {
-            const int p = t.p0 + col;
-            float *o = g.out + (size_t)(g.scatter ? g.perm[p] : p) * g.ldo + t.orow0 + 4 * t.g4;
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (t.rv[r]) *(k3v4f *)(o + 16 * r) = acc[r][cb];
         }
     }
 }
@@ -789,20 +478,15 @@ __device__ __forceinline__ int gm_src_row(const K3kGemm &g, const GmTile &t, int
     return (g.mode == 0 && g.perm) ? g.perm[p] / g.topk : p;
 }
 
-/* WV = 8: one workgroup per CU, any piece count. WV = 4 (one-piece B only): two
- * workgroups of 4 waves per CU, each with 64 KB of stages, so one workgroup's matrix work
- * fills the other's barrier and load waits. */
+/* One workgroup of a bf16 GEMM (false: it has no tile). WV = 8: one workgroup per CU, one or two pieces. WV = 4 (one-piece
+ * B only): two workgroups of 4 waves per CU, each with 64 KB of stages, so one workgroup's
+ * matrix work fills the other's barrier and load waits. */
 template <int AF, int WV>
-__global__ void __launch_bounds__(WV * 64, 8 / WV)
-k_gemm(const K3kGemm g)
+__device__ __forceinline__ bool gm_block(const K3kGemm &g, uint8_t *lds, int npr)
 {
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[WV == 8 ? 2 * GM_STAGE : 2 * GM_PIECE];
-    const int npr = (g.npieces > 1 && (!g.lo_flag || *g.lo_flag)) ? 2 : 1;
-    if (WV == 4 ? npr != 1 : (g.np_only == 2 && npr != 2)) return;
     GmTile t;
     int nb;
-    if (!gm_setup<AF, WV>(g, t, lds, nb)) return;
-    const unsigned long long t_start = g.trace ? wall_clock64() : 0;
+    if (!gm_setup<AF, WV>(g, t, lds, nb)) return false;
 
     /* ---- the activation rows this lane's DMA reads --------------------------------- */
     /* instruction i of wave w fills LDS rows 4 (WV i + w) .. + 3; lane l writes row
@@ -823,49 +507,8 @@ k_gemm(const K3kGemm g)
     /* instructions whose first row is inside the tile's 16 nb rows */
     t.ndma = min(NI, (4 * nb + WV - 1 - t.w) / WV);
 
-    bool mixed = false;
-    if constexpr (AF == 0 && WV == 8) {
-        if (g.mode == 1 && g.hmix) {
-            /* the remainder's DMA (k_gemm_f8's layout, 128 rows): instruction i of wave w
-             * fills rows 8 (8 i + w) .. + 7; waves 0 and 1 fill the scales of rows 0 .. 63
-             * and 64 .. 127 */
-            mixed = true;
-            /* offsets relative to the tile's first row p0 (its rows are p0 .. p0 + 127) */
-            auto rel = [&](int r) { return r < t.np ? r : 0; };
-            uint32_t bofb[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int r = 4 * (8 * i + t.w) + (t.lane >> 4);
-                bofb[i] = 2u * ((uint32_t)rel(r) * (uint32_t)g.ldb + (uint32_t)qoff);
-            }
-            uint32_t doff[2];
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int r = 8 * (8 * i + t.w) + (t.lane >> 3);
-                const int ls = (t.lane & 7) ^ ((r >> 1) & 7);
-                const int u = (ls & 1) ? 4 + (ls >> 1) : (ls >> 1);
-                doff[i] = (uint32_t)rel(r) * (uint32_t)g.ldhq + 16 * u;
-            }
-            const int nd = min(2, (2 * nb + 7 - t.w) / 8);
-            const int ns = nb > 4 ? 2 : 1;
-            const uint32_t soff =
-                (uint32_t)rel(64 * min(t.w, 1) + t.lane) * (uint32_t)(g.ldhq / 32);
-            switch (nb) {
-                case 1: gm_tile_mix<1>(g, t, bofb, doff, soff, nd, ns); break;
-                case 2: gm_tile_mix<2>(g, t, bofb, doff, soff, nd, ns); break;
-                case 3: gm_tile_mix<3>(g, t, bofb, doff, soff, nd, ns); break;
-                case 4: gm_tile_mix<4>(g, t, bofb, doff, soff, nd, ns); break;
-                case 5: gm_tile_mix<5>(g, t, bofb, doff, soff, nd, ns); break;
-                case 6: gm_tile_mix<6>(g, t, bofb, doff, soff, nd, ns); break;
-                case 7: gm_tile_mix<7>(g, t, bofb, doff, soff, nd, ns); break;
-                case 8: gm_tile_mix<8>(g, t, bofb, doff, soff, nd, ns); break;
-                default: break;
-            }
-        }
-    }
 #define GM_CASE(P, B) case (P) * 16 + (B): gm_tile<AF, P, B, WV>(g, t); break;
-    if (mixed) {
-    } else if constexpr (WV == 8) {
+    if constexpr (WV == 8) {
         switch (npr * 16 + nb) {
             GM_CASE(1, 1) GM_CASE(1, 2) GM_CASE(1, 3) GM_CASE(1, 4)
             GM_CASE(1, 5) GM_CASE(1, 6) GM_CASE(1, 7) GM_CASE(1, 8)
@@ -881,19 +524,60 @@ k_gemm(const K3kGemm g)
         }
     }
 #undef GM_CASE
-    if (g.trace && threadIdx.x == 0) {
-        const int slot = blockIdx.x >> 3;
-        const int rnd = slot / g.nft, xcd = blockIdx.x & 7;
-        const int grp = rnd / K3G_TILE_GROUP, gi = rnd - grp * K3G_TILE_GROUP;
-        unsigned long long *o = g.trace + 4 * (size_t)blockIdx.x;
-        o[0] = t_start;
-        o[1] = wall_clock64();
-        o[2] = (unsigned long long)(K3G_TILE_GROUP * (8 * grp + ((grp & 1) ? 7 - xcd : xcd)) +
-                                    gi) << 32 |
-               (unsigned)(slot - rnd * g.nft);
-        o[3] = (unsigned long long)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15) << 32 |
-               (unsigned)__builtin_amdgcn_s_getreg((31 << 11) | 4);
+    return true;
+}
+
+/* the dense GEMMs (tiled bf16 weights) */
+__global__ void __launch_bounds__(GM_WAVES * 64, 1)
+k_gemm(const K3kGemm g)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * GM_STAGE];
+    gm_block<1, GM_WAVES>(g, lds, g.npieces > 1 && (!g.lo_flag || *g.lo_flag) ? 2 : 1);
+}
+
+/* The routed experts' gate/up (mode 0) or down (mode 1): FP6 pieces on the FP4 x FP6 matrix cores;
+ * but gate/up of an x that is all bf16 values (its flag is clear) on the bf16 ones, where that
+ * x is one piece. Both take workgroups of 4 waves for 128 features (256 rows) and write h alike.
+ * In full tiles (32,768 pairs) gate/up takes 1.46 ms on one bf16 piece, 1.78 on four FP6
+ * pieces and took 2.58 on two bf16 pieces. */
+template <int MODE>
+__global__ void __launch_bounds__(256, 2)
+k_gemm6(const K3kGemm6 g)
+{
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[G6_LDS];
+    static_assert(G6_LDS == 4 * GM_HLDS && G6_LDS >= 2 * GM_PIECE, "LDS");
+    const unsigned long long t_start = g.trace ? wall_clock64() : 0;
+    const bool bf16 = MODE == 0 && g.xb && !*g.lo_flag;
+    if (bf16) {
+        K3kGemm b = {};
+        b.rows = g.rows;
+        b.K = g.K;
+        b.ldb = g.ldb;
+        b.eq = g.eq;
+        b.b = g.xb;
+        b.perm = g.perm;
+        b.topk = g.topk;
+        b.tiles = g.tiles;
+        b.ntiles = g.ntiles;
+        b.h6 = g.h;
+        b.b1 = g.b1;
+        b.b2 = g.b2;
+        b.nft = g.nft;
+        if (!gm_block<0, 4>(b, lds, 1)) return;
+    } else {
+        G6Tile t;
+        switch (g6_setup<MODE>(g, t, lds)) {
+            case 16 * 8 + 3: g6_run<MODE, 3, 8>(g, t); break;
+            case 16 * 8 + 4: g6_run<MODE, 4, 8>(g, t); break;
+            case 16 * 4 + 1: g6_run<MODE, 1, 4>(g, t); break;
+            case 16 * 4 + 2: g6_run<MODE, 2, 4>(g, t); break;
+            case 16 * 4 + 3: g6_run<MODE, 3, 4>(g, t); break;
+            case 16 * 4 + 4: g6_run<MODE, 4, 4>(g, t); break;
+            default: return;
+        }
     }
+    if (g.trace && threadIdx.x == 0) gm_trace(g.trace, g.nft, g.trace_step,
+                                                  bf16 ? 0 : g.halves, t_start);
 }
 
 /* ============================================================ FP4 x FP8 variant ==== */
@@ -1232,7 +916,7 @@ extern "C" int k3k_xq8(const float *x, int T, int d, int ldq, uint8_t *xq, uint8
 
 extern "C" int k3k_gemm_f8(const K3kGemm *g, hipStream_t st)
 {
-    if (g->mode < 0 || g->mode > 1 || g->afmt != 0 || !g->eq || !g->bq || !g->bs) return -1;
+    if (g->mode < 0 || g->mode > 1 || !g->eq || !g->bq || !g->bs) return -1;
     if (g->K < 32 || g->K % 32 || g->rows < 16 || g->ldb < g->K || g->ldb % 512 || g->nft < 1)
         return -1;
     if (g->mode == 0 && (g->rows % 32 || g->nft * 256 < g->rows || !g->hq || !g->hs ||
@@ -1253,55 +937,69 @@ extern "C" int k3k_gemm_f8(const K3kGemm *g, hipStream_t st)
 extern "C" int k3k_gemm(const K3kGemm *g, hipStream_t st)
 {
     /* shapes the kernel's indexing assumes */
-    if (g->mode < 0 || g->mode > 1 || g->afmt < 0 || g->afmt > 1) return -1;
+    if (g->mode < 0 || g->mode > 1) return -1;
     if (g->K < 32 || g->K % 32 || g->rows < 16 || g->ldb < g->K || g->ldb % GM_KC ||
         g->npieces < 1 || g->npieces > 2 || !g->b || g->nft < 1)
         return -1;
-    if (g->mode == 0 && (g->rows % 32 || g->nft * 256 < g->rows || !g->h || g->ldh < g->rows))
+    if (g->mode == 0 && (g->rows % 32 || g->nft * 256 < g->rows))
         return -1;
+    if (g->mode == 0 && (!g->h || g->ldh < g->rows)) return -1;
     if (g->mode == 1 && (g->rows % 16 || g->nft * 512 < g->rows || !g->out || g->ldo < g->rows ||
                          g->ldo % 4))
         return -1;
-    if (g->afmt == 0 && !g->eq) return -1;
-    if (g->hmix && (g->afmt != 0 || g->ldhq % 512 ||
-                    (g->mode == 0 ? (!g->hq || !g->hs || g->ldhq < g->rows)
-                                  : (!g->bq || !g->bs || g->ldhq < g->K || g->npieces != 1))))
+    if (!g->wa || (g->mode == 0 && !g->wb) || g->tiles || g->scatter || g->dense_rows < 1)
         return -1;
-    if (g->afmt == 1 && (!g->wa || (g->mode == 0 && !g->wb))) return -1;
-    if (g->tiles ? (!g->ntiles || g->max_tiles < 1) : g->dense_rows < 1) return -1;
-    if ((g->scatter || (g->mode == 0 && g->tiles)) && !g->perm) return -1;
     const int ks_n = g->ksplit > 1 ? g->ksplit : 1;
-    if (ks_n > 1 && (g->tiles || g->afmt != 1 || !g->part || g->K % GM_KC ||
+    if (ks_n > 1 && (!g->part || g->K % GM_KC ||
                      ks_n > g->K / GM_KC || (g->mode == 0 && g->rows % 4)))
         return -1;
-    const long long maxt = g->tiles ? g->max_tiles
-                                    : (long long)((g->dense_rows + GM_COLS - 1) / GM_COLS) * ks_n;
+    const long long maxt = (long long)((g->dense_rows + GM_COLS - 1) / GM_COLS) * ks_n;
     const long long grid = 8 * (long long)K3G_TILE_ROUNDS(maxt) * g->nft;
     if (grid > 0x7fffffff) return -1;
-    if (g->afmt == 0 && g->mode == 0) {
-        /* gate/up of MXFP4 experts: 4-wave workgroups when x is one piece (the usual case:
-         * decided on the device from the flag), 8-wave ones for two pieces; each launch
-         * leaves at once when the other one's case holds */
-        K3kGemm g4 = *g, g8 = *g;
-        g4.nft = (g->rows + 127) / 128;
-        g8.np_only = 2;
-        const long long grid4 = 8 * (long long)K3G_TILE_ROUNDS(maxt) * g4.nft;
-        if (grid4 > 0x7fffffff) return -1;
-        hipLaunchKernelGGL((k_gemm<0, 4>), dim3((unsigned)grid4), dim3(4 * 64), 0, st, g4);
-        if (g->npieces > 1)
-            hipLaunchKernelGGL((k_gemm<0, 8>), dim3((unsigned)grid), dim3(GM_WAVES * 64), 0, st, g8);
-    } else if (g->afmt == 0) {
-        hipLaunchKernelGGL((k_gemm<0, 8>), dim3((unsigned)grid), dim3(GM_WAVES * 64), 0, st, *g);
-    } else {
-        K3kGemm g1 = *g;
-        g1.ksplit = ks_n;
-        hipLaunchKernelGGL((k_gemm<1, 8>), dim3((unsigned)grid), dim3(GM_WAVES * 64), 0, st, g1);
-        if (ks_n > 1) {
-            const long long n = (long long)g->dense_rows * (g->rows / 4);
-            hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                               g->part, ks_n, g->dense_rows, g->rows, g->mode, g->b1, g->b2,
-                               g->h, g->hpiece, g->ldh, g->out, g->ldo);
-        }
+    K3kGemm g1 = *g;
+    g1.ksplit = ks_n;
+    hipLaunchKernelGGL(k_gemm, dim3((unsigned)grid), dim3(GM_WAVES * 64), 0, st, g1);
+    if (ks_n > 1) {
+        const long long n = (long long)g->dense_rows * (g->rows / 4);
+        hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
+                           g->part, ks_n, g->dense_rows, g->rows, g->mode, g->b1, g->b2,
+                           g->h, g->hpiece, g->ldh, g->out, g->ldo);
     }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+extern "C" int k3k_x6(const float *x, int T, int K, uint8_t *o, const int32_t *run_flag,
+                      hipStream_t st)
+{
+    if (T < 1 || K < 32 || K % 32 || ((uintptr_t)o & 15)) return -1;
+    const long long n = (long long)T * 4 * ((K + 127) / 128);
+    const dim3 grid((unsigned)((n + 255) / 256));
+    if (((uintptr_t)x & 15) == 0)
+        hipLaunchKernelGGL(k_x6<true>, grid, dim3(256), 0, st, x, T, K, o, run_flag);
+    else
+        hipLaunchKernelGGL(k_x6<false>, grid, dim3(256), 0, st, x, T, K, o, run_flag);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+extern "C" int k3k_gemm6(const K3kGemm6 *g, hipStream_t st)
+{
+    /* shapes the kernel's indexing assumes */
+    if (g->mode < 0 || g->mode > 1 || !g->eq || !g->b || ((uintptr_t)g->b & 15) || !g->tiles ||
+        !g->ntiles || g->max_tiles < 1 || !g->perm || g->topk < 1 || g->halves < 0 || g->halves > 1 || g->K < 32 || g->K % 32 ||
+        g->rows < 32 || g->rows % 32)
+        return -1;
+    if (g->mode == 0 ? (!g->h || ((uintptr_t)g->h & 15) != 0)
+                     : (!g->out || g->ldo < g->rows || g->ldo % 4))
+        return -1;
+    if (g->xb && (g->mode != 0 || !g->lo_flag || g->ldb < g->K || g->ldb % GM_KC)) return -1;
+    K3kGemm6 a = *g;
+    const int per = g->mode == 0 ? G6_ROWS / 2 : G6_ROWS;
+    a.nft = (g->rows + per - 1) / per;
+    const long long grid = 8 * (long long)K3G_TILE_ROUNDS((long long)g->max_tiles << g->halves) * a.nft;
+    if (grid > 0x7fffffff) return -1;
+    if (g->mode == 0)
+        hipLaunchKernelGGL(k_gemm6<0>, dim3((unsigned)grid), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL(k_gemm6<1>, dim3((unsigned)grid), dim3(256), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -118,7 +118,6 @@ typedef struct {
  * pairs grouped by expert (tiles) or all tokens (dense, the shared expert). */
 typedef struct {
     int mode;                 /* 0: gate/up + activation -> h pieces; 1: down -> fp32 rows */
-    int afmt;                 /* 0: tiled MXFP4 per expert (eq); 1: tiled bf16 (wa, wb) */
     int rows;                 /* output rows of one weight matrix: inter (mode 0), hidden (1) */
     int K;                    /* reduction length */
     int ldb;                  /* row stride of the B pieces (elements), K rounded up to 128 */
@@ -147,22 +146,53 @@ typedef struct {
     const uint8_t *bq, *bs;
     uint8_t *hq, *hs;
     int ldhq;                 /* bytes per h row (scales: ldhq / 32) */
-    /* k3k_gemm with MXFP4 weights: h as bf16 piece 0 (h, b) plus its remainder
-     * h - bf16(h) as MXFP8 (mode 0 writes hq/hs, mode 1 reads bq/bs; row stride ldhq bytes)
-     * on the scaled FP8 matrix cores; mode 1 then takes npieces = 1 */
-    int hmix;
-    int np_only;              /* set by k3k_gemm: 2 = a launch that runs only two-piece B */
+    uint8_t *h6;              /* k3k_gemm with MXFP4 weights: h as FP6 quads (K3kGemm6) */
     /* dense tiled-bf16 GEMMs only: K cut into ksplit slices of whole 128-column steps
      * (1: none); the slices' fp32 sums go to part ([ksplit][columns][2][rows] gate/up,
      * [ksplit][columns][rows] down) and k3k_gemm reduces them in slice order */
     int ksplit;
     float *part;
-    /* instrumentation (NULL: off): per workgroup of the launch that does the work, wave
-     * 0's start and end (wall clock), tile << 32 | feature tile, XCC << 32 | HW_ID */
-    unsigned long long *trace;
 } K3kGemm;
 
 int k3k_gemm(const K3kGemm *g, hipStream_t st);
+
+/* bytes of an activation quad: 512 columns of one row as four FP6 pieces (k3g_gemm6.h) */
+#define K3G_P6_QUAD 1664
+
+/* One grouped GEMM of tiled MXFP4 experts on the FP4 x FP6 matrix cores (k3g_gemm6.h).
+ * Columns are (token, slot) pairs grouped by expert (tiles). */
+typedef struct {
+    int mode;                 /* 0: gate/up + activation -> h quads; 1: down -> fp32 rows */
+    int rows;                 /* output rows of one weight matrix: inter (mode 0), hidden (1) */
+    int K;                    /* reduction length */
+    const K3ExpertQ *eq;      /* mode 0: p1, p3; mode 1: p2 (tiled MXFP4) */
+    const uint8_t *b;         /* activation rows of ceil(K / 512) quads: by token (mode 0) or
+                               * by sorted position (mode 1) */
+    const int32_t *perm;      /* sorted position -> pair id (t * topk + j) */
+    int topk;
+    const int32_t *tiles;     /* {expert, first sorted position, count, 0} */
+    const int32_t *ntiles;
+    int max_tiles;            /* bound on *ntiles (grid size) */
+    uint8_t *h;               /* mode 0 out: rows of ceil(rows / 512) quads by sorted position */
+    float b1, b2;             /* activation caps */
+    float *out;               /* mode 1 out: row perm[column], stride ldo */
+    int ldo;
+    /* mode 0: x's first bf16 piece (rows of ldb), taken instead of b when *lo_flag, x's
+     * piece-1 flag, is 0; NULL: always b */
+    const uint16_t *xb;
+    int ldb;
+    const int32_t *lo_flag;
+    int halves;               /* 1: a tile may hold more than 64 pairs (it is two work items) */
+    int nft;                  /* set by k3k_gemm6: feature tiles */
+    /* instrumentation (NULL: off): per workgroup of every trace_step-th feature tile wave 0's
+     * start and end (wall clock), item << 32 | feature tile, XCC << 32 | HW_ID */
+    unsigned long long *trace;
+    int trace_step;
+} K3kGemm6;
+
+int k3k_gemm6(const K3kGemm6 *g, hipStream_t st);
+/* x (fp32 [T][K]) -> activation quads [T][ceil(K / 512)]; nothing when *run_flag is 0 */
+int k3k_x6(const float *x, int T, int K, uint8_t *o, const int32_t *run_flag, hipStream_t st);
 /* The K slices a dense GEMM of nft feature tiles x ntl column tiles over K columns uses
  * to give the GPU about 256 workgroups (1 = no split), and the part buffer bytes a
  * context needs for any column count (rows: the GEMM's output rows; x2 for gate/up). */
