@@ -148,25 +148,26 @@ __device__ __forceinline__ gm_v32f gm_from_fp6(const gm_v6u &p, float scale)
     return r;
 }
 
-/* One block of 32 values (even and odd elements apart) as four pieces into its place in a quad:
- * step j, block q. Each piece's scale puts the block's largest remainder in [4, 8). A block
- * with an infinity or NaN gets the NaN scale, so the products are NaN as they were. */
-__device__ __forceinline__ void gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *quad, int j, int q)
+/* 32 values (even and odd elements apart) as NP pieces: piece p's six dwords at d + 6 p, its E8M0
+ * byte s[p]; each piece's scale puts the largest remainder in [4, 8). True when a value is
+ * infinite or NaN (the pieces then mean nothing). */
+template <int NP>
+__device__ __forceinline__ bool gm_pieces(gm_v16f ev, gm_v16f od, uint32_t (&d)[6 * NP],
+                                          uint8_t (&s)[NP])
 {
-    uint32_t d[24], sw = 0;
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < 16; ++i)
         bad |= !(fabsf(ev[i]) < __builtin_inff()) || !(fabsf(od[i]) < __builtin_inff());
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
+    for (int p = 0; p < NP; ++p) {
         float m = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) m = fmaxf(m, fmaxf(fabsf(ev[i]), fabsf(od[i])));
         const int sb = m > 0.0f ? max((int)(__float_as_uint(m) >> 23) - 2, 1) : 127;
         const float scale = __uint_as_float((uint32_t)sb << 23);
         const gm_v6u w = gm_to_fp6(ev, od, scale);
-        if (p < 3) {
+        if (p < NP - 1) {
             const gm_v32f y = gm_from_fp6(w, scale);
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
@@ -176,9 +177,18 @@ __device__ __forceinline__ void gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *
         }
 #pragma unroll
         for (int i = 0; i < 6; ++i) d[6 * p + i] = w[i];
-        sw |= (uint32_t)sb << (8 * p);
+        s[p] = (uint8_t)sb;
     }
-    if (bad) sw = 0xffffffffu;
+    return bad;
+}
+
+/* One block of 32 values as four pieces into its place in a quad (k3g_gemm6.h): step j, block q.
+ * A block with an infinity or NaN gets the NaN scale, so the products are NaN as they were. */
+__device__ __forceinline__ void gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *quad, int j, int q)
+{
+    uint32_t d[24];
+    uint8_t s[4];
+    const bool bad = gm_pieces<4>(ev, od, d, s);
     uint8_t *o = quad + 384 * j;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
@@ -186,7 +196,8 @@ __device__ __forceinline__ void gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *
             make_uint4(d[6 * p], d[6 * p + 1], d[6 * p + 2], d[6 * p + 3]);
         *(uint2 *)(o + 256 + 32 * p + 8 * q) = make_uint2(d[6 * p + 4], d[6 * p + 5]);
     }
-    *(uint32_t *)(quad + 1536 + 16 * j + 4 * q) = sw;
+    *(uint32_t *)(quad + 1536 + 16 * j + 4 * q) =
+        bad ? 0xffffffffu : s[0] | (uint32_t)s[1] << 8 | (uint32_t)s[2] << 16 | (uint32_t)s[3] << 24;
 }
 
 /* This wave's LDS writes are visible to its own later reads, whichever lane made them */

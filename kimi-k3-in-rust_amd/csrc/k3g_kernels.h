@@ -211,6 +211,26 @@ int k3k_gemm_tiles(const int32_t *off, int E, int32_t *tiles, int32_t *ntiles,
 int k3k_xpieces(const float *x, int T, int d, int ldb, uint16_t *xb, long long piece,
                 int32_t *flag, hipStream_t st);
 
+/* The routed experts of checkpoint-layout MXFP4 weights on the FP4 x FP6 matrix cores
+ * (k3g_rows.hip): h = act(W1 z, W3 z) (mode 0) or contrib = W2 h (mode 1) for every active
+ * expert's pairs, K a multiple of 32. */
+typedef struct {
+    int mode;
+    int rows, K;                      /* inter, latent (mode 0); latent, inter (mode 1) */
+    const K3ExpertQ *eq;
+    const int32_t *act, *nact, *off, *perm;   /* as K3kRouted */
+    int topk;
+    const float *z;                   /* [.][K] by token (mode 0), by pair (mode 1) */
+    const uint8_t *x;                 /* its rows as pieces, k3k_rows_bytes(K) each (k3k_rows_x) */
+    float *h;                         /* mode 0 out [T * topk][rows] */
+    float *out;                       /* mode 1 out [T * topk][rows] */
+    float b1, b2;
+} K3kRows;
+int k3k_rows(const K3kRows *g, int maxU, hipStream_t st);
+/* bytes of an activation row of K values; x (fp32 [T][K]) -> activation rows */
+size_t k3k_rows_bytes(int K);
+int k3k_rows_x(const float *x, int T, int K, uint8_t *o, hipStream_t st);
+
 /* K slices of the fused kernel's ticket classes (fewer when K is short); each may be set
  * at build time (-DK3G_KS_SG=...) */
 #ifndef K3G_KS_G
