@@ -83,22 +83,26 @@ k_router_logits(const float *__restrict__ x, int T, const float *__restrict__ W,
 }
 
 /* ------------------------------------------------- logits on the matrix cores ---- */
-/* Many tokens: the logits as a GEMM on v_mfma_f64_16x16x4f64 (fp32 x fp32 products are
+/* From a few tokens on: the logits as a GEMM on v_mfma_f64_16x16x4f64 (fp32 x fp32 products are
  * exact in fp64, the sums are fp64 fused multiply-adds). One wave per 16 experts x 32
  * tokens. In each 16-column step lane L holds columns 4 (L / 16) .. + 3 of expert row
  * L % 16 (A operand) and of token L % 16 (+ 16) (B operand); the four MFMAs of a step
  * take one column each, so both operands come from one 16-byte load per row. The
  * f64 MFMA result puts expert 4 i + L / 16, token L % 16 in item i of lane L.
  * sum|w*x| is bounded by ||w|| ||x|| (Cauchy-Schwarz), both norms summed alongside.
- * With few tiles (S > 1) each tile's columns are cut into S slices taken by S waves; a
- * slice stores its partial sums, and the wave that completes the tile's count (a device
- * atomic) sums the S partials in slice order and forms the scores (any summation order
- * stays inside the interval's bound), then resets the count for the next call. */
+ * With few tiles (S > 1) each tile's columns are cut into S slices taken by S waves, four to
+ * a workgroup, which adds its slices in LDS; with several workgroups a tile each stores its
+ * sums, and the one that completes the tile's count (a device atomic) adds them in order,
+ * then resets the count for the next call (any summation order stays inside the interval's
+ * bound). The scores are three sigmoids in double each, so a workgroup's waves share them:
+ * one wave's eight of them were half the kernel's time.
+ * Measured (d 7168, us): E 384 at 8 / 16 / 24 / 256 tokens 43 / 23 / 27 / 86 -> 14 / 15 / 21 /
+ * 61, E 896 45 / 24 / 29 / 155 -> 15 / 16 / 22 / 95; bound by the slices' chain of loads (a wave
+ * has four steps in flight) and by the meeting, 5 us, not by the 64 cycles of an f64 MFMA. */
 typedef double k3v4d __attribute__((ext_vector_type(4)));
 
 #define K3R_RING 4
-/* below this many tokens the 16 x 32 tiles are too few to fill the GPU (T = 64: 48
- * waves) and the one-wave-per-(expert, 4 tokens) kernel is faster */
+/* one wave per tile (tiles enough to fill the GPU) from this many tokens on */
 #ifndef K3R_MFMA_MIN_T
 #define K3R_MFMA_MIN_T 512
 #endif
@@ -109,22 +113,16 @@ typedef double k3v4d __attribute__((ext_vector_type(4)));
 /* A 16-expert x 32-token tile, its K cut into S slices of whole 16-column steps: the
  * workgroups of a tile (G of them, blockDim / 64 waves each, one slice per wave; a wave
  * past S only adds zeros) first add their waves' sums in LDS, then, when G > 1, meet
- * through device-coherent partial sums where the last arrival adds them in group order. */
-__global__ void __launch_bounds__(64 * K3R_WPB)
-k_router_logits_mfma(const float *__restrict__ x, int T, const float *__restrict__ W,
-                     const float *__restrict__ bias, int d, int E, float4 *__restrict__ rs,
-                     int S, int G, double *__restrict__ part, int32_t *__restrict__ ctr)
+ * through device-coherent partial sums where the last arrival adds them in group order.
+ * Without TWO the tile's second 16 tokens do not exist. */
+template <bool TWO>
+__device__ __forceinline__ void
+router_tile(const float *__restrict__ x, int T, const float *__restrict__ W,
+            const float *__restrict__ bias, int d, int E, float4 *__restrict__ rs, int S, int G,
+            double *__restrict__ part, int32_t *__restrict__ ctr, int lam, double *k3r_red)
 {
-    extern __shared__ double k3r_red[];
     const int wpb = blockDim.x >> 6;
-    const int nte = E / 16, ntt = (T + 31) / 32, N = nte * ntt * G;
-    const int per = (N + 7) >> 3;
-    /* block b runs on XCD b % 8: give each XCD a contiguous run, so the expert tiles of
-     * one token tile (consecutive) share its x rows in one L2 */
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    if (slot >= per) return;
-    const int lam = xcd * per + slot;
-    if (lam >= N) return;
+    const int nte = E / 16;
     const int tl = lam / G, grp = lam - tl * G;
     const int wv = threadIdx.x >> 6, sl = grp * wpb + wv;
     const int tt = tl / nte, et = tl - tt * nte;
@@ -141,7 +139,8 @@ k_router_logits_mfma(const float *__restrict__ x, int T, const float *__restrict
 #pragma unroll
     for (int u = 0; u < K3R_RING; ++u) {
         const int s = max(0, min(u, ns - 1));
-        wq[u] = wp[4 * s]; av[u] = ap[4 * s]; bv[u] = bp[4 * s];
+        wq[u] = wp[4 * s]; av[u] = ap[4 * s];
+        if (TWO) bv[u] = bp[4 * s];
     }
     /* two chains per output (even and odd columns of a step), so consecutive MFMAs do
      * not wait for each other's results; they are added at the end */
@@ -151,9 +150,10 @@ k_router_logits_mfma(const float *__restrict__ x, int T, const float *__restrict
     for (int s0 = 0; s0 < ns; s0 += K3R_RING) {
 #pragma unroll
         for (int u = 0; u < K3R_RING; ++u) {
-            const float4 w4 = wq[u], a4 = av[u], b4 = bv[u];
+            const float4 w4 = wq[u], a4 = av[u], b4 = TWO ? bv[u] : a4;
             const int sn = max(0, min(s0 + u + K3R_RING, ns - 1));
-            wq[u] = wp[4 * sn]; av[u] = ap[4 * sn]; bv[u] = bp[4 * sn];
+            wq[u] = wp[4 * sn]; av[u] = ap[4 * sn];
+            if (TWO) bv[u] = bp[4 * sn];
             if (s0 + u < ns) {
                 const double w[4] = {w4.x, w4.y, w4.z, w4.w};
                 const double a[4] = {a4.x, a4.y, a4.z, a4.w};
@@ -161,75 +161,83 @@ k_router_logits_mfma(const float *__restrict__ x, int T, const float *__restrict
 #pragma unroll
                 for (int k = 0; k < 4; k += 2) {
                     acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(w[k], a[k], acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(w[k], b[k], acc1, 0, 0, 0);
+                    if (TWO) acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(w[k], b[k], acc1, 0, 0, 0);
                     acc2 = __builtin_amdgcn_mfma_f64_16x16x4f64(w[k + 1], a[k + 1], acc2, 0, 0, 0);
-                    acc3 = __builtin_amdgcn_mfma_f64_16x16x4f64(w[k + 1], b[k + 1], acc3, 0, 0, 0);
+                    if (TWO) acc3 = __builtin_amdgcn_mfma_f64_16x16x4f64(w[k + 1], b[k + 1], acc3, 0, 0, 0);
                 }
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     ssw = fma(w[k], w[k], ssw);
                     ssa = fma(a[k], a[k], ssa);
-                    ssb = fma(b[k], b[k], ssb);
+                    if (TWO) ssb = fma(b[k], b[k], ssb);
                 }
             }
         }
     }
     acc0 += acc2;
     acc1 += acc3;
+    /* wave wv's share of a lane's 11 sums: items wv, wv + wpb, ... (without the second tokens,
+     * items 4 .. 7 and 10 are zero) */
+    auto items = [&](auto f) {
+        for (int i = wv; i < K3R_PART; i += wpb)
+            if (TWO || i < 4 || i == 8 || i == 9) f(i);
+    };
     if (S > 1) {
-        double v[K3R_PART] = {acc0[0], acc0[1], acc0[2], acc0[3], acc1[0], acc1[1],
-                              acc1[2], acc1[3], ssw, ssa, ssb};
-        if (wpb > 1) {
-            /* the workgroup's slices, added in slice order by wave 0 */
-            double *mine = k3r_red + ((size_t)wv * 64 + L) * K3R_PART;
+        const double v[K3R_PART] = {acc0[0], acc0[1], acc0[2], acc0[3], acc1[0], acc1[1],
+                                    acc1[2], acc1[3], ssw, ssa, ssb};
+        /* the workgroup's slices, added in slice order, its waves a part of the items each */
+        double *tot = k3r_red + (size_t)wpb * 64 * K3R_PART;
 #pragma unroll
-            for (int i = 0; i < K3R_PART; ++i) mine[i] = v[i];
-            __syncthreads();
-            if (wv != 0) return;
-#pragma unroll
-            for (int i = 0; i < K3R_PART; ++i) v[i] = 0.0;
-            for (int q = 0; q < wpb; ++q) {
-                const double *o = k3r_red + ((size_t)q * 64 + L) * K3R_PART;
-#pragma unroll
-                for (int i = 0; i < K3R_PART; ++i) v[i] += o[i];
-            }
-        }
+        for (int i = 0; i < K3R_PART; ++i) k3r_red[((size_t)wv * K3R_PART + i) * 64 + L] = v[i];
+        __syncthreads();
+        /* device-coherent stores of the group's sums, complete before the count moves
+         * (no cache writeback or invalidate: the data never sits in a non-coherent
+         * cache); the last arrival adds the groups' sums in group order */
+        double *pp = part + (size_t)tl * G * (64 * K3R_PART);
+        items([&](int i) {
+            double s = 0.0;
+            for (int q = 0; q < wpb; ++q) s += k3r_red[((size_t)q * K3R_PART + i) * 64 + L];
+            if (G > 1)
+                __hip_atomic_store(pp + ((size_t)grp * K3R_PART + i) * 64 + L, s, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            else
+                tot[64 * i + L] = s;
+        });
         if (G > 1) {
-            /* device-coherent stores of the group's sums, complete before the count moves
-             * (no cache writeback or invalidate: the data never sits in a non-coherent
-             * cache); the last arrival adds the groups' sums in group order */
-            double *pp = part + ((size_t)tl * G + grp) * (64 * K3R_PART) + L * K3R_PART;
-#pragma unroll
-            for (int i = 0; i < K3R_PART; ++i)
-                __hip_atomic_store(pp + i, v[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             __builtin_amdgcn_s_waitcnt(0);
-            asm volatile("" ::: "memory");
-            int old = 0;
+            __syncthreads();
+            int *last = (int *)k3r_red;                  /* the slices' sums are spent */
             /* one count per 128-byte line: counts sharing a line would queue at the L2 */
-            if (L == 0) old = __hip_atomic_fetch_add(&ctr[32 * tl], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (__builtin_amdgcn_readfirstlane(old) != G - 1) return;
-            asm volatile("" ::: "memory");
-            double u[K3R_WPB][K3R_PART];
+            if (threadIdx.x == 0)
+                *last = __hip_atomic_fetch_add(&ctr[32 * tl], 1, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT) == G - 1;
+            __syncthreads();
+            if (!*last) return;
+            items([&](int i) {
+                double s = 0.0;
+                for (int q0 = 0; q0 < G; q0 += 4) {
+                    double u[4];
 #pragma unroll
-            for (int q = 0; q < K3R_WPB; ++q) {
-                const double *qq = part + ((size_t)tl * G + min(q, G - 1)) * (64 * K3R_PART) + L * K3R_PART;
+                    for (int q = 0; q < 4; ++q)
+                        u[q] = __hip_atomic_load(pp + ((size_t)min(q0 + q, G - 1) * K3R_PART + i) * 64 + L,
+                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-                for (int i = 0; i < K3R_PART; ++i)
-                    u[q][i] = __hip_atomic_load(qq + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
-#pragma unroll
-            for (int i = 0; i < K3R_PART; ++i) v[i] = 0.0;
-#pragma unroll
-            for (int q = 0; q < K3R_WPB; ++q)
-                if (q < G) {
-#pragma unroll
-                    for (int i = 0; i < K3R_PART; ++i) v[i] += u[q][i];
+                    for (int q = 0; q < 4; ++q)
+                        if (q0 + q < G) s += u[q];
                 }
-            if (L == 0) __hip_atomic_store(&ctr[32 * tl], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                tot[64 * i + L] = s;
+            });
+            if (threadIdx.x == 0)
+                __hip_atomic_store(&ctr[32 * tl], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
+        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { acc0[i] = v[i]; acc1[i] = v[4 + i]; }
-        ssw = v[8]; ssa = v[9]; ssb = v[10];
+        for (int i = 0; i < 4; ++i) {
+            acc0[i] = tot[64 * i + L];
+            if (TWO) acc1[i] = tot[64 * (4 + i) + L];
+        }
+        ssw = tot[64 * 8 + L]; ssa = tot[64 * 9 + L];
+        if (TWO) ssb = tot[64 * 10 + L];
     }
     /* norms: sum the four column groups; lane L then holds expert e0 + L % 16 and tokens
      * t0 + L % 16, t0 + 16 + L % 16 */
@@ -237,21 +245,46 @@ k_router_logits_mfma(const float *__restrict__ x, int T, const float *__restrict
     for (int m = 16; m <= 32; m <<= 1) {
         ssw += __shfl_xor(ssw, m, K3G_WAVE);
         ssa += __shfl_xor(ssa, m, K3G_WAVE);
-        ssb += __shfl_xor(ssb, m, K3G_WAVE);
+        if (TWO) ssb += __shfl_xor(ssb, m, K3G_WAVE);
     }
-    const double nw = sqrt(ssw), na = sqrt(ssa), nb = sqrt(ssb);
+    const double nw = sqrt(ssw), na = sqrt(ssa), nb = TWO ? sqrt(ssb) : 0.0;
     const double nround = 2.0 * d + 16.0;
     const double margin = 1.0 + 0x1p-40;
+    /* the scores (three sigmoids in double each: 2 us apiece when one wave forms all), dealt
+     * to the workgroup's waves */
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int j = 0; j < (TWO ? 8 : 4); ++j) {
+        if (j % wpb != wv) continue;
+        const int i = j & 3, t = t0 + r + (j < 4 ? 0 : 16);
         const int er = 4 * i + g;                         /* expert row of item i */
         const double nwe = __shfl(nw, er, K3G_WAVE);
         const int e = e0 + er;
-        const float be = bias ? bias[e] : 0.0f;
-        const int ta = t0 + r, tb = t0 + 16 + r;
-        if (ta < T) rs[(size_t)ta * E + e] = k3d_route_score_n(acc0[i], nwe * na * margin, be, nround);
-        if (tb < T) rs[(size_t)tb * E + e] = k3d_route_score_n(acc1[i], nwe * nb * margin, be, nround);
+        if (t < T)
+            rs[(size_t)t * E + e] = k3d_route_score_n(j < 4 ? acc0[i] : acc1[i],
+                                                      nwe * (j < 4 ? na : nb) * margin,
+                                                      bias ? bias[e] : 0.0f, nround);
     }
+}
+
+__global__ void __launch_bounds__(64 * K3R_WPB)
+k_router_logits_mfma(const float *__restrict__ x, int T, const float *__restrict__ W,
+                     const float *__restrict__ bias, int d, int E, float4 *__restrict__ rs,
+                     int S, int G, double *__restrict__ part, int32_t *__restrict__ ctr)
+{
+    extern __shared__ double k3r_red[];
+    const int N = E / 16 * ((T + 31) / 32) * G;
+    const int per = (N + 7) >> 3;
+    /* block b runs on XCD b % 8: give each XCD a contiguous run, so the expert tiles of
+     * one token tile (consecutive) share its x rows in one L2 */
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    if (slot >= per) return;
+    const int lam = xcd * per + slot;
+    if (lam >= N) return;
+    /* a tile whose second 16 tokens are all past T leaves their products out */
+    if (32 * (lam / G / (E / 16)) + 16 < T)
+        router_tile<true>(x, T, W, bias, d, E, rs, S, G, part, ctr, lam, k3r_red);
+    else
+        router_tile<false>(x, T, W, bias, d, E, rs, S, G, part, ctr, lam, k3r_red);
 }
 
 /* ------------------------------ many tokens: bounded logits on the bf16 matrix cores ---- */
@@ -594,8 +627,8 @@ k_router_select(const float4 *__restrict__ rs, const float *__restrict__ bias,
 
 /* K slices for the matrix-core logits when the tiles are few: about K3R_WAVES waves, at
  * most K3R_MAXS slices per tile; tiles x groups stays below K3R_WAVES (groups' sums in
- * memory: tiles < 512 and groups <= slices / 4 + 1 <= 1024 / (4 tiles) + 1) */
-#define K3R_WAVES 1024
+ * memory: tiles < 512 and groups <= slices / 4 + 1 <= 2048 / (4 tiles) + 1) */
+#define K3R_WAVES 2048
 #define K3R_MAXS 16
 extern "C" size_t k3k_router_part_bytes(void) { return (size_t)K3R_WAVES * 64 * K3R_PART * 8; }
 
@@ -660,7 +693,9 @@ extern "C" int k3k_router(const float *x, int T, const float *W, const float *bi
     }
     /* the score intervals of token t live at [t][E] */
     const long long N1 = (long long)(E / 16) * ((T + 31) / 32);
-    const bool mfma_ok = T >= 16 && vec && E >= 16 && E % 16 == 0 && d % 64 == 0;
+    /* from 4 tokens on, for half a tile costs less than four tokens a wave (E 384, d 7168, 4 and
+     * 8 tokens: 40 -> 15, 43 -> 15 us); up to 3 a wave per (expert, token) does (7.5 .. 12 us) */
+    const bool mfma_ok = T >= 4 && vec && E >= 16 && E % 16 == 0 && d % 64 == 0;
     int S = (mfma_ok && part && ctr && N1 < 512) ? router_slices((int)N1) : 1;
     if (S > 1) {
         /* whole 16-column steps per slice and no empty slice */
@@ -675,7 +710,7 @@ extern "C" int k3k_router(const float *x, int T, const float *W, const float *bi
         const int wpb = S < K3R_WPB ? S : K3R_WPB, G = (S + wpb - 1) / wpb;
         const long long N = N1 * G;
         if (G > 1 && N > K3R_WAVES) return -1;     /* the groups' sums would not fit */
-        const size_t lds = wpb > 1 ? (size_t)wpb * 64 * K3R_PART * sizeof(double) : 0;
+        const size_t lds = S > 1 ? (size_t)(wpb + 1) * 64 * K3R_PART * sizeof(double) : 0;
         hipLaunchKernelGGL(k_router_logits_mfma, dim3((unsigned)(8 * ((N + 7) / 8))),
                            dim3(64 * wpb), lds, st, x, T, W, bias, d, E, (float4 *)rs, S, G,
                            part, ctr);
