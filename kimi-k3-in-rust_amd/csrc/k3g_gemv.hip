@@ -396,6 +396,17 @@ extern "C" int k3k_routed_down(const K3kRouted *a, int maxU, int maxtok, hipStre
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+/* Rows per wave of a bf16 product: the most, up to nr (more reuse of x), that still gives two
+ * workgroups per CU. 2 x 2048 rows of 7168 at 8 rows a wave are 64 workgroups: 4 tokens 85 us, 1
+ * token 69; at 2 (256 workgroups) 30 and 23, at 1 (512) 24 and 16. 7168 rows of 2048 at 8 and
+ * 16 rows: 27 and 26 us, at 4 rows 16 and 10; 1024 workgroups are no faster. */
+#define DENSE_WG 512
+static int dense_rows(int rows, int ty, int nr)
+{
+    while (nr > 1 && (long long)((rows + 4 * nr - 1) / (4 * nr)) * ty < DENSE_WG) nr /= 2;
+    return nr;
+}
+
 extern "C" int k3k_dense(int fmt, const void *Wa, const void *Wb, int rows, int in,
                          const float *x, int ldx, int T, float *y, int ldy, float b1,
                          float b2, hipStream_t st)
@@ -423,25 +434,32 @@ extern "C" int k3k_dense(int fmt, const void *Wa, const void *Wb, int rows, int 
     constexpr int NR = 8, NT = 4;
     dim3 g((rows + 4 * NR - 1) / (4 * NR), (T + NT - 1) / NT);
     if (fmt == K3K_BF16) {
-        if (Wb) {
-            if (T == 1)
-                hipLaunchKernelGGL((k_dense<K3K_BF16, NR, 1, true>),
-                                   dim3(g.x, T), dim3(256), 0, st, Wa, Wb, nullptr, nullptr,
-                                   rows, in, x, ldx, T, y, ldy, b1, b2);
-            else
-                hipLaunchKernelGGL((k_dense<K3K_BF16, NR, NT, true>), g, dim3(256), 0, st,
-                                   Wa, Wb, nullptr, nullptr, rows, in, x, ldx, T, y, ldy,
-                                   b1, b2);
+        auto go = [&](auto kern, int nr, int nt) {
+            hipLaunchKernelGGL(kern, dim3((rows + 4 * nr - 1) / (4 * nr), (T + nt - 1) / nt),
+                               dim3(256), 0, st, Wa, Wb, nullptr, nullptr, rows, in, x, ldx, T, y,
+                               ldy, b1, b2);
+        };
+        const int nr = dense_rows(rows, (T + NT - 1) / NT, !Wb && T == 1 ? 16 : 8);
+        if (Wb && T == 1) {
+            if (nr == 8) go(k_dense<K3K_BF16, 8, 1, true>, 8, 1);
+            else if (nr == 4) go(k_dense<K3K_BF16, 4, 1, true>, 4, 1);
+            else if (nr == 2) go(k_dense<K3K_BF16, 2, 1, true>, 2, 1);
+            else go(k_dense<K3K_BF16, 1, 1, true>, 1, 1);
+        } else if (Wb) {
+            if (nr == 8) go(k_dense<K3K_BF16, 8, NT, true>, 8, NT);
+            else if (nr == 4) go(k_dense<K3K_BF16, 4, NT, true>, 4, NT);
+            else if (nr == 2) go(k_dense<K3K_BF16, 2, NT, true>, 2, NT);
+            else go(k_dense<K3K_BF16, 1, NT, true>, 1, NT);
+        } else if (T == 1) {
+            if (nr == 16) go(k_dense<K3K_BF16, 16, 1, false>, 16, 1);
+            else if (nr == 8) go(k_dense<K3K_BF16, 8, 1, false>, 8, 1);
+            else if (nr == 4) go(k_dense<K3K_BF16, 4, 1, false>, 4, 1);
+            else go(k_dense<K3K_BF16, 2, 1, false>, 2, 1);
         } else {
-            if (T == 1)
-                hipLaunchKernelGGL((k_dense<K3K_BF16, 2 * NR, 1, false>),
-                                   dim3((rows + 8 * NR - 1) / (8 * NR), T), dim3(256), 0, st,
-                                   Wa, Wb, nullptr, nullptr, rows, in, x, ldx, T, y, ldy,
-                                   b1, b2);
-            else
-                hipLaunchKernelGGL((k_dense<K3K_BF16, NR, NT, false>), g, dim3(256), 0, st,
-                                   Wa, Wb, nullptr, nullptr, rows, in, x, ldx, T, y, ldy,
-                                   b1, b2);
+            if (nr == 8) go(k_dense<K3K_BF16, 8, NT, false>, 8, NT);
+            else if (nr == 4) go(k_dense<K3K_BF16, 4, NT, false>, 4, NT);
+            else if (nr == 2) go(k_dense<K3K_BF16, 2, NT, false>, 2, NT);
+            else go(k_dense<K3K_BF16, 1, NT, false>, 1, NT);
         }
     } else if (fmt == K3K_F32) {
         if (Wb)

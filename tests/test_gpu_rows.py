@@ -1,6 +1,8 @@
 """The routed experts of checkpoint-layout MXFP4 weights (six FP6 pieces on the FP4 x FP6 matrix
 cores) at the edges of their tiles, through k3g_expert_gemv, against the expert products in float64
 on the exactly dequantised weights."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -110,3 +112,30 @@ def test_not_finite(gpu):
     assert np.isinf(want).any() and np.isnan(want).any()
     assert np.array_equal(got[2, 0], want.astype(np.float32), equal_nan=True)
     assert np.array_equal(got[[1, 3]].view(np.uint32), clean[[1, 3]].view(np.uint32))
+
+
+# each count of rows per wave (16 .. 1 by the number of row tiles and tokens), rows that do not
+# fill the last wave, widths below and past a wave's 1024 columns
+@pytest.mark.parametrize("T", [1, 4, 5])
+@pytest.mark.parametrize("rows,K", [(37, 16), (2051, 1040), (4097, 48), (8195, 32), (16390, 16),
+                                    (32780, 16)])
+def test_dense_rows_per_wave(gpu, T, rows, K):
+    """bf16 products by row, alone and as silu(a) b, against float64: K fp32 multiply-adds."""
+    print(f"case: k3k_dense bf16 {rows} x {K}, {T} tokens", flush=True)
+    rng = np.random.default_rng(rows + K)
+    a, b = (rng.standard_normal((rows, K)).astype(np.float32).view(np.uint32) >> 16
+            for _ in range(2))
+    x = rng.standard_normal((T, K)).astype(np.float32)
+    fa, fb = ((v << 16).astype(np.uint32).view(np.float32).astype(np.float64) for v in (a, b))
+    da, db = (k3moe.DevBuf.from_array(v.astype(np.uint16)) for v in (a, b))
+    dx, dy = k3moe.DevBuf.from_array(x), k3moe.DevBuf(T * rows * 4)
+    fn = k3moe.lib().k3k_dense
+    fn.argtypes = [C.c_int, C.c_void_p, C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_int, C.c_int,
+                   C.c_void_p, C.c_int, C.c_float, C.c_float, C.c_void_p]
+    g, u = x @ fa.T, x @ fb.T
+    for wb, want in ((None, g), (db.ptr, g / (1.0 + np.exp(-g)) * u)):
+        assert fn(2, da.ptr, wb, rows, K, dx.ptr, K, T, dy.ptr, rows, k3moe.SWIGLU_CAP,
+                  k3moe.SWIGLU_CAP, None) == 0
+        k3moe.sync()
+        got = dy.download(np.float32, T * rows).reshape(T, rows)
+        assert np.linalg.norm(got - want) <= 1e-6 * np.linalg.norm(want)
