@@ -18,13 +18,15 @@
  *    No weight is ever decoded by the vector ALUs.
  *
  * 2. The work is cut into tickets, ordered so that whatever a ticket depends on has a
- *    smaller ticket, and wave w of a co-resident persistent grid of W waves takes
- *    tickets w, w + W, w + 2W, ... (a shared ticket counter would cost one contended
- *    device atomic per ticket):
+ *    smaller ticket, and wave w of a co-resident persistent grid of W waves starts with
+ *    ticket w. At one token it goes on with w + W, w + 2W, ...; at more it takes the next
+ *    ticket of its stripe (tickets w mod K3_STRIPES) from the stripe's counter, so that the
+ *    waves that got the long or late tickets take fewer (one counter for all would cost a
+ *    contended device atomic per ticket):
  *
  *      X   x -> FP8 pieces (per token, per 512 columns) and bf16 pieces
  *      R   router logits of one expert row (all tokens), fp64 with an error bound
- *      S   the certified top-k for every token (one ticket); waits for all R
+ *      S   the certified top-k of one token; waits for all R
  *      SG  shared gate/up: 16 SG_TILES rows x a K slice; the last slice of a row group
  *          (found with a returning atomic) sums the slices in slice order, applies the
  *          activation and writes the shared h as bf16 pieces
@@ -49,7 +51,9 @@
  * ordered on the stream, has finished with) for the next call. So the per-call counts
  * may change from call to call (a different token count or layer).
  *
- * Deadlock freedom: a ticket only waits on smaller tickets, all waves are resident at
+ * Deadlock freedom: a ticket only waits on smaller tickets, a stripe's tickets are taken in
+ * order (so the smallest unfinished ticket is in some wave's hands or its stripe has a free
+ * wave), all waves are resident at
  * once (the grid is sized by the occupancy calculator), and every wait is bounded (an
  * exhausted wait raises K3G_ERR_WAIT and the wave moves on, so every wave reaches the
  * exit).
@@ -86,6 +90,11 @@ typedef unsigned int k3v4u __attribute__((ext_vector_type(4)));
 #define NREP 16
 #define REP_STRIDE 4      /* lines between copies */
 #define K3_EVLINES (NREP * REP_STRIDE)
+/* Ticket counters for T > 1, 64 waves of one XCD each on 4096. Measured, K2 layer, taking the next
+ * ticket so and one K slice a routed down ticket: 2 / 3 / 4 tokens 122 / 176 / 220 -> 114 / 159 / 198
+ * us. At one token the launch is two and a half tickets a wave, and the count's round trip costs
+ * what the balance gives (71 -> 72, K3 159 -> 164 us). */
+#define K3_STRIPES 64
 
 /* ------------------------------------------------------------ geometry ---- */
 /* Ticket classes in order: X R S [LD] SG SD G D [NR LU]. The bracketed ones exist only for
@@ -100,13 +109,13 @@ struct K3Geo {
     int KSS, KSG, KSD, KSR, KSDN; /* K slices of SG, G, SD, R, D tickets */
     int nRc;                     /* router 1024-column chunks */
     int nSGt, nGt, nSDt, nDt;    /* row tiles (SG: row groups of SG_TILES tiles) */
-    int nX, nR, nSG, nG, nSD, nD, total;
+    int nX, nR, nS, nSG, nG, nSD, nD, total;
     int oSG, oG, oSD, oD;        /* first ticket of each class after S */
     /* the latent layer */
     int lat, L, Dout, nQk;       /* L; D's output rows (L or d); G's K in 512-column quads */
     int nCL, KSLD, KSLU, nLDt, nLUt, nNR, nLD, nLU, oLD, oNR, oLU;
     /* counter lines */
-    int lR, lSD, lD, lTSG, lTG, lRE, lDT, lLD, lLU, cX, cX16, cR, cSGF, cGF, cZ, cA, cN, eX,
+    int lR, lSD, lD, lTSG, lTG, lRE, lDT, lLD, lLU, lS, lTK, cX, cX16, cR, cSGF, cGF, cZ, cA, cN, eX,
         eX16, eR, eSEL, eSGF, eGF, eZ, eA, eN, cOD, nlines;
 };
 
@@ -135,7 +144,8 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.KSD = SI > 0 ? (ksd < g.nCsi ? ksd : g.nCsi) : 0;
     g.nRc = (d + 1023) / 1024;
     g.KSR = ksr < g.nRc ? ksr : g.nRc;
-    g.KSDN = ksdn < g.nQi ? ksdn : g.nQi;
+    /* one token's down tickets, unsliced, would leave half the waves without one */
+    g.KSDN = T > 1 ? 1 : ksdn < g.nQi ? ksdn : g.nQi;
     g.KSLD = g.lat ? (K3G_KS_LD < g.nCd ? K3G_KS_LD : g.nCd) : 0;
     g.KSLU = g.lat ? (K3G_KS_LU < g.nCL ? K3G_KS_LU : g.nCL) : 0;
     g.nSGt = (SI + 16 * SG_TILES - 1) / (16 * SG_TILES);
@@ -147,13 +157,17 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.nNR = g.lat ? (L + 63) / 64 : 0;
     g.nX = T * ((g.nCd + 1) / 2);
     g.nR = E * g.KSR;
+    /* one select per token, in workgroups of their own (4 waves each, the selection's LDS is
+     * the workgroup's): of every four tickets the first works. One ticket for all tokens took 7 us
+     * a token: 42 us until the routed weights started at 3 tokens, 27 so */
+    g.nS = 4 * (T - 1) + 1;
     g.nLD = g.nLDt * g.KSLD;
     g.nSG = g.nSGt * g.KSS;
     g.nG = g.P * g.nGt * g.KSG;
     g.nSD = g.nSDt * g.KSD;
     g.nD = g.P * g.nDt * g.KSDN;
     g.nLU = g.nLUt * g.KSLU;
-    g.oLD = g.nX + g.nR + 1;
+    g.oLD = g.nX + g.nR + g.nS;
     g.oSG = g.oLD + g.nLD;
     g.oSD = g.oSG + g.nSG;
     g.oG = g.oSD + g.nSD;
@@ -172,7 +186,9 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.lLD = g.lDT + g.nDt;
     g.lLU = g.lLD + g.nLDt;
     /* event counters: a top line and NSUB sub-counter lines each (k3d_arrive_event2) */
-    g.cX = g.lLU + g.nLUt;
+    g.lS = g.lLU + g.nLUt;
+    g.lTK = g.lS + 1;
+    g.cX = g.lTK + K3_STRIPES;
     g.cX16 = g.cX + 1 + NSUB;
     g.cR = g.cX16 + 1 + NSUB;
     g.cSGF = g.cR + 1 + NSUB;
@@ -184,7 +200,7 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.eX16 = g.eX + K3_EVLINES;
     g.eR = g.eX16 + K3_EVLINES;
     g.eSEL = g.eR + K3_EVLINES;
-    g.eSGF = g.eSEL + K3_EVLINES;
+    g.eSGF = g.eSEL + T * K3_EVLINES;
     g.eZ = g.eSGF + K3_EVLINES;
     g.eA = g.eZ + K3_EVLINES;
     g.eN = g.eA + K3_EVLINES;
@@ -223,6 +239,16 @@ __device__ __forceinline__ bool k3d_arrive(int *ctr, int last_old, int lane)
     old = __builtin_amdgcn_readfirstlane(old);
     asm volatile("" ::: "memory");
     return old == last_old;
+}
+
+/* k3d_arrive that also takes the wave's next ticket from its stripe's counter (if any): the two
+ * round trips, of the stores and of the count, pass together. */
+__device__ __forceinline__ bool k3d_arrive_next(int *ctr, int last_old, int lane, int *count,
+                                                int &next)
+{
+    if (lane == 0 && count)
+        next = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return k3d_arrive(ctr, last_old, lane);
 }
 
 /* Wait until the counters line(first) .. line(first + n - 1) sum to at least target.
@@ -646,40 +672,35 @@ struct K3Dec {
         double acc[NT], ab[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) { acc[t] = 0.0; ab[t] = 0.0; }
-        for (int cb = ch0; cb < ch1; cb += 2) {
-            /* two 1024-column chunks per batch; columns past the slice or the row read
-             * zero */
-            uint4 W[8];
+        /* CH 1024-column chunks per batch, the rows of every token loaded before any is used
+         * (behind the shared expert's weights a round trip takes 4 us); columns past the slice
+         * or the row read zero */
+        constexpr int CH = NT <= 2 ? 2 : 1;
+        for (int cb = ch0; cb < ch1; cb += CH) {
+            uint4 W[4 * CH], X[NT][4 * CH];
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int col = (cb + h) * 1024 + lane * 16;
-                const bool on = cb + h < ch1 && col < a.d;
+            for (int h = 0; h < CH; ++h)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) W[4 * h + i] = k3d_b128(rg, on ? col * 4 + 16 * i : K3_OOB);
-            }
+                for (int i = 0; i < 4; ++i) {
+                    const int col = (cb + h) * 1024 + 256 * i + 4 * lane;
+                    const bool on = cb + h < ch1 && col < a.d;
+                    W[4 * h + i] = k3d_b128(rg, on ? col * 4 : K3_OOB);
+#pragma unroll
+                    for (int t = 0; t < NT; ++t)
+                        X[t][4 * h + i] = k3d_b128(rx, on && t < a.T ? (t * a.d + col) * 4 : K3_OOB);
+                }
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                if (t < a.T) {
-                    uint4 X[8];
 #pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const int col = (cb + h) * 1024 + lane * 16;
-                        const bool on = cb + h < ch1 && col < a.d;
+                for (int i = 0; i < 4 * CH; ++i) {
+                    const float w4[4] = {__uint_as_float(W[i].x), __uint_as_float(W[i].y),
+                                         __uint_as_float(W[i].z), __uint_as_float(W[i].w)};
+                    const float x4[4] = {__uint_as_float(X[t][i].x), __uint_as_float(X[t][i].y),
+                                         __uint_as_float(X[t][i].z), __uint_as_float(X[t][i].w)};
 #pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            X[4 * h + i] = k3d_b128(rx, on ? (t * a.d + col) * 4 + 16 * i : K3_OOB);
-                    }
-#pragma unroll
-                    for (int i = 0; i < 8; ++i) {
-                        const float w4[4] = {__uint_as_float(W[i].x), __uint_as_float(W[i].y),
-                                             __uint_as_float(W[i].z), __uint_as_float(W[i].w)};
-                        const float x4[4] = {__uint_as_float(X[i].x), __uint_as_float(X[i].y),
-                                             __uint_as_float(X[i].z), __uint_as_float(X[i].w)};
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            acc[t] = fma((double)w4[q], (double)x4[q], acc[t]);
-                            ab[t] = fma(fabs((double)w4[q]), fabs((double)x4[q]), ab[t]);
-                        }
+                    for (int q = 0; q < 4; ++q) {
+                        acc[t] = fma((double)w4[q], (double)x4[q], acc[t]);
+                        ab[t] = fma(fabs((double)w4[q]), fabs((double)x4[q]), ab[t]);
                     }
                 }
             }
@@ -746,37 +767,41 @@ struct K3Dec {
     }
 
     /* ----------------------------------------------------------------- S ---- */
-    static __device__ __noinline__ void select(K3ArgPtr ap, int lane, K3SelectLds *lds)
+    static __device__ __noinline__ void select(K3ArgPtr ap, int tk_, int lane, K3SelectLds *lds)
     {
         const K3kDecode a = *k3d_uniform_cptr(ap);
+        const int tk = k3d_uniform(tk_), t = tk >> 2;
         const K3Geo G = k3_geo(a.T, a.d, a.E, a.k, a.I, a.SI, a.L);
+        if (tk & 3) return;
         if (a.given) {
             /* the routing came with the call: publish it once x's pieces exist */
+            if (tk) return;
             if (!k3d_wait_event(a.sync, G.eX, 0, a.spin_limit, a.err, lane)) return;
-            k3d_set_event(a.sync, G.eSEL, lane);
+            for (int i = 0; i < a.T; ++i) k3d_set_event(a.sync, G.eSEL + i * K3_EVLINES, lane);
             host_routing(a, lane);
             return;
         }
         /* the routed tickets also need x's pieces: the routing is published once both
          * exist. x's pieces are done long before the router rows, so their event is
          * checked first, off the path from the last row to the publication. */
-        if (!k3d_wait_event(a.sync, G.eX, 0, a.spin_limit, a.err, lane)) return;
-        /* every router row in: the select is the only waiter, so it reads the rows'
-         * sub-counters itself instead of waiting for the top count and the event flags
+        if (!k3d_wait_event(a.sync, G.eX, t, a.spin_limit, a.err, lane)) return;
+        /* every router row in: the selects are the only waiters, so they read the rows'
+         * sub-counters themselves instead of waiting for the top count and the event flags
          * (one returning atomic and a flag store less on the routed experts' path) */
         if (!k3d_wait_sum(a.sync, G.cR + 1, NSUB, a.E, a.spin_limit, a.err, lane)) return;
         /* instrumentation: after the trace's [ticket][2] stamps, the select's own phases */
-        if (a.trace && lane == 0) a.trace[3 * G.total] = wall_clock64();
+        if (a.trace && t == 0 && lane == 0) a.trace[3 * G.total] = wall_clock64();
         /* everything routed waits for this wave: let it issue ahead of its SIMD's others */
         __builtin_amdgcn_s_setprio(3);
-        for (int t = 0; t < a.T; ++t)
-            k3d_select_token(lds, t, (const float4 *)a.rs, a.bias, a.gate, a.x, a.d, a.E, a.k,
-                             a.renorm, a.routed_scale, a.idx, a.wt, a.force, a.stats, lane,
-                             a.trace && t == 0 ? a.trace + 3 * G.total + 2 : nullptr);
-        if (a.trace && lane == 0) a.trace[3 * G.total + 1] = wall_clock64();
-        k3d_set_event(a.sync, G.eSEL, lane);
+        k3d_select_token(lds, t, (const float4 *)a.rs, a.bias, a.gate, a.x, a.d, a.E, a.k,
+                         a.renorm, a.routed_scale, a.idx, a.wt, a.force, a.stats, lane,
+                         a.trace && t == 0 ? a.trace + 3 * G.total + 2 : nullptr);
+        if (a.trace && t == 0 && lane == 0) a.trace[3 * G.total + 1] = wall_clock64();
+        k3d_set_event(a.sync, G.eSEL + t * K3_EVLINES, lane);
         __builtin_amdgcn_s_setprio(0);
-        host_routing(a, lane);
+        /* the host's copies, once every token's routing is in */
+        if (a.hidx && (a.T == 1 || k3d_arrive(k3d_line(a.sync, G.lS), a.T - 1, lane)))
+            host_routing(a, lane);
     }
 
     /* the published routing to the caller's host copies (after the event, off the routed
@@ -828,10 +853,12 @@ struct K3Dec {
     }
 
     /* ---------------------------------------------------------------- SG ---- */
-    static __device__ __noinline__ void shared_gateup(K3ArgPtr ap, int tk_, int lane)
+    static __device__ __noinline__ int shared_gateup(K3ArgPtr ap, int tk_, int lane, int *count_)
     {
         const K3kDecode a = *k3d_uniform_cptr(ap);
         const int tk = k3d_uniform(tk_);
+        int *count = k3d_uniform_ptr(count_);
+        int next = -1;
         const K3Geo G = k3_geo(a.T, a.d, a.E, a.k, a.I, a.SI, a.L);
         const int rg = tk / G.KSS, ks = tk - rg * G.KSS;    /* row group, K slice */
         const int c0 = ks * G.nCd / G.KSS, c1 = (ks + 1) * G.nCd / G.KSS;
@@ -878,7 +905,7 @@ struct K3Dec {
                 if (first) {
                     /* the first weights stream in while x's bf16 pieces are made */
                     if (!k3d_wait_event(a.sync, G.eX16, tk, a.spin_limit, a.err, lane))
-                        return;
+                        return next;
                     k3d_trace_go(a.trace, G.oSG + tk, lane);
                     first = false;
                 }
@@ -908,7 +935,7 @@ struct K3Dec {
                 k3d_st4_sc1(rp, (((ks * a.T + t) * 2 + 1) * a.SI + row) * 4, u[j]);
             }
         }
-        if (!k3d_arrive(k3d_line(a.sync, G.lTSG + rg), G.KSS - 1, lane)) return;
+        if (!k3d_arrive_next(k3d_line(a.sync, G.lTSG + rg), G.KSS - 1, lane, count, next)) return next;
         /* last slice of the row group: h = act(gate, up) for its 64 rows x T tokens (lane:
          * row) -> bf16 pieces */
         const int row = 16 * SG_TILES * rg + lane;
@@ -931,22 +958,25 @@ struct K3Dec {
             }
         }
         k3d_arrive_event2(a.sync, G.cSGF, G.nSGt, rg, G.eSGF, lane);
+        return next;
     }
 
     /* ----------------------------------------------------------------- G ---- */
-    static __device__ __noinline__ void routed_gateup(K3ArgPtr ap, int tk_, int lane)
+    static __device__ __noinline__ int routed_gateup(K3ArgPtr ap, int tk_, int lane, int *count_)
     {
         const K3kDecode a = *k3d_uniform_cptr(ap);
         const int tk = k3d_uniform(tk_);
+        int *count = k3d_uniform_ptr(count_);
+        int next = -1;
         const K3Geo G = k3_geo(a.T, a.d, a.E, a.k, a.I, a.SI, a.L);
         const int per = G.nGt * G.KSG;
         const int p = tk / per, rem = tk - p * per;
         const int gt = rem / G.KSG, ks = rem - gt * G.KSG;
         const int q0 = ks * G.nQk / G.KSG, q1 = (ks + 1) * G.nQk / G.KSG;
         const int t = p / a.k;
-        if (!k3d_wait_event(a.sync, G.eSEL, tk, a.spin_limit, a.err, lane)) return;
+        if (!k3d_wait_event(a.sync, G.eSEL + t * K3_EVLINES, tk, a.spin_limit, a.err, lane)) return next;
         /* the latent layer's routed input is z = down x */
-        if (G.lat && !k3d_wait_event(a.sync, G.eZ, tk, a.spin_limit, a.err, lane)) return;
+        if (G.lat && !k3d_wait_event(a.sync, G.eZ, tk, a.spin_limit, a.err, lane)) return next;
         k3d_trace_go(a.trace, G.oG + tk, lane);
         const int e = k3d_uniform(__hip_atomic_load(&a.idx[p], __ATOMIC_RELAXED,
                                                     __HIP_MEMORY_SCOPE_AGENT));
@@ -1013,8 +1043,8 @@ struct K3Dec {
                 k3d_st4_sc1(rp, (((p * G.KSG + ks) * 2 + (m >> 1)) * a.I + r4 + 16 * (m & 1)) * 4,
                             acc[m]);
         }
-        if (!k3d_arrive(k3d_line(a.sync, G.lTG + p * G.nGt + gt), G.KSG - 1, lane))
-            return;
+        if (!k3d_arrive_next(k3d_line(a.sync, G.lTG + p * G.nGt + gt), G.KSG - 1, lane, count, next))
+            return next;
         /* last slice of the tile: 32 rows of h = act(gate, up) -> FP8 pieces (one block) */
         const int r = lane & 31, row = 32 * gt + r;
         const float gs = k3d_sum_sc1<K3G_KS_G_MAX>(rp, ((p * G.KSG * 2 + 0) * a.I + row) * 4,
@@ -1034,13 +1064,16 @@ struct K3Dec {
             }
         }
         k3d_arrive_event2(a.sync, G.cGF + p * (1 + NSUB), G.nGt, gt, G.eGF + p * K3_EVLINES, lane);
+        return next;
     }
 
     /* ---------------------------------------------------------------- SD ---- */
-    static __device__ __noinline__ void shared_down(K3ArgPtr ap, int tk_, int lane)
+    static __device__ __noinline__ int shared_down(K3ArgPtr ap, int tk_, int lane, int *count_)
     {
         const K3kDecode a = *k3d_uniform_cptr(ap);
         const int tk = k3d_uniform(tk_);
+        int *count = k3d_uniform_ptr(count_);
+        int next = -1;
         const K3Geo G = k3_geo(a.T, a.d, a.E, a.k, a.I, a.SI, a.L);
         const int rt = tk / G.KSD, ks = tk - rt * G.KSD;
         const int c0 = ks * G.nCsi / G.KSD, c1 = (ks + 1) * G.nCsi / G.KSD;
@@ -1061,7 +1094,7 @@ struct K3Dec {
                 A1[i] = k3d_b128(r2, c < c1 ? o1 + c * 1024 : K3_OOB);
             }
             if (first) {   /* the first weights stream in while the shared h is finished */
-                if (!k3d_wait_event(a.sync, G.eSGF, tk, a.spin_limit, a.err, lane)) return;
+                if (!k3d_wait_event(a.sync, G.eSGF, tk, a.spin_limit, a.err, lane)) return next;
                 k3d_trace_go(a.trace, G.oSD + tk, lane);
                 first = false;
             }
@@ -1086,24 +1119,28 @@ struct K3Dec {
             k3d_st4_sc1(rp, ((ks * a.T + t) * a.d + row + 16) * 4, y1);
         }
         if (G.lat) {
-            if (k3d_arrive(k3d_line(a.sync, G.lLU + rt), G.KSLU + G.KSD - 1, lane))
+            if (k3d_arrive_next(k3d_line(a.sync, G.lLU + rt), G.KSLU + G.KSD - 1, lane, count, next))
                 combine_out(a, G, rt, lane);
-        } else if (k3d_arrive(k3d_line(a.sync, G.lDT + rt), G.P * G.KSDN + G.KSD - 1, lane)) {
+        } else if (k3d_arrive_next(k3d_line(a.sync, G.lDT + rt), G.P * G.KSDN + G.KSD - 1, lane, count, next)) {
             combine_rows(a, G, rt, lane);
         }
+        return next;
     }
 
     /* ----------------------------------------------------------------- D ---- */
-    static __device__ __noinline__ void routed_down(K3ArgPtr ap, int tk_, int lane)
+    static __device__ __noinline__ int routed_down(K3ArgPtr ap, int tk_, int lane, int *count_)
     {
         const K3kDecode a = *k3d_uniform_cptr(ap);
         const int tk = k3d_uniform(tk_);
+        int *count = k3d_uniform_ptr(count_);
+        int next = -1;
         const K3Geo G = k3_geo(a.T, a.d, a.E, a.k, a.I, a.SI, a.L);
         const int per = G.nDt * G.KSDN;
         const int p = tk / per, rem = tk - p * per;
         const int dt = rem / G.KSDN, ks = rem - dt * G.KSDN;
         const int q0 = ks * G.nQi / G.KSDN, q1 = (ks + 1) * G.nQi / G.KSDN;
-        if (!k3d_wait_event(a.sync, G.eSEL, tk, a.spin_limit, a.err, lane)) return;
+        if (!k3d_wait_event(a.sync, G.eSEL + p / a.k * K3_EVLINES, tk, a.spin_limit, a.err, lane))
+            return next;
         const int e = k3d_uniform(__hip_atomic_load(&a.idx[p], __ATOMIC_RELAXED,
                                                     __HIP_MEMORY_SCOPE_AGENT));
         k3v4f y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};
@@ -1128,7 +1165,7 @@ struct K3Dec {
                 if (first) {   /* the first weights stream in while this pair's h finishes */
                     if (!k3d_wait_event(a.sync, G.eGF + p * K3_EVLINES, tk, a.spin_limit,
                                         a.err, lane))
-                        return;
+                        return next;
                     k3d_trace_go(a.trace, G.oD + tk, lane);
                     first = false;
                 }
@@ -1161,11 +1198,12 @@ struct K3Dec {
         }
         if (G.lat) {
             /* the latent layer: the slots' aggregate (the shared expert joins after up) */
-            if (k3d_arrive(k3d_line(a.sync, G.lDT + dt), G.P * G.KSDN - 1, lane))
+            if (k3d_arrive_next(k3d_line(a.sync, G.lDT + dt), G.P * G.KSDN - 1, lane, count, next))
                 combine_latent(a, G, dt, lane);
-        } else if (k3d_arrive(k3d_line(a.sync, G.lDT + dt), G.P * G.KSDN + G.KSD - 1, lane)) {
+        } else if (k3d_arrive_next(k3d_line(a.sync, G.lDT + dt), G.P * G.KSDN + G.KSD - 1, lane, count, next)) {
             combine_rows(a, G, dt, lane);
         }
+        return next;
     }
 
     /* ---------------------------------------------------------------- LD ---- */
@@ -1173,10 +1211,12 @@ struct K3Dec {
      * pieces, as the shared gate/up reads them); the last slice of a row tile sums the
      * slices in slice order and writes the 32 values' FP8 pieces (one MX block) for the
      * routed gate/up (src/core/k3_ops.c:600: z = down x). */
-    static __device__ __noinline__ void latent_down(K3ArgPtr ap, int tk_, int lane)
+    static __device__ __noinline__ int latent_down(K3ArgPtr ap, int tk_, int lane, int *count_)
     {
         const K3kDecode a = *k3d_uniform_cptr(ap);
         const int tk = k3d_uniform(tk_);
+        int *count = k3d_uniform_ptr(count_);
+        int next = -1;
         const K3Geo G = k3_geo(a.T, a.d, a.E, a.k, a.I, a.SI, a.L);
         const int rt = tk / G.KSLD, ks = tk - rt * G.KSLD;
         const int c0 = ks * G.nCd / G.KSLD, c1 = (ks + 1) * G.nCd / G.KSLD;
@@ -1210,7 +1250,7 @@ struct K3Dec {
             } else {
                 if (first) {
                     if (!k3d_wait_event(a.sync, G.eX16, tk, a.spin_limit, a.err, lane))
-                        return;
+                        return next;
                     k3d_trace_go(a.trace, G.oLD + tk, lane);
                     first = false;
                 }
@@ -1234,7 +1274,7 @@ struct K3Dec {
             k3d_st4_sc1(rp, ((ks * a.T + t) * G.L + row) * 4, y0);
             k3d_st4_sc1(rp, ((ks * a.T + t) * G.L + row + 16) * 4, y1);
         }
-        if (!k3d_arrive(k3d_line(a.sync, G.lLD + rt), G.KSLD - 1, lane)) return;
+        if (!k3d_arrive_next(k3d_line(a.sync, G.lLD + rt), G.KSLD - 1, lane, count, next)) return next;
         /* last slice of the row tile: rows 32 rt + r (lane r < 32) of z -> FP8 pieces */
         const int r = lane & 31, row = 32 * rt + r;
         const K3Rsrc rz = k3d_rsrc(a.zq8, (size_t)a.T * G.nQk * K3G_BQ);
@@ -1255,6 +1295,7 @@ struct K3Dec {
             }
         }
         k3d_arrive_event2(a.sync, G.cZ, G.nLDt, rt, G.eZ, lane);
+        return next;
     }
 
     /* ---------------------------------------------------------------- NR ---- */
@@ -1304,10 +1345,12 @@ struct K3Dec {
      * normalised aggregate's bf16 pieces): the first weights stream in while the norm
      * finishes. The last arrival of an output tile (LU's and the shared down's slices)
      * writes out (src/core/k3_ops.c:647-654). */
-    static __device__ __noinline__ void latent_up(K3ArgPtr ap, int tk_, int lane)
+    static __device__ __noinline__ int latent_up(K3ArgPtr ap, int tk_, int lane, int *count_)
     {
         const K3kDecode a = *k3d_uniform_cptr(ap);
         const int tk = k3d_uniform(tk_);
+        int *count = k3d_uniform_ptr(count_);
+        int next = -1;
         const K3Geo G = k3_geo(a.T, a.d, a.E, a.k, a.I, a.SI, a.L);
         const int rt = tk / G.KSLU, ks = tk - rt * G.KSLU;
         const int c0 = ks * G.nCL / G.KSLU, c1 = (ks + 1) * G.nCL / G.KSLU;
@@ -1328,7 +1371,7 @@ struct K3Dec {
                 A1[i] = k3d_b128(rw, c < c1 ? o1 + c * 1024 : K3_OOB);
             }
             if (first) {
-                if (!k3d_wait_event(a.sync, G.eN, tk, a.spin_limit, a.err, lane)) return;
+                if (!k3d_wait_event(a.sync, G.eN, tk, a.spin_limit, a.err, lane)) return next;
                 k3d_trace_go(a.trace, G.oLU + tk, lane);
                 first = false;
             }
@@ -1351,8 +1394,9 @@ struct K3Dec {
             k3d_st4_sc1(rp, ((ks * a.T + t) * a.d + row) * 4, y0);
             k3d_st4_sc1(rp, ((ks * a.T + t) * a.d + row + 16) * 4, y1);
         }
-        if (k3d_arrive(k3d_line(a.sync, G.lLU + rt), G.KSLU + G.KSD - 1, lane))
+        if (k3d_arrive_next(k3d_line(a.sync, G.lLU + rt), G.KSLU + G.KSD - 1, lane, count, next))
             combine_out(a, G, rt, lane);
+        return next;
     }
 
     /* The latent layer's aggregate for latent rows 32 dt .. + 31, once every slot's
@@ -1535,24 +1579,36 @@ k_decode_fused(K3kDecode a)
                            G.nX + G.nR <= W;
     if (threadIdx.x == 0) rl.count = 0;
     __syncthreads();
-    for (int tk = w; tk < G.total; tk += W) {
+    /* (the router's and the selection's use of the workgroup's LDS needs their tickets in the
+     * first round) */
+    const int stripe = w % K3_STRIPES;
+    int *count = a.T > 1 && W % K3_STRIPES == 0 && G.nX + G.nR + G.nS <= W
+                     ? k3d_line(a.sync, G.lTK + stripe) : nullptr;
+    for (int tk = w; tk < G.total;) {
         if (a.trace && lane == 0) {
             const unsigned long long now = wall_clock64();
             a.trace[3 * tk] = now;
             a.trace[3 * tk + 1] = now;
         }
-        int t = tk;
+        int t = tk, next = -1;
         if (t < G.nX) K3Dec<NT>::prep(ap, t, lane);
         else if ((t -= G.nX) < G.nR) K3Dec<NT>::router(ap, t, lane, &rl, wg_slices);
-        else if ((t -= G.nR) < 1) K3Dec<NT>::select(ap, lane, &lds);
-        else if ((t -= 1) < G.nLD) K3Dec<NT>::latent_down(ap, t, lane);
-        else if ((t -= G.nLD) < G.nSG) K3Dec<NT>::shared_gateup(ap, t, lane);
-        else if ((t -= G.nSG) < G.nSD) K3Dec<NT>::shared_down(ap, t, lane);
-        else if ((t -= G.nSD) < G.nG) K3Dec<NT>::routed_gateup(ap, t, lane);
-        else if ((t -= G.nG) < G.nD) K3Dec<NT>::routed_down(ap, t, lane);
+        else if ((t -= G.nR) < G.nS) K3Dec<NT>::select(ap, t, lane, &lds);
+        else if ((t -= G.nS) < G.nLD) next = K3Dec<NT>::latent_down(ap, t, lane, count);
+        else if ((t -= G.nLD) < G.nSG) next = K3Dec<NT>::shared_gateup(ap, t, lane, count);
+        else if ((t -= G.nSG) < G.nSD) next = K3Dec<NT>::shared_down(ap, t, lane, count);
+        else if ((t -= G.nSD) < G.nG) next = K3Dec<NT>::routed_gateup(ap, t, lane, count);
+        else if ((t -= G.nG) < G.nD) next = K3Dec<NT>::routed_down(ap, t, lane, count);
         else if ((t -= G.nD) < G.nNR) K3Dec<NT>::norm(ap, t, lane);
-        else K3Dec<NT>::latent_up(ap, t - G.nNR, lane);
+        else next = K3Dec<NT>::latent_up(ap, t - G.nNR, lane, count);
         if (a.trace && lane == 0) a.trace[3 * tk + 2] = wall_clock64();
+        if (!count) {
+            tk += W;
+            continue;
+        }
+        if (lane == 0 && next < 0)
+            next = __hip_atomic_fetch_add(count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        tk = W + K3_STRIPES * k3d_uniform(next) + stripe;
     }
 }
 
