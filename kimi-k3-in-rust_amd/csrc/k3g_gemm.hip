@@ -405,10 +405,22 @@ __device__ __forceinline__ bool gm_setup(const K3kGemm &g, GmTile &t, uint8_t *l
     const int ntl = (g.tiles ? *g.ntiles : (g.dense_rows + GM_COLS - 1) / GM_COLS) * ks_n *
                     (halves ? 2 : 1);
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-    const int rnd = slot / g.nft, f = slot - rnd * g.nft;
-    const int grp = rnd / K3G_TILE_GROUP, gi = rnd - grp * K3G_TILE_GROUP;
-    int tks = K3G_TILE_GROUP * (8 * grp + ((grp & 1) ? 7 - xcd : xcd)) + gi;
-    if (tks >= ntl) return false;
+    int f, tks;
+    if (AF == 0) {
+        const int rnd = slot / g.nft;
+        f = slot - rnd * g.nft;
+        tks = gm_tile_of(rnd, xcd);
+        if (tks >= ntl) return false;
+    } else {
+        /* dense: equal items, an eighth of them to each XCD, feature tile by feature tile, so
+         * that an XCD streams its own eighth of the weights. Dealt like the routed tiles, 16
+         * column tiles were the work of four XCDs: 2,000 tokens on 2 x 6144 rows of 7168 1449 ->
+         * 781 us, back 566 -> 354; column tile by column tile 819 and 385. */
+        const int N = ntl * g.nft, per = (N + 7) >> 3, lam = xcd * per + slot;
+        if (slot >= per || lam >= N) return false;
+        f = lam / ntl;
+        tks = lam - f * ntl;
+    }
     const int hf = halves ? (tks & 1) : 0;
     if (halves) tks >>= 1;
     const int tile = tks / ks_n;
@@ -954,7 +966,7 @@ extern "C" int k3k_gemm(const K3kGemm *g, hipStream_t st)
                      ks_n > g->K / GM_KC || (g->mode == 0 && g->rows % 4)))
         return -1;
     const long long maxt = (long long)((g->dense_rows + GM_COLS - 1) / GM_COLS) * ks_n;
-    const long long grid = 8 * (long long)K3G_TILE_ROUNDS(maxt) * g->nft;
+    const long long grid = 8 * ((maxt * g->nft + 7) / 8);
     if (grid > 0x7fffffff) return -1;
     K3kGemm g1 = *g;
     g1.ksplit = ks_n;
