@@ -550,7 +550,7 @@ k_gemm(const K3kGemm g)
 /* The routed experts' gate/up (mode 0) or down (mode 1): FP6 pieces on the FP4 x FP6 matrix cores;
  * but gate/up of an x that is all bf16 values (its flag is clear) on the bf16 ones, where that
  * x is one piece. Both take workgroups of 4 waves for 128 features (256 rows) and write h alike.
- * In full tiles (32,768 pairs) gate/up takes 1.46 ms on one bf16 piece, 1.78 on four FP6
+ * In full tiles (32,768 pairs) gate/up takes 1.46 ms on one bf16 piece, 1.73 on four FP6
  * pieces and took 2.58 on two bf16 pieces. */
 template <int MODE>
 __global__ void __launch_bounds__(256, 2)

@@ -25,7 +25,7 @@
  * Work unit: one workgroup of 4 waves = (up to 64 pairs of a column tile, 512 or 256 weight
  * rows: half gate and the same up rows, or output rows). Wave w owns 16 RG rows (RG = 8 or 4)
  * and all NB column blocks of 16. Its weights go from HBM to registers, two steps ahead;
- * the activations are copied to LDS one step ahead by global_load_lds_dwordx4, eight columns
+ * the activations are copied to LDS ahead by global_load_lds_dwordx4, eight columns
  * x one whole line per instruction (instructions that took 64 bytes of 16 columns met the
  * other half of each line still on its way: the cache stalls on that, and 49-75 % of its
  * cycles went there), the 16-byte units of column c swizzled by c % 8 so that the B-operand
@@ -34,9 +34,9 @@
  *
  * What bounds it: with 1 and 2 column blocks the weight stream (gate/up of 256 tokens of the K2
  * layer, 6.0 GB, 0.93 ms, 6.4 TB/s); with full tiles the matrix cores, which hold 1.7 GHz on FP6
- * data (gate/up of 32,768 pairs in full tiles 1.78 ms, 1.08 PFLOP/s; on two bf16 pieces it
+ * data (gate/up of 32,768 pairs in full tiles 1.73 ms, 1.11 PFLOP/s; on two bf16 pieces it
  * took 2.58; down 0.99, as bf16 + MXFP8 remainder 1.27-1.30). K3, 2,000 tokens (896 experts of
- * about 36 pairs): gate/up 4.33 -> 3.26 ms beside the shared expert; K2, 4,096 bf16 tokens: down
+ * about 36 pairs): gate/up 4.33 -> 3.01 ms beside the shared expert; K2, 4,096 bf16 tokens: down
  * 1.68 -> 1.40.
  *
  * Workgroup order: k3g_gemm.hip's (tiles largest first, dealt to the XCDs in groups). */
@@ -47,7 +47,7 @@
 #define G6_ROWS 256                 /* weight rows per workgroup (twice that with RG = 8) */
 #define G6_QB K3G_P6_QUAD           /* bytes of one activation quad */
 #define G6_BLK (6 * 1024)           /* a step of one column block in LDS */
-#define G6_LDS (72 * 1024)          /* 2 stages of 4 blocks, 2 quads of their scales; the epilogue
+#define G6_LDS (72 * 1024)          /* 2 stages of 4 blocks or 3 of 3, 2 quads of their scales; the epilogue
                                      * takes all of it */
 #ifndef G6_BIG_MIN
 #define G6_BIG_MIN 1024
@@ -121,15 +121,21 @@ __device__ __forceinline__ const uint8_t *g6_block(const K3kGemm6 &g, const G6Ti
 
 /* One tile's products. The copies of a step: wave w takes column block w (NB = 3, 4), half a block
  * (NB = 2), or half of one's lines (NB = 1); lane 8 c + s of an instruction brings unit s ^ c
- * of its column's line to LDS unit 8 c + s. Step c waits for its copies (issued one step
- * before) and weights: with DEPTH 2 all but the loads of step c + 1's weights. */
+ * of its column's line to LDS unit 8 c + s. Weights are loaded DEPTH steps ahead. With 2 and 3
+ * blocks the copies are issued two steps ahead as well (three stages): one step ahead, every
+ * step lasted a trip to memory and then the matrix work (K3, 36 pairs an expert: 1.94 ms of
+ * weights + 0.84 of matrix work took 2.80 ms; 2.56 so, and down 1.46 -> 1.36). With one block,
+ * short steps, that is 2 % slower. Step c waits for all but the loads of step c + 1's weights;
+ * of the three-stage order the wait takes in as many of those loads as there are copies behind
+ * them, so the scales, three times of four already in the cache, are loaded first. */
 template <int MODE, int NB, int RG>
 __device__ __forceinline__ void g6_run(const K3kGemm6 &g, const G6Tile &t)
 {
     /* 128 accumulators leave room for the weights of one step ahead only */
     constexpr int DEPTH = RG * NB > 24 ? 1 : 2, NBUF = DEPTH + 1;
-    constexpr int STAGE = NB * G6_BLK, SCL0 = 2 * STAGE, SCL = NB * 1024;
-    static_assert(2 * (STAGE + SCL) <= G6_LDS, "LDS");
+    constexpr int NST = DEPTH == 2 && NB > 1 && NB <= 3 ? 3 : 2;
+    constexpr int STAGE = NB * G6_BLK, SCL0 = NST * STAGE, SCL = NB * 1024;
+    static_assert(SCL0 + 2 * SCL <= G6_LDS, "LDS");
     const int lane = t.lane, c16 = lane & 15, q4 = lane >> 4;
     k3v4f acc[RG][NB];
 #pragma unroll
@@ -154,10 +160,10 @@ __device__ __forceinline__ void g6_run(const K3kGemm6 &g, const G6Tile &t)
     for (int h = 0; h < NH; ++h)
         src[h] = rowof(8 * (h0 + h) + (lane >> 3)) + 16 * ((lane & 7) ^ (lane >> 3));
     ssrc = rowof(lane >> 2) + 1536 + 16 * (lane & 3);
-    auto copy = [&](int c) {
+    auto copy = [&](int c, int stage) {
         if (NB == 3 && t.w == 3) return;
         const size_t o = (size_t)(c >> 2) * G6_QB;
-        const uint32_t l = t.lds + (c & 1) * STAGE + blk * G6_BLK;
+        const uint32_t l = t.lds + stage * STAGE + blk * G6_BLK;
 #pragma unroll
         for (int h = 0; h < NH; ++h)
 #pragma unroll
@@ -180,11 +186,11 @@ __device__ __forceinline__ void g6_run(const K3kGemm6 &g, const G6Tile &t)
     auto wload = [&](int c, uint4 (&d)[RG], uint32_t (&s)[RG]) {
         const size_t qo = (size_t)(c >> 2) * G6_QT;
 #pragma unroll
-        for (int r = 0; r < RG; ++r) {
-            const uint8_t *p = rbase[r] + qo;
-            d[r] = gm_ld16(p + 1024 * (c & 3) + 16 * lane);
-            s[r] = gm_ld4(p + 4096 + 4 * lane);
-        }
+        for (int r = 0; r < RG; ++r) s[r] = gm_ld4(rbase[r] + qo + 4096 + 4 * lane);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int r = 0; r < RG; ++r) d[r] = gm_ld16(rbase[r] + qo + 1024 * (c & 3) + 16 * lane);
+        __builtin_amdgcn_sched_barrier(0);
     };
     /* piece p of column c16's block q4: 16 bytes at bx (bx ^ 64 for odd p) in lines p / 2, 8
      * bytes at by ^ 32 p in line 2; its scales at bz */
@@ -192,15 +198,16 @@ __device__ __forceinline__ void g6_run(const K3kGemm6 &g, const G6Tile &t)
     const uint32_t by = 4096 + (c16 >> 3) * 1024 + (c16 & 7) * 128 +
                         16 * ((q4 >> 1) ^ (c16 & 7)) + 8 * (q4 & 1);
     const uint32_t bz = SCL0 + 64 * c16 + 4 * q4;
-    auto step = [&](int c, const uint4 (&w)[RG], const uint32_t (&sc)[RG], uint4 (&nw)[RG],
+    auto step = [&](int c, int stage, const uint4 (&w)[RG], const uint32_t (&sc)[RG], uint4 (&nw)[RG],
                     uint32_t (&ns)[RG]) {
         gm_wait_vm<(DEPTH == 2 ? 2 * RG : 0)>();
         __syncthreads();
-        if (c + 1 < t.nK) copy(c + 1);
+        if (NST == 2 && c + 1 < t.nK) copy(c + 1, 1 - stage);
         wload(min(c + DEPTH, t.nK - 1), nw, ns);
+        if (NST == 3 && c + 2 < t.nK) copy(c + 2, (stage + 2) % 3);
         __builtin_amdgcn_sched_barrier(0);
         if (c >= t.nK) return;
-        const uint8_t *st = t.ldsp + (c & 1) * STAGE;
+        const uint8_t *st = t.ldsp + stage * STAGE;
         const uint8_t *sl = t.ldsp + ((c >> 2) & 1) * SCL + 16 * (c & 3) + bz;
         const int sh = 8 * (c & 3);
         uint32_t sa[RG];
@@ -236,13 +243,16 @@ __device__ __forceinline__ void g6_run(const K3kGemm6 &g, const G6Tile &t)
             for (int r = 0; r < RG; ++r) g6_pin(acc[r][n]);
         }
     };
-    copy(0);
+    if (NST == 2) copy(0, 0);
 #pragma unroll
-    for (int s = 0; s < DEPTH; ++s) wload(min(s, t.nK - 1), wb[s], ws[s]);
+    for (int s = 0; s < DEPTH; ++s) {
+        wload(min(s, t.nK - 1), wb[s], ws[s]);
+        if (NST == 3 && s < t.nK) copy(s, s);
+    }
     for (int c = 0; c < t.nK; c += NBUF) {
 #pragma unroll
         for (int u = 0; u < NBUF; ++u)
-            step(c + u, wb[u], ws[u], wb[(u + DEPTH) % NBUF], ws[(u + DEPTH) % NBUF]);
+            step(c + u, NST == 3 ? u : (c + u) & 1, wb[u], ws[u], wb[(u + DEPTH) % NBUF], ws[(u + DEPTH) % NBUF]);
     }
     gm_wait_vm<0>();
 
