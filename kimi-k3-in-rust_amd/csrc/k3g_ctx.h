@@ -84,7 +84,7 @@ struct K3gCtx {
     hipEvent_t ev_in, ev_shared;
     int gemm_fp8;                /* routed experts on the FP4 x FP8 matrix cores */
     uint8_t *xr, *hr;            /* the routed experts' input per token and h per pair as FP6
-                                  * pieces, rows of quads (k3g_gemm6.hip) */
+                                  * pieces, rows of quads (k3g_gemm6.h) */
     uint8_t *xq8b, *hq8b;        /* MXFP8 x [T][d512] + scales, h [T*k][I512] + scales */
     unsigned long long *trace;   /* optional per-ticket timestamps of the fused kernel */
     /* optional pinned host copies that the fused kernel writes directly (the routing, a

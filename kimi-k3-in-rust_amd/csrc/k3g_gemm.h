@@ -1,4 +1,4 @@
-/* k3g_gemm.h - device helpers of the grouped GEMMs (k3g_gemm.hip, k3g_gemm6.hip). */
+/* k3g_gemm.h - device helpers of the grouped GEMMs (k3g_gemm.hip, k3g_gemm6.h). */
 #pragma once
 
 #include "k3g_dev.h"

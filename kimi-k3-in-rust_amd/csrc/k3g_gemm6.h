@@ -49,9 +49,7 @@
 #define G6_BLK (6 * 1024)           /* a step of one column block in LDS */
 #define G6_LDS (72 * 1024)          /* 2 stages of 4 blocks or 3 of 3, 2 quads of their scales; the epilogue
                                      * takes all of it */
-#ifndef G6_BIG_MIN
-#define G6_BIG_MIN 1024
-#endif
+#define G6_BIG_MIN 1024             /* workgroups from which on RG = 8 (g6_setup) */
 #define G6_QT 4352                  /* tiled MXFP4 quad tile */
 
 /* x (fp32 [T][K]) -> activation quads, one thread per block of 32; the blocks of the last

@@ -103,9 +103,7 @@ typedef double k3v4d __attribute__((ext_vector_type(4)));
 
 #define K3R_RING 4
 /* one wave per tile (tiles enough to fill the GPU) from this many tokens on */
-#ifndef K3R_MFMA_MIN_T
 #define K3R_MFMA_MIN_T 512
-#endif
 
 #define K3R_PART 11    /* doubles per lane of a slice's partial sums */
 #define K3R_WPB 4      /* waves per workgroup when K is sliced */
