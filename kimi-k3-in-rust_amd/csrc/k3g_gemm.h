@@ -102,6 +102,17 @@ __device__ __forceinline__ int gm_tile_of(int rnd, int xcd)
     return K3G_TILE_GROUP * (8 * grp + ((grp & 1) ? 7 - xcd : xcd)) + gi;
 }
 
+/* The item of a round of n: as gm_tile_of; but where every expert is one item (single: no two
+ * share weights) and the groups of four would leave the fullest XCD a sixth above the mean, one by
+ * one. 40 items (5 tokens of the K2 layer) in groups are 8 for two XCDs and 4 for the others. Whole
+ * calls, us: K2 at 5 / 6 / 10 / 16 tokens 287 / 307 / 427 / 561 -> 269 / 294 / 403 / 545, K3 at 5 /
+ * 9 tokens 437 / 594 -> 417 / 580. */
+__device__ __forceinline__ int gm_item_of(int rnd, int xcd, int n, bool single)
+{
+    if (!single || 7 * n > 6 * 8 * K3G_TILE_ROUNDS(n)) return gm_tile_of(rnd, xcd);
+    return 8 * rnd + ((rnd & 1) ? 7 - xcd : xcd);
+}
+
 /* a compile-time integer as an argument */
 template <int N> struct GmInt { static constexpr int value = N; };
 
@@ -109,11 +120,11 @@ template <int N> struct GmInt { static constexpr int value = N; };
  * feature tile in a launch of one item per column tile (the second half of a tile that is two
  * items has none) and one record for every step-th of the nft feature tiles. */
 __device__ __forceinline__ void gm_trace(unsigned long long *trace, int nft, int step, int halves,
-                                         unsigned long long t_start)
+                                         int n, bool single, unsigned long long t_start)
 {
     const int slot = blockIdx.x >> 3;
     const int rnd = slot / nft, ft = slot - rnd * nft, nf = (nft + step - 1) / step;
-    const int item = gm_tile_of(rnd, blockIdx.x & 7), tile = item >> halves;
+    const int item = gm_item_of(rnd, blockIdx.x & 7, n, single), tile = item >> halves;
     if (ft % step || (item & halves)) return;
     const int grp = tile / K3G_TILE_GROUP, q = grp >> 3;
     const int xcd = (q & 1) ? 7 - (grp & 7) : grp & 7;

@@ -409,7 +409,7 @@ __device__ __forceinline__ bool gm_setup(const K3kGemm &g, GmTile &t, uint8_t *l
     if (AF == 0) {
         const int rnd = slot / g.nft;
         f = slot - rnd * g.nft;
-        tks = gm_tile_of(rnd, xcd);
+        tks = gm_item_of(rnd, xcd, ntl, g.single);
         if (tks >= ntl) return false;
     } else {
         /* dense: equal items, an eighth of them to each XCD, feature tile by feature tile, so
@@ -575,6 +575,7 @@ k_gemm6(const K3kGemm6 g)
         b.b1 = g.b1;
         b.b2 = g.b2;
         b.nft = g.nft;
+        b.single = !g.halves;
         if (!gm_block<0, 4>(b, lds, 1)) return;
     } else {
         G6Tile t;
@@ -589,7 +590,8 @@ k_gemm6(const K3kGemm6 g)
         }
     }
     if (g.trace && threadIdx.x == 0) gm_trace(g.trace, g.nft, g.trace_step,
-                                                  bf16 ? 0 : g.halves, t_start);
+                                                  bf16 ? 0 : g.halves, *g.ntiles, !g.halves,
+                                                  t_start);
 }
 
 /* ============================================================ FP4 x FP8 variant ==== */

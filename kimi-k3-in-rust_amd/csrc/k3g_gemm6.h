@@ -285,7 +285,7 @@ __device__ __forceinline__ int g6_setup(const K3kGemm6 &g, G6Tile &t, uint8_t *l
     const int ntl = *g.ntiles;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int rnd = slot / g.nft, ft = slot - rnd * g.nft;
-    const int item = gm_tile_of(rnd, xcd);
+    const int item = gm_item_of(rnd, xcd, ntl, !g.halves);
     if (item >= (ntl << g.halves)) return 0;
     const int4 tv = ((const int4 *)g.tiles)[item >> g.halves];
     const int e = gm_uniform(tv.x), hf = 64 * (item & g.halves);

@@ -140,6 +140,7 @@ typedef struct {
     float *out;               /* mode 1 out: row per column, stride ldo */
     int ldo;
     int scatter;              /* mode 1: out row = perm[column] (else the column) */
+    int single;               /* no expert has two column tiles or halves (gm_item_of) */
     int nft;                  /* feature tiles: ceil(rows / 256) (mode 0), / 512 (mode 1) */
     /* MXFP8 activations (k3k_gemm_f8, MXFP4 weights only): E4M3 bytes [rows][ldb] and
      * E8M0 block scales [rows][ldb / 32]; mode 0 writes h the same way to hq/hs */
