@@ -137,7 +137,7 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     /* the grouped GEMMs' activation pieces and column tiles */
     const size_t d128 = (d + 127) / 128 * 128;
     const size_t SI128 = (SI + 127) / 128 * 128;
-    const size_t maxt = (P + 127) / 128 + E;
+    const size_t maxt = (P + 63) / 64 + E;
     const size_t o_xb = carve(&at, 2 * T * d128 * 2);
     const size_t o_hsb = carve(&at, 2 * T * (SI128 ? SI128 : 128) * 2);
     /* the dense GEMMs' K-slice sums when few columns leave the GPU idle: the shared
@@ -435,6 +435,15 @@ static int gemm_body(K3gCtx *c, const K3gLayer *L, const float *x, int T,
                      const int32_t *idx, const float *wt, float *out, float *contrib, int fp8,
                      int full, int routed, hipStream_t st);
 
+/* Pairs per column tile of T tokens with topk slots each. A tile of up to 64 pairs is one work
+ * item. Routed by k3g_moe's own router an expert has at most T pairs, but for the tokens with
+ * fewer than topk selectable experts (NaN scores, a bias of -inf): they have expert 0 in every
+ * slot left over, as in the engine. So up to 64 tokens the tiles themselves end at 64 pairs. */
+static int tile_cols(int T, int topk, int routed)
+{
+    return (routed ? T : T * topk) <= 64 ? 64 : 128;
+}
+
 static int experts_gemm(K3gCtx *c, const K3gLayer *L, const float *x, int T,
                         const int32_t *idx, const float *wt, float *out, float *contrib,
                         int fp8, int full, hipStream_t st)
@@ -442,7 +451,8 @@ static int experts_gemm(K3gCtx *c, const K3gLayer *L, const float *x, int T,
     int rc = 0;
     k3g_stage_begin(c, K3G_ST_DISPATCH, st);
     rc |= k3k_dispatch_tiles(idx, T * L->topk, L->n_experts, c->cnt, c->base, c->off, c->act,
-                             c->nact, c->perm, c->err, c->tiles, c->ntiles, c->xflag, st);
+                             c->nact, c->perm, c->err, tile_cols(T, L->topk, 0), c->tiles,
+                             c->ntiles, c->xflag, st);
     k3g_stage_end(c, K3G_ST_DISPATCH, st);
     return rc | gemm_body(c, L, x, T, idx, wt, out, contrib, fp8, full, 0, st);
 }
@@ -521,12 +531,14 @@ static int gemm_pieces(K3gCtx *c, const K3gLayer *L, const float *x, int T, int 
     return rc;
 }
 
-/* The routed experts on the column tiles, x or z -> h -> contrib rows (k3g_gemm6.h). max_np:
- * no expert has more pairs than this */
-static int routed_f6(K3gCtx *c, const K3gLayer *L, int lat, int max_tiles, int max_np,
+/* The routed experts on the column tiles of up to cols pairs, x or z -> h -> contrib rows
+ * (k3g_gemm6.h) */
+static int routed_f6(K3gCtx *c, const K3gLayer *L, int T, int lat, int cols, int max_tiles,
                      float *contrib, hipStream_t st)
 {
-    const int I = L->inter;
+    const int I = L->inter, P = T * L->topk;
+    /* the trace's places: as many tiles as the header says */
+    const int trace_tiles = (P + 127) / 128 + (L->n_experts < P ? L->n_experts : P);
     int rc = 0;
     K3kGemm6 g;
     memset(&g, 0, sizeof g);
@@ -545,18 +557,19 @@ static int routed_f6(K3gCtx *c, const K3gLayer *L, int lat, int max_tiles, int m
     g.tiles = c->tiles;
     g.ntiles = c->ntiles;
     g.max_tiles = max_tiles;
-    g.halves = max_np > 64;
+    g.halves = cols > 64;
     g.h = c->hr;
     g.b1 = L->act_b1;
     g.b2 = L->act_b2;
     g.trace = c->trace;
     g.trace_step = 1;
+    g.trace_tiles = trace_tiles;
     k3g_stage_begin(c, K3G_ST_GATEUP, st);
     rc |= k3k_gemm6(&g, st);
     k3g_stage_end(c, K3G_ST_GATEUP, st);
     /* the down launch's stamps follow the gate/up launch's */
     if (g.trace)
-        g.trace += 4 * 8 * (size_t)K3G_TILE_ROUNDS(max_tiles) * (size_t)((I + 127) / 128);
+        g.trace += 4 * 8 * (size_t)K3G_TILE_ROUNDS(trace_tiles) * (size_t)((I + 127) / 128);
     g.mode = 1;
     g.rows = lat;
     g.K = I;
@@ -621,9 +634,9 @@ static int routed_f8(K3gCtx *c, const K3gLayer *L, int T, int lat, int max_tiles
 
 /* The grouped GEMMs after the dispatch (column tiles built, x's piece-1 flag cleared):
  * x pieces, [latent down], the shared expert, the routed gate/up and down, [combine,
- * latent up, + shared]. routed: called by k3g_moe after its own router (no token has an expert
- * twice, so no expert has more than T pairs); x's pieces are already made and the shared expert
- * runs on the side stream (ev_shared marks its end; the combine waits for it). */
+ * latent up, + shared]. routed: called by k3g_moe after its own router; x's pieces are already
+ * made and the shared expert runs on the side stream (ev_shared marks its end; the combine waits
+ * for it). */
 static int gemm_body(K3gCtx *c, const K3gLayer *L, const float *x, int T,
                      const int32_t *idx, const float *wt, float *out, float *contrib, int fp8,
                      int full, int routed, hipStream_t st)
@@ -641,7 +654,8 @@ static int gemm_body(K3gCtx *c, const K3gLayer *L, const float *x, int T,
         rc |= routed_input(c, c->z, T, lat, fp8, NULL, st);
         k3g_stage_end(c, K3G_ST_LATENT, st);
     }
-    const int max_tiles = (P + 127) / 128 + (E < P ? E : P);
+    const int cols = tile_cols(T, k, routed);
+    const int max_tiles = (P + cols - 1) / cols + (E < P ? E : P);
     if (SI > 0 && !routed) rc |= shared_expert(c, L, T, c->kpart, st);
     /* routed experts last, after any copies they wait for (the shared expert above
      * overlaps them) */
@@ -650,7 +664,7 @@ static int gemm_body(K3gCtx *c, const K3gLayer *L, const float *x, int T,
         c->routed_wait = NULL;
     }
     rc |= fp8 ? routed_f8(c, L, T, lat, max_tiles, contrib, st)
-              : routed_f6(c, L, lat, max_tiles, routed ? T : P, contrib, st);
+              : routed_f6(c, L, T, lat, cols, max_tiles, contrib, st);
 
     if (SI > 0 && routed && hipStreamWaitEvent(st, c->ev_shared, 0) != hipSuccess) rc = -1;
     if (full && !projected && !L->up && !L->latent_norm) {
@@ -1034,8 +1048,8 @@ int k3g_moe(K3gCtx *c, const K3gLayer *L, const float *x, int T, float *out, int
         /* the dispatch's flag argument (cleared) is the spare one: x's is set above */
         k3g_stage_begin(c, K3G_ST_DISPATCH, st);
         rc |= k3k_dispatch_tiles(idx, T * L->topk, L->n_experts, c->cnt, c->base, c->off,
-                                 c->act, c->nact, c->perm, c->err, c->tiles, c->ntiles,
-                                 c->zflag, st);
+                                 c->act, c->nact, c->perm, c->err, tile_cols(T, L->topk, 1),
+                                 c->tiles, c->ntiles, c->zflag, st);
         k3g_stage_end(c, K3G_ST_DISPATCH, st);
         rc |= gemm_body(c, L, x, T, idx, wt, out, c->contrib, c->gemm_fp8, 1, 1, st);
         return rc ? -1 : 0;

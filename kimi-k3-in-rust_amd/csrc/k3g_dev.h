@@ -135,16 +135,17 @@ __device__ __forceinline__ void k3d_block_exscan_n(int (&v)[N], int (&tot)[N], i
     __syncthreads();
 }
 
-/* Column tiles of up to K3G_TILE_COLS pairs per expert, largest first: every full tile
- * (in expert order), then the experts' last partial tiles by their count of 16-column
+/* Column tiles of up to `cols` pairs per expert (64 or K3G_TILE_COLS), largest first: every full
+ * tile (in expert order), then the experts' last partial tiles by their count of 16-column
  * blocks, 8 down to 1 (in expert order within a count); clears *flag. Called by every
  * thread of a block of 1024 (thread e < E for expert e, its pair count and first sorted
  * position); lds holds (16 + 1) * 9 ints. */
-__device__ __forceinline__ void k3d_build_tiles(int e, int E, int cnt, int off_e, int4 *tiles,
-                                                int32_t *ntiles, int32_t *flag, int *lds)
+__device__ __forceinline__ void k3d_build_tiles(int e, int E, int cnt, int off_e, int cols,
+                                                int4 *tiles, int32_t *ntiles, int32_t *flag,
+                                                int *lds)
 {
     if (e >= E) cnt = 0;
-    const int nfull = cnt / K3G_TILE_COLS, rem = cnt - nfull * K3G_TILE_COLS;
+    const int nfull = cnt / cols, rem = cnt - nfull * cols;
     const int cls = rem ? (rem + 15) / 16 : 0;          /* block count of the last tile */
     int v[9], tot[9];
     v[0] = nfull;
@@ -152,12 +153,12 @@ __device__ __forceinline__ void k3d_build_tiles(int e, int E, int cnt, int off_e
     for (int j = 1; j < 9; ++j) v[j] = cls == 9 - j;
     k3d_block_exscan_n<9, 16>(v, tot, lds);
     for (int i = 0; i < nfull; ++i)
-        tiles[v[0] + i] = make_int4(e, off_e + K3G_TILE_COLS * i, K3G_TILE_COLS, 0);
+        tiles[v[0] + i] = make_int4(e, off_e + cols * i, cols, 0);
     int base = tot[0];
 #pragma unroll
     for (int j = 1; j < 9; ++j) {
         if (cls == 9 - j)
-            tiles[base + v[j]] = make_int4(e, off_e + K3G_TILE_COLS * nfull, rem, 0);
+            tiles[base + v[j]] = make_int4(e, off_e + cols * nfull, rem, 0);
         base += tot[j];
     }
     if (e == 0) { *ntiles = base; *flag = 0; }

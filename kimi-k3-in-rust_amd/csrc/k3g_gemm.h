@@ -102,8 +102,8 @@ __device__ __forceinline__ int gm_tile_of(int rnd, int xcd)
     return K3G_TILE_GROUP * (8 * grp + ((grp & 1) ? 7 - xcd : xcd)) + gi;
 }
 
-/* The item of a round of n: as gm_tile_of; but where every expert is one item (single: no two
- * share weights) and the groups of four would leave the fullest XCD a sixth above the mean, one by
+/* The item of a round of n: as gm_tile_of; but where an expert is one item (single: as a
+ * rule no two share weights) and the groups of four would leave the fullest XCD a sixth above the mean, one by
  * one. 40 items (5 tokens of the K2 layer) in groups are 8 for two XCDs and 4 for the others. Whole
  * calls, us: K2 at 5 / 6 / 10 / 16 tokens 287 / 307 / 427 / 561 -> 269 / 294 / 403 / 545, K3 at 5 /
  * 9 tokens 437 / 594 -> 417 / 580. */
@@ -118,14 +118,15 @@ template <int N> struct GmInt { static constexpr int value = N; };
 
 /* Instrumentation: one record of a workgroup's start and end, at the place of its column tile and
  * feature tile in a launch of one item per column tile (the second half of a tile that is two
- * items has none) and one record for every step-th of the nft feature tiles. */
+ * items has none, nor do tiles from `limit` on) and one record for every step-th of the nft feature
+ * tiles. */
 __device__ __forceinline__ void gm_trace(unsigned long long *trace, int nft, int step, int halves,
-                                         int n, bool single, unsigned long long t_start)
+                                         int n, bool single, int limit, unsigned long long t_start)
 {
     const int slot = blockIdx.x >> 3;
     const int rnd = slot / nft, ft = slot - rnd * nft, nf = (nft + step - 1) / step;
     const int item = gm_item_of(rnd, blockIdx.x & 7, n, single), tile = item >> halves;
-    if (ft % step || (item & halves)) return;
+    if (ft % step || (item & halves) || tile >= limit) return;
     const int grp = tile / K3G_TILE_GROUP, q = grp >> 3;
     const int xcd = (q & 1) ? 7 - (grp & 7) : grp & 7;
     const size_t r = (size_t)(K3G_TILE_GROUP * q + tile % K3G_TILE_GROUP) * nf + ft / step;

@@ -591,7 +591,7 @@ k_gemm6(const K3kGemm6 g)
     }
     if (g.trace && threadIdx.x == 0) gm_trace(g.trace, g.nft, g.trace_step,
                                                   bf16 ? 0 : g.halves, *g.ntiles, !g.halves,
-                                                  t_start);
+                                                  g.trace_tiles, t_start);
 }
 
 /* ============================================================ FP4 x FP8 variant ==== */
@@ -765,13 +765,13 @@ k_gemm_f8(const K3kGemm g)
  * (n_experts <= 1024). */
 static_assert(GM_COLS == K3G_TILE_COLS, "column tile width");
 __global__ void __launch_bounds__(1024)
-k_gemm_tiles(const int32_t *__restrict__ off, int E, int4 *__restrict__ tiles,
+k_gemm_tiles(const int32_t *__restrict__ off, int E, int cols, int4 *__restrict__ tiles,
              int32_t *__restrict__ ntiles, int32_t *__restrict__ flag)
 {
     __shared__ int red[17 * 9];
     const int e = threadIdx.x;
     const int cnt = e < E ? off[e + 1] - off[e] : 0;
-    k3d_build_tiles(e, E, cnt, e < E ? off[e] : 0, tiles, ntiles, flag, red);
+    k3d_build_tiles(e, E, cnt, e < E ? off[e] : 0, cols, tiles, ntiles, flag, red);
 }
 
 /* x (fp32 [T][d]) -> two bf16 pieces [2][T][ldb]; raises *flag when any piece 1 is not
@@ -867,11 +867,11 @@ extern "C" size_t k3k_gemm_part_bytes(int nft, int rows2)
 }
 
 /* ------------------------------------------------------------------ launchers ---- */
-extern "C" int k3k_gemm_tiles(const int32_t *off, int E, int32_t *tiles, int32_t *ntiles,
-                              int32_t *flag, hipStream_t st)
+extern "C" int k3k_gemm_tiles(const int32_t *off, int E, int cols, int32_t *tiles,
+                              int32_t *ntiles, int32_t *flag, hipStream_t st)
 {
-    if (E < 1 || E > 1024) return -1;
-    hipLaunchKernelGGL(k_gemm_tiles, dim3(1), dim3(1024), 0, st, off, E, (int4 *)tiles, ntiles,
+    if (E < 1 || E > 1024 || (cols != 64 && cols != GM_COLS)) return -1;
+    hipLaunchKernelGGL(k_gemm_tiles, dim3(1), dim3(1024), 0, st, off, E, cols, (int4 *)tiles, ntiles,
                        flag);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }

@@ -140,7 +140,7 @@ typedef struct {
     float *out;               /* mode 1 out: row per column, stride ldo */
     int ldo;
     int scatter;              /* mode 1: out row = perm[column] (else the column) */
-    int single;               /* no expert has two column tiles or halves (gm_item_of) */
+    int single;               /* tiles of up to 64 pairs, as a rule one an expert (gm_item_of) */
     int nft;                  /* feature tiles: ceil(rows / 256) (mode 0), / 512 (mode 1) */
     /* MXFP8 activations (k3k_gemm_f8, MXFP4 weights only): E4M3 bytes [rows][ldb] and
      * E8M0 block scales [rows][ldb / 32]; mode 0 writes h the same way to hq/hs */
@@ -183,12 +183,12 @@ typedef struct {
     const uint16_t *xb;
     int ldb;
     const int32_t *lo_flag;
-    int halves;               /* 1: a tile may hold more than 64 pairs (it is two work items) */
+    int halves;               /* 1: tiles of up to 128 pairs, two work items each; 0: of up to 64 */
     int nft;                  /* set by k3k_gemm6: feature tiles */
     /* instrumentation (NULL: off): per workgroup of every trace_step-th feature tile wave 0's
      * start and end (wall clock), item << 32 | feature tile, XCC << 32 | HW_ID */
     unsigned long long *trace;
-    int trace_step;
+    int trace_step, trace_tiles;  /* tiles the trace has room for */
 } K3kGemm6;
 
 int k3k_gemm6(const K3kGemm6 *g, hipStream_t st);
@@ -205,8 +205,9 @@ int k3k_gemm_f8(const K3kGemm *g, hipStream_t st);
 /* x -> MXFP8 (OCP MX: block scale 2^(floor(log2 amax) - 8), E4M3 nearest-even, clamped
  * to +-448): bytes [T][ldq], scales [T][ldq / 32]; the padding columns stay zero. */
 int k3k_xq8(const float *x, int T, int d, int ldq, uint8_t *xq, uint8_t *xs, hipStream_t st);
-/* column tiles from the dispatch's per-expert ranges; clears *flag */
-int k3k_gemm_tiles(const int32_t *off, int E, int32_t *tiles, int32_t *ntiles,
+/* column tiles of up to cols (64 or 128) pairs from the dispatch's per-expert ranges; clears
+ * *flag */
+int k3k_gemm_tiles(const int32_t *off, int E, int cols, int32_t *tiles, int32_t *ntiles,
                    int32_t *flag, hipStream_t st);
 /* x -> bf16 pieces [2][T][ldb]; *flag = 1 when some piece 1 is not zero */
 int k3k_xpieces(const float *x, int T, int d, int ldb, uint16_t *xb, long long piece,
@@ -313,7 +314,8 @@ int k3k_dispatch(const int32_t *idx, int P, int E, int32_t *cnt, int32_t *base,
  * launch when P <= 4096. */
 int k3k_dispatch_tiles(const int32_t *idx, int P, int E, int32_t *cnt, int32_t *base,
                        int32_t *off, int32_t *act, int32_t *nact, int32_t *perm, int *err,
-                       int32_t *tiles, int32_t *ntiles, int32_t *flag, hipStream_t st);
+                       int cols, int32_t *tiles, int32_t *ntiles, int32_t *flag,
+                       hipStream_t st);
 
 /* h = act(W1 z, W3 z) and contrib = W2 h for every active expert's pairs. maxU bounds
  * the number of active experts (min(E, T*k)); maxtok bounds tokens per expert. */

@@ -36,7 +36,7 @@ __device__ __forceinline__ int k3d_key(const int32_t *idx, int p, int P, int E, 
 #define K3G_DSORT 4096
 __global__ void __launch_bounds__(1024)
 k_disp_sort(const int32_t *idx, int P, int E, int32_t *off, int32_t *act, int32_t *nact,
-            int32_t *perm, int *err, int4 *tiles, int32_t *ntiles, int32_t *flag)
+            int32_t *perm, int *err, int cols, int4 *tiles, int32_t *ntiles, int32_t *flag)
 {
     __shared__ __attribute__((aligned(16))) uint32_t kv[2][K3G_DSORT];
     __shared__ int cnt[K3G_MAX_EXPERTS];
@@ -83,7 +83,7 @@ k_disp_sort(const int32_t *idx, int P, int E, int32_t *off, int32_t *act, int32_
             for (int q = 0; q < w; ++q) at += wc[q][key];
             perm[at] = tid;
         }
-        if (tiles) k3d_build_tiles(tid, E, ce, v[0], tiles, ntiles, flag, red);
+        if (tiles) k3d_build_tiles(tid, E, ce, v[0], cols, tiles, ntiles, flag, red);
         return;
     }
     __syncthreads();
@@ -142,7 +142,7 @@ k_disp_sort(const int32_t *idx, int P, int E, int32_t *off, int32_t *act, int32_
     if (tid == 0) { off[E] = tot[0]; *nact = tot[1]; }
     /* the pairs of real experts come first, in expert order, each expert's in pair order */
     for (int i = tid; i < tot[0]; i += 1024) perm[i] = (int32_t)(kv[cur][i] & 4095u);
-    if (tiles) k3d_build_tiles(tid, E, ce, v[0], tiles, ntiles, flag, red);
+    if (tiles) k3d_build_tiles(tid, E, ce, v[0], cols, tiles, ntiles, flag, red);
 }
 
 /* Large P: three passes over chunks of 256 pairs, no single-block step (a lone large
@@ -248,13 +248,14 @@ k_disp_scatter(const int32_t *idx, int P, int E, const int32_t *base, const int3
 
 extern "C" int k3k_dispatch_tiles(const int32_t *idx, int P, int E, int32_t *cnt,
                                   int32_t *base, int32_t *off, int32_t *act, int32_t *nact,
-                                  int32_t *perm, int *err, int32_t *tiles, int32_t *ntiles,
-                                  int32_t *flag, hipStream_t st)
+                                  int32_t *perm, int *err, int cols, int32_t *tiles,
+                                  int32_t *ntiles, int32_t *flag, hipStream_t st)
 {
     if (E < 1 || E > K3G_MAX_EXPERTS || P < 1) return -1;
+    if (tiles && cols != 64 && cols != K3G_TILE_COLS) return -1;
     if (P <= K3G_DSORT) {
         hipLaunchKernelGGL(k_disp_sort, dim3(1), dim3(1024), 0, st, idx, P, E, off, act, nact,
-                           perm, err, (int4 *)tiles, ntiles, flag);
+                           perm, err, cols, (int4 *)tiles, ntiles, flag);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     const int nch = (P + K3G_DCH - 1) / K3G_DCH;
@@ -266,15 +267,15 @@ extern "C" int k3k_dispatch_tiles(const int32_t *idx, int P, int E, int32_t *cnt
     hipLaunchKernelGGL(k_disp_scatter, dim3(nch), dim3(256), 0, st, idx, P, E, base, tot, off,
                        act, nact, perm);
     if (hipGetLastError() != hipSuccess) return -1;
-    return tiles ? k3k_gemm_tiles(off, E, tiles, ntiles, flag, st) : 0;
+    return tiles ? k3k_gemm_tiles(off, E, cols, tiles, ntiles, flag, st) : 0;
 }
 
 extern "C" int k3k_dispatch(const int32_t *idx, int P, int E, int32_t *cnt, int32_t *base,
                             int32_t *off, int32_t *act, int32_t *nact, int32_t *perm,
                             int *err, hipStream_t st)
 {
-    return k3k_dispatch_tiles(idx, P, E, cnt, base, off, act, nact, perm, err, nullptr,
-                              nullptr, nullptr, st);
+    return k3k_dispatch_tiles(idx, P, E, cnt, base, off, act, nact, perm, err, 0,
+                              nullptr, nullptr, nullptr, st);
 }
 
 /* ---------------------------------------------------------------- combine ---- */
