@@ -404,7 +404,8 @@ int  k3g_ctx_paths(K3gCtx *ctx, int clear);
 /* Routed experts of calls beyond the fused decode kernel on the FP4 x FP8 matrix cores
  * (v_mfma_scale_f32_16x16x128_f8f6f4): MXFP4 weights as stored, x and the activation h
  * quantised to MXFP8 (OCP MX: E4M3, an E8M0 scale per 32 values). Off by default
- * (activations in pieces that hold about 20 bits). The shared expert stays bf16. No
+ * (activations in pieces that hold about 20 bits of a block's largest value, 32 columns, and 40
+ * where the block's other values lie far below it). The shared expert stays bf16. No
  * reference counterpart. */
 void k3g_ctx_set_fp8(K3gCtx *ctx, int on);
 
@@ -459,8 +460,8 @@ int  k3g_expert_gemv(K3gCtx *ctx, const K3gLayer *L, const float *x, int T,
                      const int32_t *idx, float *contrib, void *stream);
 
 /* The same contrib rows as grouped GEMMs over 128-pair column tiles: gate/up with the
- * activation fused, then down (weights exact, x and h as four FP6 pieces each on the scaled
- * FP4 x FP6 matrix cores, or x as it is on the bf16 ones when every value is a bf16 value;
+ * activation fused, then down (weights exact, x and h as four FP6 pieces each, eight in blocks
+ * of 32 whose values lie far below the largest, on the scaled FP4 x FP6 matrix cores, or x as it is on the bf16 ones when every value is a bf16 value;
  * fp32 accumulation; rel-L2 about 1.5e-6) or, for _f8f6f4, the
  * scaled FP4 x FP8 ones with x and h quantised to MXFP8. Experts in the tiled layout
  * (K3G_EXPERT_MXFP4_TILED), hidden and inter multiples of 32. */

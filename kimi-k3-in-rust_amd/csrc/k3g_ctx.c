@@ -164,13 +164,13 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     const size_t o_kpart2 = carve(&at, part2 ? part2 : 16);
     const size_t L128 = (L + 127) / 128 * 128;
     const size_t o_zb = carve(&at, L != d ? 2 * T * L128 * 2 : 16);
-    const size_t o_zflag = carve(&at, 4);
+    const size_t o_zflag = carve(&at, 3 * 4);
     const size_t o_rtpart = carve(&at, k3k_router_part_bytes());
     const size_t o_rtctr = carve(&at, 512 * 128);
     const size_t rbf = k3k_router_bf3_floats((int)T, (int)E);
     const size_t o_rbpart = carve(&at, rbf ? rbf * 4 : 16);
     const size_t o_tiles = carve(&at, maxt * 16), o_ntiles = carve(&at, 4);
-    const size_t o_xflag = carve(&at, 4);
+    const size_t o_xflag = carve(&at, 3 * 4);
     const size_t d512 = (d + 511) / 512 * 512, I512 = (I + 511) / 512 * 512;
     const size_t L512 = (L + 511) / 512 * 512, q512 = d512 > L512 ? d512 : L512;
     const size_t o_xq8b = carve(&at, T * q512 + T * q512 / 32);
@@ -179,8 +179,9 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     const size_t xq = (nQd > nQL ? nQd : nQL) * K3G_P6_QUAD, hq = nQi * K3G_P6_QUAD;
     /* (or six pieces, k3g_rows.hip, whose rows are longer) */
     const size_t xrow = k3k_rows_bytes((int)(d > L ? d : L)), hrow = k3k_rows_bytes((int)I);
-    const size_t o_xr = carve(&at, T * (xq > xrow ? xq : xrow));
-    const size_t o_hr = carve(&at, P * (hq > hrow ? hq : hrow));
+    const size_t o_xr = carve(&at, T * (2 * xq > xrow ? 2 * xq : xrow));
+    const size_t o_hr = carve(&at, P * (2 * hq > hrow ? 2 * hq : hrow));
+    const size_t o_xrow = carve(&at, T), o_hrow = carve(&at, P);
     /* two banks of counters, one per call in turn; each a multiple of 256 bytes */
     /* the larger of the latent layer's geometry and the plain one (a layer without the
      * latent projections may run on a context sized for them) */
@@ -247,6 +248,10 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     c->hq8b = (uint8_t *)(b + o_hq8b);
     c->xr = (uint8_t *)(b + o_xr);
     c->hr = (uint8_t *)(b + o_hr);
+    c->xmore = T * xq;
+    c->hmore = P * hq;
+    c->xrow = (uint8_t *)(b + o_xrow);
+    c->hrow = (uint8_t *)(b + o_hrow);
     c->fused = 1;
     if (hipMemset(c->ws, 0, at) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
         hipFree(c->ws);
@@ -452,7 +457,7 @@ static int experts_gemm(K3gCtx *c, const K3gLayer *L, const float *x, int T,
     k3g_stage_begin(c, K3G_ST_DISPATCH, st);
     rc |= k3k_dispatch_tiles(idx, T * L->topk, L->n_experts, c->cnt, c->base, c->off, c->act,
                              c->nact, c->perm, c->err, tile_cols(T, L->topk, 0), c->tiles,
-                             c->ntiles, c->xflag, st);
+                             c->ntiles, c->xflag, c->hrow, st);
     k3g_stage_end(c, K3G_ST_DISPATCH, st);
     return rc | gemm_body(c, L, x, T, idx, wt, out, contrib, fp8, full, 0, st);
 }
@@ -514,7 +519,7 @@ static int routed_input(K3gCtx *c, const float *z, int T, int n, int fp8,
                         const int32_t *run_flag, hipStream_t st)
 {
     return fp8 ? k3k_xq8(z, T, n, r512(n), c->xq8b, c->xq8b + (size_t)T * r512(n), st)
-               : k3k_x6(z, T, n, c->xr, run_flag, st);
+               : k3k_x6(z, T, n, c->xr, c->xmore, c->xrow, c->xflag + 1, run_flag, st);
 }
 
 /* x's two bf16 pieces (the piece-1 flag cleared before; the shared expert, the latent down and
@@ -547,6 +552,9 @@ static int routed_f6(K3gCtx *c, const K3gLayer *L, int T, int lat, int cols, int
     g.K = lat;
     g.eq = L->experts;
     g.b = c->xr;
+    g.more = c->xmore;
+    g.wrow = c->xrow;
+    g.wide = c->xflag + 1;
     if (!L->down) {                      /* routed experts on x itself */
         g.xb = c->xb;
         g.ldb = r128(L->hidden);
@@ -559,6 +567,9 @@ static int routed_f6(K3gCtx *c, const K3gLayer *L, int T, int lat, int cols, int
     g.max_tiles = max_tiles;
     g.halves = cols > 64;
     g.h = c->hr;
+    g.hmore = c->hmore;
+    g.hrow = c->hrow;
+    g.hwide = c->xflag + 2;
     g.b1 = L->act_b1;
     g.b2 = L->act_b2;
     g.trace = c->trace;
@@ -574,6 +585,9 @@ static int routed_f6(K3gCtx *c, const K3gLayer *L, int T, int lat, int cols, int
     g.rows = lat;
     g.K = I;
     g.b = c->hr;
+    g.more = c->hmore;
+    g.wrow = c->hrow;
+    g.wide = c->xflag + 2;
     g.xb = NULL;
     g.h = NULL;
     g.out = contrib;
@@ -1031,7 +1045,7 @@ int k3g_moe(K3gCtx *c, const K3gLayer *L, const float *x, int T, float *out, int
         /* x's pieces, then the shared expert on the side stream (only the final combine
          * needs it) beside the router, the dispatch and the routed experts on this one */
         c->paths |= 4;
-        int rc = k3k_set_i32(c->xflag, 0, st);
+        int rc = k3k_set_i32(c->xflag, 3, 0, st);
         rc |= gemm_pieces(c, L, x, T, c->gemm_fp8, st);
         if (L->shared_inter > 0) {
             if (hipEventRecord(c->ev_in, st) != hipSuccess ||
@@ -1049,7 +1063,7 @@ int k3g_moe(K3gCtx *c, const K3gLayer *L, const float *x, int T, float *out, int
         k3g_stage_begin(c, K3G_ST_DISPATCH, st);
         rc |= k3k_dispatch_tiles(idx, T * L->topk, L->n_experts, c->cnt, c->base, c->off,
                                  c->act, c->nact, c->perm, c->err, tile_cols(T, L->topk, 1),
-                                 c->tiles, c->ntiles, c->zflag, st);
+                                 c->tiles, c->ntiles, c->zflag, c->hrow, st);
         k3g_stage_end(c, K3G_ST_DISPATCH, st);
         rc |= gemm_body(c, L, x, T, idx, wt, out, c->contrib, c->gemm_fp8, 1, 1, st);
         return rc ? -1 : 0;

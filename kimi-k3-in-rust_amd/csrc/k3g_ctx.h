@@ -66,7 +66,7 @@ struct K3gCtx {
     /* grouped GEMMs on the matrix cores (more than 4 tokens, tiled layouts) */
     uint16_t *xb, *hsb;          /* bf16 pieces of x [2][T][d128], the shared h */
     uint16_t *zb;                /* bf16 pieces of the latent input / aggregate [2][T][L128] */
-    int32_t *zflag;              /* their piece-1 flag (written, not read) */
+    int32_t *zflag;              /* three as xflag, for them (written, not read) */
     float *kpart;                /* K-slice sums of the dense GEMMs */
     float *kpart2;               /* the shared expert's, when it runs on the side stream */
     double *rtpart;              /* K-slice sums of the router's matrix-core logits */
@@ -84,7 +84,10 @@ struct K3gCtx {
     hipEvent_t ev_in, ev_shared;
     int gemm_fp8;                /* routed experts on the FP4 x FP8 matrix cores */
     uint8_t *xr, *hr;            /* the routed experts' input per token and h per pair as FP6
-                                  * pieces, rows of quads (k3g_gemm6.h) */
+                                  * pieces, rows of quads (k3g_gemm6.h), the second four pieces
+                                  * of all rows xmore and hmore bytes on */
+    size_t xmore, hmore;
+    uint8_t *xrow, *hrow;        /* rows with such second pieces (1) */
     uint8_t *xq8b, *hq8b;        /* MXFP8 x [T][d512] + scales, h [T*k][I512] + scales */
     unsigned long long *trace;   /* optional per-ticket timestamps of the fused kernel */
     /* optional pinned host copies that the fused kernel writes directly (the routing, a

@@ -137,7 +137,7 @@ __device__ __forceinline__ void k3d_block_exscan_n(int (&v)[N], int (&tot)[N], i
 
 /* Column tiles of up to `cols` pairs per expert (64 or K3G_TILE_COLS), largest first: every full
  * tile (in expert order), then the experts' last partial tiles by their count of 16-column
- * blocks, 8 down to 1 (in expert order within a count); clears *flag. Called by every
+ * blocks, 8 down to 1 (in expert order within a count); clears flag[0 .. 2]. Called by every
  * thread of a block of 1024 (thread e < E for expert e, its pair count and first sorted
  * position); lds holds (16 + 1) * 9 ints. */
 __device__ __forceinline__ void k3d_build_tiles(int e, int E, int cnt, int off_e, int cols,
@@ -161,7 +161,8 @@ __device__ __forceinline__ void k3d_build_tiles(int e, int E, int cnt, int off_e
             tiles[base + v[j]] = make_int4(e, off_e + cols * nfull, rem, 0);
         base += tot[j];
     }
-    if (e == 0) { *ntiles = base; *flag = 0; }
+    if (e == 0) *ntiles = base;
+    if (e < 3) flag[e] = 0;
 }
 
 __device__ __forceinline__ float k3d_wave_sum(float v)

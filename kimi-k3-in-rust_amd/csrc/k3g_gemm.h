@@ -160,47 +160,84 @@ __device__ __forceinline__ gm_v32f gm_from_fp6(const gm_v6u &p, float scale)
     return r;
 }
 
+/* ev, od less the piece w at its scale byte */
+__device__ __forceinline__ void gm_less(gm_v16f &ev, gm_v16f &od, const gm_v6u &w, uint32_t sb)
+{
+    const gm_v32f y = gm_from_fp6(w, __uint_as_float(sb << 23));
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        ev[i] -= y[2 * i];
+        od[i] -= y[2 * i + 1];
+    }
+}
+
 /* 32 values (even and odd elements apart) as NP pieces: piece p's six dwords at d + 6 p, its E8M0
- * byte s[p]; each piece's scale puts the largest remainder in [4, 8). True when a value is
- * infinite or NaN (the pieces then mean nothing). */
+ * byte s[p]; each piece's scale puts the largest remainder in [4, 8), so a piece leaves at most
+ * 1/16 of the block's largest remainder and 1/32 in the mean. ev and od become what the pieces
+ * before the last leave. */
 template <int NP>
-__device__ __forceinline__ bool gm_pieces(gm_v16f ev, gm_v16f od, uint32_t (&d)[6 * NP],
+__device__ __forceinline__ void gm_pieces(gm_v16f &ev, gm_v16f &od, uint32_t (&d)[6 * NP],
                                           uint8_t (&s)[NP])
 {
-    bool bad = false;
-#pragma unroll
-    for (int i = 0; i < 16; ++i)
-        bad |= !(fabsf(ev[i]) < __builtin_inff()) || !(fabsf(od[i]) < __builtin_inff());
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         float m = 0.0f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) m = fmaxf(m, fmaxf(fabsf(ev[i]), fabsf(od[i])));
         const int sb = m > 0.0f ? max((int)(__float_as_uint(m) >> 23) - 2, 1) : 127;
-        const float scale = __uint_as_float((uint32_t)sb << 23);
-        const gm_v6u w = gm_to_fp6(ev, od, scale);
-        if (p < NP - 1) {
-            const gm_v32f y = gm_from_fp6(w, scale);
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                ev[i] -= y[2 * i];
-                od[i] -= y[2 * i + 1];
-            }
-        }
+        const gm_v6u w = gm_to_fp6(ev, od, __uint_as_float((uint32_t)sb << 23));
+        if (p < NP - 1) gm_less(ev, od, w, sb);
 #pragma unroll
         for (int i = 0; i < 6; ++i) d[6 * p + i] = w[i];
         s[p] = (uint8_t)sb;
     }
+}
+
+/* a value is infinite or NaN (pieces then mean nothing) */
+__device__ __forceinline__ bool gm_bad(const gm_v16f &ev, const gm_v16f &od)
+{
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+        bad |= !(fabsf(ev[i]) < __builtin_inff()) || !(fabsf(od[i]) < __builtin_inff());
     return bad;
 }
 
-/* One block of 32 values as four pieces into its place in a quad (k3g_gemm6.h): step j, block q.
- * A block with an infinity or NaN gets the NaN scale, so the products are NaN as they were. */
-__device__ __forceinline__ void gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *quad, int j, int q)
+/* How far a block's values lie below its largest: the sum over its 32 values (zeros left out) of
+ * the square of the binary orders between, each at most 16. Normally distributed values 243, one
+ * block in 100,000 above 790; silu(g) u of such g and u 674, one in 100,000 above 1994; normal
+ * values beside one 16 to 31 times as large 992 in the mean, beside one 256 times as large 2790. */
+__device__ __forceinline__ int gm_spread(const gm_v16f &ev, const gm_v16f &od)
 {
-    uint32_t d[24];
-    uint8_t s[4];
-    const bool bad = gm_pieces<4>(ev, od, d, s);
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) m = fmaxf(m, fmaxf(fabsf(ev[i]), fabsf(od[i])));
+    const int top = (int)(__float_as_uint(m) >> 23);
+    int sum = 0;
+    auto add = [&](float v) {
+        const int n = min(top - (int)(__float_as_uint(v) << 1 >> 24), 16);
+        sum += v == 0.0f ? 0 : n * n;
+    };
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        add(ev[i]);
+        add(od[i]);
+    }
+    return sum;
+}
+
+/* Spreads from which on a block takes eight pieces. Four leave 3e-7 of the block's largest value
+ * on every one of its values: less than the two bf16 pieces that x had been (2.5e-6 of each
+ * value) down to an eighth of it, and less than the bf16 piece with its MXFP8 remainder that h
+ * had been (3.9e-5) down to 1/130. Blocks whose values lie lower get four pieces more: 2e-14
+ * beside a value 16 times as large, 1.6e-11 beside 1000, 1.6e-8 beside 10^6. */
+#define GM_WIDE_X 832
+#define GM_WIDE_H 2560
+
+/* One block's four pieces in a quad (k3g_gemm6.h): step j, block q. */
+__device__ __forceinline__ void gm_put_pieces(const uint32_t (&d)[24], uint32_t scales,
+                                              uint8_t *quad, int j, int q)
+{
     uint8_t *o = quad + 384 * j;
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
@@ -208,8 +245,33 @@ __device__ __forceinline__ void gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *
             make_uint4(d[6 * p], d[6 * p + 1], d[6 * p + 2], d[6 * p + 3]);
         *(uint2 *)(o + 256 + 32 * p + 8 * q) = make_uint2(d[6 * p + 4], d[6 * p + 5]);
     }
-    *(uint32_t *)(quad + 1536 + 16 * j + 4 * q) =
-        bad ? 0xffffffffu : s[0] | (uint32_t)s[1] << 8 | (uint32_t)s[2] << 16 | (uint32_t)s[3] << 24;
+    *(uint32_t *)(quad + 1536 + 16 * j + 4 * q) = scales;
+}
+
+__device__ __forceinline__ uint32_t gm_bytes(const uint8_t (&s)[4])
+{
+    return s[0] | (uint32_t)s[1] << 8 | (uint32_t)s[2] << 16 | (uint32_t)s[3] << 24;
+}
+
+/* One block of 32 values into its place in a quad, and where its spread is `at` or more (true) the
+ * next four pieces into the same place `more` bytes on; elsewhere that place gets scales of zero.
+ * A block with an infinity or NaN gets the NaN scale, so the products are NaN as they were. */
+__device__ __forceinline__ bool gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *quad, size_t more,
+                                               int at, int j, int q)
+{
+    uint32_t d[24];
+    uint8_t s[4];
+    const bool bad = gm_bad(ev, od), w = !bad && gm_spread(ev, od) >= at;
+    gm_pieces<4>(ev, od, d, s);
+    gm_put_pieces(d, bad ? 0xffffffffu : gm_bytes(s), quad, j, q);
+    if (w) {
+        gm_less(ev, od, gm_v6u{d[18], d[19], d[20], d[21], d[22], d[23]}, s[3]);
+        gm_pieces<4>(ev, od, d, s);
+        gm_put_pieces(d, gm_bytes(s), quad + more, j, q);
+    } else {
+        *(uint32_t *)(quad + more + 1536 + 16 * j + 4 * q) = 0;
+    }
+    return w;
 }
 
 /* This wave's LDS writes are visible to its own later reads, whichever lane made them */
@@ -225,13 +287,15 @@ __device__ __forceinline__ void gm_wave_sync()
 
 /* A wave's gate and up sums (row groups r < RG / 2 the gates, the others the ups of the same 8 RG
  * features from f0 on; column block n's column lane % 16) -> activations -> h rows p0 + column
- * as FP6 quads of `rows` features (those past it zero), columns below np. wl: GM_HLDS bytes of
+ * as FP6 quads of `rows` features (those past it zero; rows with blocks of eight pieces are marked in
+ * wrow and raise *wide), columns below np. wl: GM_HLDS bytes of
  * LDS of this wave's own. The sums go to rows [feature block b][column block n][column c] of 32
  * gates and 32 ups (each padded to 36), the activations over the gates, eight per lane and
  * block; then every lane makes the pieces of one row. */
 template <int RG, int NBW>
 __device__ __forceinline__ void gm_store_h(k3v4f (&acc)[RG][NBW], float *wl, int lane, int f0,
-                                           int rows, int p0, int np, float b1, float b2, uint8_t *h)
+                                           int rows, int p0, int np, float b1, float b2, uint8_t *h,
+                                           size_t more, uint8_t *wrow, int32_t *wide)
 {
     const int c16 = lane & 15, q4 = lane >> 4;
     const int nQh = (rows + 511) / 512;
@@ -272,8 +336,11 @@ __device__ __forceinline__ void gm_store_h(k3v4f (&acc)[RG][NBW], float *wl, int
                 ev[2 * i] = v.x; od[2 * i] = v.y; ev[2 * i + 1] = v.z; od[2 * i + 1] = v.w;
             }
             const int f = f0 + 32 * b;
-            gm_store_block(ev, od, h + ((size_t)(p0 + col) * nQh + (f >> 9)) * K3G_P6_QUAD,
-                           (f >> 7) & 3, (f >> 5) & 3);
+            if (gm_store_block(ev, od, h + ((size_t)(p0 + col) * nQh + (f >> 9)) * K3G_P6_QUAD, more,
+                               GM_WIDE_H, (f >> 7) & 3, (f >> 5) & 3)) {
+                wrow[p0 + col] = 1;
+                *wide = 1;
+            }
         }
         gm_wave_sync();
     };

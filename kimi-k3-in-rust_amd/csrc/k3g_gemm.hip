@@ -355,7 +355,7 @@ __device__ __forceinline__ void gm_tile(const K3kGemm &g, const GmTile &t)
     if constexpr (AF == 0) {
         __syncthreads();                 /* every wave is done with the LDS */
         gm_store_h<4, NB>(acc, (float *)(t.ldsp + t.w * GM_HLDS), lane, t.orow0, g.rows, t.p0, t.np,
-                          g.b1, g.b2, g.h6);
+                          g.b1, g.b2, g.h6, g.hmore, g.hrow, g.hwide);
         return;
     }
     if (g.mode == 0) {
@@ -572,6 +572,9 @@ k_gemm6(const K3kGemm6 g)
         b.tiles = g.tiles;
         b.ntiles = g.ntiles;
         b.h6 = g.h;
+        b.hmore = g.hmore;
+        b.hrow = g.hrow;
+        b.hwide = g.hwide;
         b.b1 = g.b1;
         b.b2 = g.b2;
         b.nft = g.nft;
@@ -586,6 +589,10 @@ k_gemm6(const K3kGemm6 g)
             case 16 * 4 + 2: g6_run<MODE, 2, 4>(g, t); break;
             case 16 * 4 + 3: g6_run<MODE, 3, 4>(g, t); break;
             case 16 * 4 + 4: g6_run<MODE, 4, 4>(g, t); break;
+            case 256 + 16 * 4 + 1: g6_run<MODE, 1, 4, true>(g, t); break;
+            case 256 + 16 * 4 + 2: g6_run<MODE, 2, 4, true>(g, t); break;
+            case 256 + 16 * 4 + 3: g6_run<MODE, 3, 4, true>(g, t); break;
+            case 256 + 16 * 4 + 4: g6_run<MODE, 4, 4, true>(g, t); break;
             default: return;
         }
     }
@@ -982,16 +989,18 @@ extern "C" int k3k_gemm(const K3kGemm *g, hipStream_t st)
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-extern "C" int k3k_x6(const float *x, int T, int K, uint8_t *o, const int32_t *run_flag,
-                      hipStream_t st)
+extern "C" int k3k_x6(const float *x, int T, int K, uint8_t *o, size_t more, uint8_t *wrow,
+                      int32_t *wide, const int32_t *run_flag, hipStream_t st)
 {
-    if (T < 1 || K < 32 || K % 32 || ((uintptr_t)o & 15)) return -1;
-    const long long n = (long long)T * 4 * ((K + 127) / 128);
-    const dim3 grid((unsigned)((n + 255) / 256));
+    if (T < 1 || K < 32 || K % 32 || ((uintptr_t)o & 15) || more % 16 || !wrow || !wide ||
+        more < (size_t)T * ((K + 511) / 512) * G6_QB)
+        return -1;
+    const int nbk = 4 * ((K + 127) / 128);
+    const dim3 grid((unsigned)T), block(nbk < 256 ? (nbk + 63) / 64 * 64 : 256);
     if (((uintptr_t)x & 15) == 0)
-        hipLaunchKernelGGL(k_x6<true>, grid, dim3(256), 0, st, x, T, K, o, run_flag);
+        hipLaunchKernelGGL(k_x6<true>, grid, block, 0, st, x, K, o, more, wrow, wide, run_flag);
     else
-        hipLaunchKernelGGL(k_x6<false>, grid, dim3(256), 0, st, x, T, K, o, run_flag);
+        hipLaunchKernelGGL(k_x6<false>, grid, block, 0, st, x, K, o, more, wrow, wide, run_flag);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1002,7 +1011,8 @@ extern "C" int k3k_gemm6(const K3kGemm6 *g, hipStream_t st)
         !g->ntiles || g->max_tiles < 1 || !g->perm || g->topk < 1 || g->halves < 0 || g->halves > 1 || g->K < 32 || g->K % 32 ||
         g->rows < 32 || g->rows % 32)
         return -1;
-    if (g->mode == 0 ? (!g->h || ((uintptr_t)g->h & 15) != 0)
+    if (!g->wide || !g->wrow || g->more % 16 || (g->K + 127) / 128 > (G6_LDS - G6_LIST) / 2) return -1;
+    if (g->mode == 0 ? (!g->h || ((uintptr_t)g->h & 15) != 0 || g->hmore % 16 || !g->hrow || !g->hwide)
                      : (!g->out || g->ldo < g->rows || g->ldo % 4))
         return -1;
     if (g->xb && (g->mode != 0 || !g->lo_flag || g->ldb < g->K || g->ldb % GM_KC)) return -1;

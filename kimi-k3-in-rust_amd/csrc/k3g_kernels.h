@@ -148,6 +148,9 @@ typedef struct {
     uint8_t *hq, *hs;
     int ldhq;                 /* bytes per h row (scales: ldhq / 32) */
     uint8_t *h6;              /* k3k_gemm with MXFP4 weights: h as FP6 quads (K3kGemm6) */
+    size_t hmore;
+    uint8_t *hrow;
+    int32_t *hwide;
     /* dense tiled-bf16 GEMMs only: K cut into ksplit slices of whole 128-column steps
      * (1: none); the slices' fp32 sums go to part ([ksplit][columns][2][rows] gate/up,
      * [ksplit][columns][rows] down) and k3k_gemm reduces them in slice order */
@@ -169,12 +172,18 @@ typedef struct {
     const K3ExpertQ *eq;      /* mode 0: p1, p3; mode 1: p2 (tiled MXFP4) */
     const uint8_t *b;         /* activation rows of ceil(K / 512) quads: by token (mode 0) or
                                * by sorted position (mode 1) */
+    size_t more;              /* bytes from a quad to the second four pieces of its blocks */
+    const uint8_t *wrow;      /* per row of b: it has such blocks */
+    const int32_t *wide;      /* 0: no row has */
     const int32_t *perm;      /* sorted position -> pair id (t * topk + j) */
     int topk;
     const int32_t *tiles;     /* {expert, first sorted position, count, 0} */
     const int32_t *ntiles;
     int max_tiles;            /* bound on *ntiles (grid size) */
-    uint8_t *h;               /* mode 0 out: rows of ceil(rows / 512) quads by sorted position */
+    uint8_t *h;               /* mode 0 out: rows of ceil(rows / 512) quads by sorted position, */
+    size_t hmore;             /* as b, more, wrow (set where h has such blocks; zero before) and */
+    uint8_t *hrow;            /* wide */
+    int32_t *hwide;
     float b1, b2;             /* activation caps */
     float *out;               /* mode 1 out: row perm[column], stride ldo */
     int ldo;
@@ -192,8 +201,10 @@ typedef struct {
 } K3kGemm6;
 
 int k3k_gemm6(const K3kGemm6 *g, hipStream_t st);
-/* x (fp32 [T][K]) -> activation quads [T][ceil(K / 512)]; nothing when *run_flag is 0 */
-int k3k_x6(const float *x, int T, int K, uint8_t *o, const int32_t *run_flag, hipStream_t st);
+/* x (fp32 [T][K]) -> activation quads [T][ceil(K / 512)] and, where a block needs them, its second
+ * four pieces `more` bytes on (wrow[t] = 1, else 0; *wide raised); nothing when *run_flag is 0 */
+int k3k_x6(const float *x, int T, int K, uint8_t *o, size_t more, uint8_t *wrow, int32_t *wide,
+           const int32_t *run_flag, hipStream_t st);
 /* The K slices a dense GEMM of nft feature tiles x ntl column tiles over K columns uses
  * to give the GPU about 256 workgroups (1 = no split), and the part buffer bytes a
  * context needs for any column count (rows: the GEMM's output rows; x2 for gate/up). */
@@ -206,7 +217,7 @@ int k3k_gemm_f8(const K3kGemm *g, hipStream_t st);
  * to +-448): bytes [T][ldq], scales [T][ldq / 32]; the padding columns stay zero. */
 int k3k_xq8(const float *x, int T, int d, int ldq, uint8_t *xq, uint8_t *xs, hipStream_t st);
 /* column tiles of up to cols (64 or 128) pairs from the dispatch's per-expert ranges; clears
- * *flag */
+ * flag[0 .. 2] */
 int k3k_gemm_tiles(const int32_t *off, int E, int cols, int32_t *tiles, int32_t *ntiles,
                    int32_t *flag, hipStream_t st);
 /* x -> bf16 pieces [2][T][ldb]; *flag = 1 when some piece 1 is not zero */
@@ -311,11 +322,11 @@ int k3k_dispatch(const int32_t *idx, int P, int E, int32_t *cnt, int32_t *base,
                  int32_t *off, int32_t *act, int32_t *nact, int32_t *perm, int *err,
                  hipStream_t st);
 /* The same, followed by the grouped GEMMs' column tiles (as k3k_gemm_tiles), in one
- * launch when P <= 4096. */
+ * launch when P <= 4096; clears prow[0 .. P - 1]. */
 int k3k_dispatch_tiles(const int32_t *idx, int P, int E, int32_t *cnt, int32_t *base,
                        int32_t *off, int32_t *act, int32_t *nact, int32_t *perm, int *err,
                        int cols, int32_t *tiles, int32_t *ntiles, int32_t *flag,
-                       hipStream_t st);
+                       uint8_t *prow, hipStream_t st);
 
 /* h = act(W1 z, W3 z) and contrib = W2 h for every active expert's pairs. maxU bounds
  * the number of active experts (min(E, T*k)); maxtok bounds tokens per expert. */
@@ -348,7 +359,7 @@ int k3k_rmsnorm(float *y, const float *x, const float *w, int n, int T, float ep
                 hipStream_t st);
 
 /* *p = v, in stream order */
-int k3k_set_i32(int32_t *p, int32_t v, hipStream_t st);
+int k3k_set_i32(int32_t *p, int n, int32_t v, hipStream_t st);
 
 /* y += a, elementwise */
 int k3k_add(float *y, const float *a, size_t n, hipStream_t st);

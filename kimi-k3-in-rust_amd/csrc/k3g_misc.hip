@@ -36,7 +36,8 @@ __device__ __forceinline__ int k3d_key(const int32_t *idx, int p, int P, int E, 
 #define K3G_DSORT 4096
 __global__ void __launch_bounds__(1024)
 k_disp_sort(const int32_t *idx, int P, int E, int32_t *off, int32_t *act, int32_t *nact,
-            int32_t *perm, int *err, int cols, int4 *tiles, int32_t *ntiles, int32_t *flag)
+            int32_t *perm, int *err, int cols, int4 *tiles, int32_t *ntiles, int32_t *flag,
+            uint8_t *prow)
 {
     __shared__ __attribute__((aligned(16))) uint32_t kv[2][K3G_DSORT];
     __shared__ int cnt[K3G_MAX_EXPERTS];
@@ -46,6 +47,8 @@ k_disp_sort(const int32_t *idx, int P, int E, int32_t *off, int32_t *act, int32_
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int nch = (P + 63) / 64;
     cnt[tid] = 0;
+    if (tiles)
+        for (int i = tid; i < P; i += 1024) prow[i] = 0;
     if (P <= 1024) {
         /* wc[q][e]: wave q's pairs of expert e */
         uint16_t (*wc)[K3G_MAX_EXPERTS] = (uint16_t (*)[K3G_MAX_EXPERTS])kv;
@@ -188,12 +191,13 @@ k_disp_scan(const int32_t *cnt, int nch, int E, int32_t *base, int32_t *tot)
 
 __global__ void __launch_bounds__(256)
 k_disp_scatter(const int32_t *idx, int P, int E, const int32_t *base, const int32_t *tot,
-               int32_t *off, int32_t *act, int32_t *nact, int32_t *perm)
+               int32_t *off, int32_t *act, int32_t *nact, int32_t *perm, uint8_t *prow)
 {
     __shared__ int wc[4][K3G_MAX_EXPERTS];
     __shared__ int first[K3G_MAX_EXPERTS];
     __shared__ int red[5 * 2];
     const int c = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (prow && c * K3G_DCH + tid < P) prow[c * K3G_DCH + tid] = 0;
     for (int e = tid; e < E; e += 256) wc[0][e] = wc[1][e] = wc[2][e] = wc[3][e] = 0;
     /* the expert ranges: thread i scans experts 4 i .. 4 i + 3 (E <= 1024) */
     {
@@ -249,13 +253,14 @@ k_disp_scatter(const int32_t *idx, int P, int E, const int32_t *base, const int3
 extern "C" int k3k_dispatch_tiles(const int32_t *idx, int P, int E, int32_t *cnt,
                                   int32_t *base, int32_t *off, int32_t *act, int32_t *nact,
                                   int32_t *perm, int *err, int cols, int32_t *tiles,
-                                  int32_t *ntiles, int32_t *flag, hipStream_t st)
+                                  int32_t *ntiles, int32_t *flag, uint8_t *prow,
+                                  hipStream_t st)
 {
     if (E < 1 || E > K3G_MAX_EXPERTS || P < 1) return -1;
     if (tiles && cols != 64 && cols != K3G_TILE_COLS) return -1;
     if (P <= K3G_DSORT) {
         hipLaunchKernelGGL(k_disp_sort, dim3(1), dim3(1024), 0, st, idx, P, E, off, act, nact,
-                           perm, err, cols, (int4 *)tiles, ntiles, flag);
+                           perm, err, cols, (int4 *)tiles, ntiles, flag, prow);
         return hipGetLastError() == hipSuccess ? 0 : -1;
     }
     const int nch = (P + K3G_DCH - 1) / K3G_DCH;
@@ -265,7 +270,7 @@ extern "C" int k3k_dispatch_tiles(const int32_t *idx, int P, int E, int32_t *cnt
     hipLaunchKernelGGL(k_disp_scan, dim3((E + 63) / 64), dim3(64), 0, st, cnt, nch, E, base,
                        tot);
     hipLaunchKernelGGL(k_disp_scatter, dim3(nch), dim3(256), 0, st, idx, P, E, base, tot, off,
-                       act, nact, perm);
+                       act, nact, perm, tiles ? prow : nullptr);
     if (hipGetLastError() != hipSuccess) return -1;
     return tiles ? k3k_gemm_tiles(off, E, cols, tiles, ntiles, flag, st) : 0;
 }
@@ -275,7 +280,7 @@ extern "C" int k3k_dispatch(const int32_t *idx, int P, int E, int32_t *cnt, int3
                             int *err, hipStream_t st)
 {
     return k3k_dispatch_tiles(idx, P, E, cnt, base, off, act, nact, perm, err, 0,
-                              nullptr, nullptr, nullptr, st);
+                              nullptr, nullptr, nullptr, nullptr, st);
 }
 
 /* ---------------------------------------------------------------- combine ---- */
@@ -489,17 +494,17 @@ extern "C" int k3k_copy(void *dst, const void *src, size_t n, hipStream_t st)
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-/* *p = v (a flag cleared in stream order by a kernel, which a captured graph replays
+/* p[0 .. n - 1] = v, n <= 64 (flags cleared in stream order by a kernel, which a captured graph replays
  * the same way every time) */
-__global__ void __launch_bounds__(64) k_set_i32(int32_t *p, int32_t v)
+__global__ void __launch_bounds__(64) k_set_i32(int32_t *p, int n, int32_t v)
 {
-    if (threadIdx.x == 0) *p = v;
+    if ((int)threadIdx.x < n) p[threadIdx.x] = v;
 }
 
-extern "C" int k3k_set_i32(int32_t *p, int32_t v, hipStream_t st)
+extern "C" int k3k_set_i32(int32_t *p, int n, int32_t v, hipStream_t st)
 {
-    if (!p) return -1;
-    hipLaunchKernelGGL(k_set_i32, dim3(1), dim3(64), 0, st, p, v);
+    if (!p || n < 1 || n > 64) return -1;
+    hipLaunchKernelGGL(k_set_i32, dim3(1), dim3(64), 0, st, p, n, v);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -57,7 +57,8 @@ k_rows_x(const float *__restrict__ x, int T, int K, uint8_t *__restrict__ o)
     }
     uint32_t d[6 * RW_NP];
     uint8_t s[RW_NP];
-    const bool bad = gm_pieces<RW_NP>(ev, od, d, s);
+    const bool bad = gm_bad(ev, od);
+    gm_pieces<RW_NP>(ev, od, d, s);
     uint8_t *q = o + ((size_t)t * (nbk / 4) + (k >> 2)) * RW_STEP;
 #pragma unroll
     for (int p = 0; p < RW_NP; ++p) {
