@@ -177,7 +177,7 @@ int k3g_ctx_create(K3gCtx **out, int device, const K3gLayer *s, int max_tokens)
     const size_t o_hq8b = carve(&at, P * I512 + P * I512 / 32);
     /* the routed experts' input and h as FP6 pieces (k3g_gemm6.h) */
     const size_t xq = (nQd > nQL ? nQd : nQL) * K3G_P6_QUAD, hq = nQi * K3G_P6_QUAD;
-    /* (or six pieces, k3g_rows.hip, whose rows are longer) */
+    /* (or eight pieces, k3g_rows.hip) */
     const size_t xrow = k3k_rows_bytes((int)(d > L ? d : L)), hrow = k3k_rows_bytes((int)I);
     const size_t o_xr = carve(&at, T * (2 * xq > xrow ? 2 * xq : xrow));
     const size_t o_hr = carve(&at, P * (2 * hq > hrow ? 2 * hq : hrow));

@@ -4,12 +4,14 @@
  * The engine computes, per (token, slot) pair, three MXFP4 GEMVs per expert
  * (src/core/k3_ops.c:604-640, :751-778); here an expert's pairs share one pass over its rows,
  * eight at a time. The codes and scales go to v_mfma_scale_f32_16x16x128_f8f6f4 as they are
- * stored. An activation is the sum of six FP6 (E2M3) pieces, each with its own E8M0 scale per
+ * stored. An activation is the sum of eight FP6 (E2M3) pieces, each with its own E8M0 scale per
  * 32 values: each piece leaves at most 1/16 of the block's largest value and 1/32 in the mean,
- * so six hold fp32's 24 bits (7e-10 of normally distributed values, 2-norm). The pieces are six
+ * so eight hold fp32's 24 bits of values down to 2^-8 of the largest at worst, 2^-16 in the mean
+ * (beside one 10^6 times as large 1.6e-8 is left of normally distributed values, 2-norm). A pair
+ * with a block where that is not enough is summed without pieces (k_rows_x). The pieces are eight
  * columns of the B operand (two pairs per instruction, columns 8 pi + piece), 128 products
  * sum exactly before they are added to the fp32 accumulator, and a row's result is the
- * sum of its six columns.
+ * sum of its eight columns.
  *
  * Bound by the weight stream. A wave's operand rows are 64 bytes at a stride of a whole row, which
  * the cache serves badly (each line is asked for in two halves), so every wave copies its own
@@ -21,24 +23,28 @@
  * against a wave per row tile with fp32 multiply-adds, which decodes every weight once per
  * four tokens; error against 64 bits 3.2e-7 -> 1.6e-7.
  *
- * Activation rows: per 128 columns 640 bytes: dwords 0 .. 3 of piece p of block q at
- * 16 (4 p + q), dwords 4 and 5 at 384 + 8 (4 p + q), the scale byte at 576 + 4 p + q; a row is
+ * Activation rows: per 128 columns 800 bytes: dwords 0 .. 3 of piece p of block q at
+ * 16 (4 p + q), dwords 4 and 5 at 512 + 8 (4 p + q), the scale byte at 768 + 4 p + q; a row is
  * whole intervals of 256 columns, zero past the end. */
 #include "k3g_gemm.h"
 
-#define RW_STEP 640                 /* bytes of 128 columns of an activation row */
-#define RW_NP 6                     /* pieces */
+#define RW_STEP 800                 /* bytes of 128 columns of an activation row */
+#define RW_NP 8                     /* pieces */
 #define RW_PAIRS 8                  /* pairs per pass */
 #define RW_WST 4096                 /* a wave's weights of one interval: 32 rows x 128 bytes */
 #define RW_SCL 768                  /* a wave's scales of two intervals: 32 rows x 20 bytes */
-#define RW_BST (RW_PAIRS * 2 * RW_STEP)
+#define RW_BST ((RW_PAIRS * 2 * RW_STEP + 1023) / 1024 * 1024)   /* whole copy instructions */
 #define RW_B0 (4 * 3 * RW_WST)
 #define RW_S0 (RW_B0 + 2 * RW_BST)
 #define RW_LDS (RW_S0 + 4 * 2 * RW_SCL)
 
 typedef int rw_v8i __attribute__((ext_vector_type(8)));
 
-/* x (fp32 [T][K]) -> activation rows, one thread per block of 32 */
+/* x (fp32 [T][K]) -> activation rows, one thread per block of 32. The scales are NaN where a value
+ * is not finite, and where the pieces leave more than 2^-22 of all but one or an eighth of the
+ * block's values that are not zero: values of less than about 2^-20 of its largest, or a block that
+ * small that a scale has no byte. The row's products are then NaN, and are summed again from the
+ * fp32 values (rw_plain). */
 __global__ void __launch_bounds__(256)
 k_rows_x(const float *__restrict__ x, int T, int K, uint8_t *__restrict__ o)
 {
@@ -47,43 +53,59 @@ k_rows_x(const float *__restrict__ x, int T, int K, uint8_t *__restrict__ o)
     if (b >= (long long)T * nbk) return;
     const int t = (int)(b / nbk), k = (int)(b - (long long)t * nbk);
     gm_v16f ev = {}, od = {};
+    const float4 *src = (const float4 *)(x + (size_t)t * K + 32 * k);
     if (32 * k < K) {
-        const float *p = x + (size_t)t * K + 32 * k;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            const float4 v = ((const float4 *)p)[i];
+            const float4 v = src[i];
             ev[2 * i] = v.x; od[2 * i] = v.y; ev[2 * i + 1] = v.z; od[2 * i + 1] = v.w;
         }
     }
     uint32_t d[6 * RW_NP];
     uint8_t s[RW_NP];
-    const bool bad = gm_bad(ev, od);
+    bool bad = gm_bad(ev, od);
     gm_pieces<RW_NP>(ev, od, d, s);
+    constexpr int LP = 6 * (RW_NP - 1);
+    gm_less(ev, od, gm_v6u{d[LP], d[LP + 1], d[LP + 2], d[LP + 3], d[LP + 4], d[LP + 5]}, s[RW_NP - 1]);
+    if (32 * k < K) {
+        int n = 0, left = 0;
+        auto look = [&](float v, float r) {
+            n += v != 0.0f;
+            left += fabsf(r) > 0x1p-22f * fabsf(v);
+        };
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float4 v = src[i];
+            look(v.x, ev[2 * i]); look(v.y, od[2 * i]); look(v.z, ev[2 * i + 1]); look(v.w, od[2 * i + 1]);
+        }
+        bad |= left > 0 && left >= n - 1 - n / 8;
+    }
     uint8_t *q = o + ((size_t)t * (nbk / 4) + (k >> 2)) * RW_STEP;
 #pragma unroll
     for (int p = 0; p < RW_NP; ++p) {
         const int u = 4 * p + (k & 3);
         *(uint4 *)(q + 16 * u) = make_uint4(d[6 * p], d[6 * p + 1], d[6 * p + 2], d[6 * p + 3]);
-        *(uint2 *)(q + 384 + 8 * u) = make_uint2(d[6 * p + 4], d[6 * p + 5]);
-        q[576 + u] = bad ? 255 : s[p];
+        *(uint2 *)(q + 512 + 8 * u) = make_uint2(d[6 * p + 4], d[6 * p + 5]);
+        q[768 + u] = bad ? 255 : s[p];
     }
 }
 
-/* A row's product in fp32, column by column: what an infinity or NaN, or a sum that overflowed,
- * needs, for the pieces have no infinities. */
+/* A row's product column by column: what an infinity or NaN, a sum that overflowed, or a block of
+ * too wide a range needs, for the pieces have no infinities. One lane sums all columns, so in
+ * double. */
 __device__ __attribute__((noinline)) float rw_plain(const uint8_t *w, const uint8_t *s,
                                                     const float *x, int K)
 {
-    float a = 0.0f;
+    double a = 0.0;
     for (int c = 0; c < K; c += 8) {
         uint32_t v;
         __builtin_memcpy(&v, w + c / 2, 4);
         float f[8];
         k3d_fp4x8(v, k3d_e8m0(s[c / 32]), f);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) a = fmaf(f[i], x[c + i], a);
+        for (int i = 0; i < 8; ++i) a = fma((double)f[i], (double)x[c + i], a);
     }
-    return a;
+    return (float)a;
 }
 
 /* One pass over a workgroup's rows for the np <= 2 NG pairs at sorted positions p0 .. */
@@ -136,15 +158,15 @@ __device__ __forceinline__ void rw_pass(const K3kRows &g, const K3ExpertQ &q, in
         const int mis = (int)((uintptr_t)(smat(i) + (size_t)row(i) * ks) & 3);
         sat[r] = (uint32_t)(RW_S0 + w * 2 * RW_SCL + 20 * i + mis + q4);
     }
-    /* the activation copies: 160 NG units of 16 bytes an interval, wave w the 64-unit instructions
+    /* the activation copies: 200 NG units of 16 bytes an interval, wave w the 64-unit instructions
      * w, w + 4, ... */
-    constexpr int NI = (160 * NG + 63) / 64, NB = (NI + 3) / 4;
+    constexpr int UP = RW_STEP / 8, NI = (2 * UP * NG + 63) / 64, NB = (NI + 3) / 4;
     const uint8_t *bsrc[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-        const int u = min(64 * (4 * i + w) + lane, 160 * NG - 1), pi = u / 80;
+        const int u = min(64 * (4 * i + w) + lane, 2 * UP * NG - 1), pi = u / UP;
         const int p = g.perm[p0 + (pi < np ? pi : 0)];
-        bsrc[i] = g.x + (size_t)(MODE == 0 ? p / g.topk : p) * ns * RW_STEP + 16 * (u - 80 * pi);
+        bsrc[i] = g.x + (size_t)(MODE == 0 ? p / g.topk : p) * ns * RW_STEP + 16 * (u - UP * pi);
     }
     auto bcopy = [&](int s) {
         const uint32_t l = lds + RW_B0 + (s & 1) * RW_BST;
@@ -176,9 +198,9 @@ __device__ __forceinline__ void rw_pass(const K3kRows &g, const K3ExpertQ &q, in
         }
     };
     /* operand reads: row i's unit u of an interval at (i / 8) 1024 + (i % 8) 128 + 16 (u ^ i % 8);
-     * column 8 pi + piece (pieces past the sixth read the sixth and are left out at the end) */
+     * column 8 pi + piece */
     const uint32_t abase = 3 * w * RW_WST + (c16 >> 3) * 1024 + (c16 & 7) * 128;
-    const int pc = min(c16 & 7, RW_NP - 1), bu = 4 * pc + q4;
+    const int bu = 4 * (c16 & 7) + q4;
     const uint32_t bbase = RW_B0 + (c16 >> 3) * 2 * RW_STEP;
     auto interval = [&](auto par, int s, int slot) {
         constexpr int PAR = decltype(par)::value;
@@ -210,8 +232,8 @@ __device__ __forceinline__ void rw_pass(const K3kRows &g, const K3ExpertQ &q, in
             for (int n = 0; n < NG; ++n) {
                 const uint8_t *b = ldsp + bbase + (s & 1) * RW_BST + (4 * n + st) * RW_STEP;
                 const uint4 u = *(const uint4 *)(b + 16 * bu);
-                const uint2 v = *(const uint2 *)(b + 384 + 8 * bu);
-                const int sb = b[576 + bu];
+                const uint2 v = *(const uint2 *)(b + 512 + 8 * bu);
+                const int sb = b[768 + bu];
 #pragma unroll
                 for (int r = 0; r < 2; ++r)
                     acc[r][n] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(
@@ -247,7 +269,7 @@ __device__ __forceinline__ void rw_pass(const K3kRows &g, const K3ExpertQ &q, in
             k3v4f t = acc[r][n];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                float x = e < RW_NP ? t[i] : 0.0f;
+                float x = t[i];
                 x += __shfl_xor(x, 4, K3G_WAVE);
                 x += __shfl_xor(x, 2, K3G_WAVE);
                 x += __shfl_xor(x, 1, K3G_WAVE);
@@ -260,7 +282,7 @@ __device__ __forceinline__ void rw_pass(const K3kRows &g, const K3ExpertQ &q, in
             const float *x = g.z + (size_t)(MODE == 0 ? p / g.topk : p) * g.K;
 #pragma unroll
             for (int r = 0; r < 2; ++r)
-                if (v[r] != v[r]) {
+                if (!(fabsf(v[r]) < __builtin_inff())) {
                     const int i = 16 * r + 4 * q4 + e;
                     v[r] = rw_plain(mat(i) + (size_t)row(i) * kb, smat(i) + (size_t)row(i) * ks, x,
                                     g.K);
@@ -286,6 +308,7 @@ __global__ void __launch_bounds__(256, 2)
 k_rows(const K3kRows g)
 {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[RW_LDS];
+    static_assert(2 * RW_LDS <= 160 * 1024, "two workgroups per CU");
     if ((int)blockIdx.y >= *g.nact) return;
     const int e = gm_uniform(g.act[blockIdx.y]);
     const K3ExpertQ q = g.eq[e];

@@ -116,3 +116,18 @@ def test_grouped_h(gpu, hidden, inter, pairs, big_h, bf16):
     ctx.destroy()
     print(f"  rel-L2 {rel:.2e}", flush=True)
     assert rel <= 4e-5
+
+
+# checkpoint-layout experts: fp32's 24 bits of each value, K / 128 sums (1e-6 as for ordinary values)
+@pytest.mark.parametrize("hidden,inter,pairs", [(512, 256, 2), (544, 416, 9), (1184, 160, 6)])
+@pytest.mark.parametrize("scale,big_h", [(1000, 1), (1e5, 1), (1e9, 1), (1, 4096), (1, 2**40)])
+def test_rows(gpu, hidden, inter, pairs, scale, big_h):
+    print(f"case: expert rows {hidden} x {inter}, {pairs} pairs each, one column of 32 {scale} and one "
+          f"feature {big_h} times as large", flush=True)
+    m = _Layer(hidden, inter, 73, False, big_h)
+    x, idx = _inputs(m, pairs, scale, 1)
+    ctx = k3moe.Ctx(m.L, max_tokens=x.shape[0])
+    rel = m.error(x, idx, ctx)
+    ctx.destroy()
+    print(f"  rel-L2 {rel:.2e}", flush=True)
+    assert rel <= 1e-6

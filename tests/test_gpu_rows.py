@@ -1,4 +1,4 @@
-"""The routed experts of checkpoint-layout MXFP4 weights (six FP6 pieces on the FP4 x FP6 matrix
+"""The routed experts of checkpoint-layout MXFP4 weights (eight FP6 pieces on the FP4 x FP6 matrix
 cores) at the edges of their tiles, through k3g_expert_gemv, against the expert products in float64
 on the exactly dequantised weights."""
 import ctypes as C
@@ -11,7 +11,7 @@ import oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# Six E2M3 pieces leave at most 2^-24 of a block's largest value (1/16 each), as fp32 itself; the
+# Eight E2M3 pieces leave at most 2^-32 of a block's largest value (1/16 each); the
 # products accumulate in fp32, K / 128 sums a column: 6e-8 sqrt(K / 128) of the largest partial
 # sum, below 3e-7 of the result at K <= 1200, over gate, up and down.
 REL = 1e-6
