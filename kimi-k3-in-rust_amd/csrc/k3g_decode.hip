@@ -144,8 +144,11 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.KSD = SI > 0 ? (ksd < g.nCsi ? ksd : g.nCsi) : 0;
     g.nRc = (d + 1023) / 1024;
     g.KSR = ksr < g.nRc ? ksr : g.nRc;
-    /* one token's down tickets, unsliced, would leave half the waves without one */
-    g.KSDN = T > 1 ? 1 : ksdn < g.nQi ? ksdn : g.nQi;
+    /* a routed down ticket takes the whole width where that leaves at least half of the 4096 waves
+     * one (K2 and K3 from 2 tokens on, where unsliced is faster, K3_STRIPES); one token's, and few
+     * tokens' of a small layer, are sliced: 2048 x 1408, top 6, at 2 / 3 / 4 tokens unsliced 44.0 /
+     * 55.2 / 65.9 us, sliced 43.1 / 53.0 / 64.1 */
+    g.KSDN = T > 1 && T * k * (g.Dout / 32) >= 2048 ? 1 : ksdn < g.nQi ? ksdn : g.nQi;
     g.KSLD = g.lat ? (K3G_KS_LD < g.nCd ? K3G_KS_LD : g.nCd) : 0;
     g.KSLU = g.lat ? (K3G_KS_LU < g.nCL ? K3G_KS_LU : g.nCL) : 0;
     g.nSGt = (SI + 16 * SG_TILES - 1) / (16 * SG_TILES);

@@ -8,7 +8,8 @@ import k3moe
 pytestmark = pytest.mark.gpu
 
 
-# one round of tickets and many, widths ragged in the 512-column quads and 1024-column chunks
+# one round of tickets and many, widths ragged in the 512-column quads and 1024-column chunks; the
+# last one's routed down tickets are sliced at 2 tokens (1536 of them whole) and whole at 3 (2304)
 @pytest.mark.parametrize("hidden,inter,experts,topk", [(256, 64, 8, 2), (1184, 544, 48, 6),
                                                        (3072, 1056, 96, 8)])
 def test_few_tokens_match_single_tokens(gpu, hidden, inter, experts, topk):
