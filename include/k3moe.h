@@ -412,12 +412,13 @@ void k3g_ctx_set_fp8(K3gCtx *ctx, int on);
 /* Instrumentation: with a device buffer of 3 * tickets + 5 uint64, the fused kernel writes
  * for each ticket its start, the end of its waits and its end as wall-clock stamps
  * (100 MHz counter), then the top-k ticket's stamps after its wait, after its selection
- * and inside the selection. Calls on the grouped GEMMs write 4 uint64 per workgroup of
- * the routed gate/up launch (8 * 4 ceil(tiles / 32) * ceil(inter / 128) workgroups, tiles =
- * ceil(T topk / 128) + min(n_experts, T topk); of a tile of more than 64 pairs the first
- * 64), then of every second workgroup of the routed down launch (one per 512 rows): wave 0's
- * start and end, column tile << 32 | feature tile, XCC << 32 | HW_ID. NULL turns it off.
- * No reference counterpart. */
+ * and inside the selection. Calls on the grouped GEMMs write 4 uint64 per column tile of the
+ * dispatch and feature tile of the routed gate/up (128 features; a buffer of 8 * 4
+ * ceil(tiles / 32) * ceil(inter / 128) records, tiles = ceil(T topk / 128) + min(n_experts,
+ * T topk); tiles without pairs write none), then per column tile and 512 rows of the routed down:
+ * wave 0's start and end in the workgroup that took it (of a tile of more than 64 pairs the one of
+ * the first 64; of two feature tiles taken together both records alike), column tile << 32 |
+ * feature tile, XCC << 32 | HW_ID. NULL turns it off. No reference counterpart. */
 void k3g_ctx_set_trace(K3gCtx *ctx, void *dev_buf);
 
 /* Force the router's exact re-routing path (testing only): 0 normal, 1 every token

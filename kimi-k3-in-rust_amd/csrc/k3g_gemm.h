@@ -116,26 +116,32 @@ __device__ __forceinline__ int gm_item_of(int rnd, int xcd, int n, bool single)
 /* a compile-time integer as an argument */
 template <int N> struct GmInt { static constexpr int value = N; };
 
-/* Instrumentation: one record of a workgroup's start and end, at the place of its column tile and
- * feature tile in a launch of one item per column tile (the second half of a tile that is two
- * items has none, nor do tiles from `limit` on) and one record for every step-th of the nft feature
- * tiles. */
-__device__ __forceinline__ void gm_trace(unsigned long long *trace, int nft, int step, int halves,
-                                         int n, bool single, int limit, unsigned long long t_start)
+/* Instrumentation: a workgroup's start and end as the records of its column tile and its `tall`
+ * feature tiles of the nft, at their places in a launch of one item per column tile and one feature
+ * tile per workgroup (the second half of a tile that is two items has none, nor do tiles from
+ * `limit` on); every step-th feature tile has one. */
+__device__ __forceinline__ void gm_trace(unsigned long long *trace, int nft, int step, int tall,
+                                         int halves, int n, bool single, int limit,
+                                         unsigned long long t_start)
 {
     const int slot = blockIdx.x >> 3;
-    const int rnd = slot / nft, ft = slot - rnd * nft, nf = (nft + step - 1) / step;
+    const int rnd = slot / nft, f0 = tall * (slot - rnd * nft), nf = (nft + step - 1) / step;
     const int item = gm_item_of(rnd, blockIdx.x & 7, n, single), tile = item >> halves;
-    if (ft % step || (item & halves) || tile >= limit) return;
+    if ((item & halves) || tile >= limit) return;
     const int grp = tile / K3G_TILE_GROUP, q = grp >> 3;
     const int xcd = (q & 1) ? 7 - (grp & 7) : grp & 7;
-    const size_t r = (size_t)(K3G_TILE_GROUP * q + tile % K3G_TILE_GROUP) * nf + ft / step;
-    unsigned long long *o = trace + 4 * (8 * r + xcd);
-    o[0] = t_start;
-    o[1] = wall_clock64();
-    o[2] = (unsigned long long)tile << 32 | (unsigned)(ft / step);
-    o[3] = (unsigned long long)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15) << 32 |
-           (unsigned)__builtin_amdgcn_s_getreg((31 << 11) | 4);
+    const size_t r = (size_t)(K3G_TILE_GROUP * q + tile % K3G_TILE_GROUP) * nf;
+    const unsigned long long t_end = wall_clock64();
+    const unsigned long long id = (unsigned long long)(__builtin_amdgcn_s_getreg((3 << 11) | 20) & 15) << 32 |
+                                  (unsigned)__builtin_amdgcn_s_getreg((31 << 11) | 4);
+    for (int f = f0; f < min(f0 + tall, nft); ++f) {
+        if (f % step) continue;
+        unsigned long long *o = trace + 4 * (8 * (r + f / step) + xcd);
+        o[0] = t_start;
+        o[1] = t_end;
+        o[2] = (unsigned long long)tile << 32 | (unsigned)(f / step);
+        o[3] = id;
+    }
 }
 
 typedef float gm_v16f __attribute__((ext_vector_type(16)));

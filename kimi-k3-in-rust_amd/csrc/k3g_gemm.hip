@@ -560,6 +560,7 @@ k_gemm6(const K3kGemm6 g)
     static_assert(G6_LDS == 4 * GM_HLDS && G6_LDS >= 2 * GM_PIECE, "LDS");
     const unsigned long long t_start = g.trace ? wall_clock64() : 0;
     const bool bf16 = MODE == 0 && g.xb && !*g.lo_flag;
+    int tall = 1;                        /* feature tiles of this workgroup */
     if (bf16) {
         K3kGemm b = {};
         b.rows = g.rows;
@@ -582,7 +583,9 @@ k_gemm6(const K3kGemm6 g)
         if (!gm_block<0, 4>(b, lds, 1)) return;
     } else {
         G6Tile t;
-        switch (g6_setup<MODE>(g, t, lds)) {
+        const int form = g6_setup<MODE>(g, t, lds);
+        tall = (form >> 4 & 15) == 8 ? 2 : 1;
+        switch (form) {
             case 16 * 8 + 3: g6_run<MODE, 3, 8>(g, t); break;
             case 16 * 8 + 4: g6_run<MODE, 4, 8>(g, t); break;
             case 16 * 4 + 1: g6_run<MODE, 1, 4>(g, t); break;
@@ -596,9 +599,9 @@ k_gemm6(const K3kGemm6 g)
             default: return;
         }
     }
-    if (g.trace && threadIdx.x == 0) gm_trace(g.trace, g.nft, g.trace_step,
-                                                  bf16 ? 0 : g.halves, *g.ntiles, !g.halves,
-                                                  g.trace_tiles, t_start);
+    if (g.trace && threadIdx.x == 0)
+        gm_trace(g.trace, g.nft, g.trace_step, tall, bf16 ? 0 : g.halves, *g.ntiles, !g.halves,
+                 g.trace_tiles, t_start);
 }
 
 /* ============================================================ FP4 x FP8 variant ==== */

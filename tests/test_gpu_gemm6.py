@@ -1,6 +1,8 @@
 """The routed experts' grouped GEMMs (FP6 pieces on the FP4 x FP6 matrix cores; bf16 gate/up where
 every x is a bf16 value) at the edges of their tiles, through k3g_grouped_gemm_bf16, against the
 expert products in float64 on the exactly dequantised weights."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -16,21 +18,22 @@ pytestmark = pytest.mark.gpu
 REL = 1e-5
 
 
-def _dequant(layer):
+def _expert(layer, e):
+    """One expert's w1, w3, w2 as float64."""
     s, g = layer.shape, layer.geo
     d, i = s.hidden, s.inter
-    out = []
-    for e in range(s.n_experts):
-        run = layer.expert_host(e)
-        m = [O.oracle().dequant(run[po:po + r * c // 2], run[so:so + r * (c // 32)], r, c // 2)
-             .reshape(r, c).astype(np.float64)
-             for po, so, r, c in ((g.p1_off, g.s1_off, i, d), (g.p3_off, g.s3_off, i, d),
-                                  (g.p2_off, g.s2_off, d, i))]
-        out.append(m)
-    return out
+    run = layer.expert_host(e)
+    return [O.oracle().dequant(run[po:po + r * c // 2], run[so:so + r * (c // 32)], r, c // 2)
+            .reshape(r, c).astype(np.float64)
+            for po, so, r, c in ((g.p1_off, g.s1_off, i, d), (g.p3_off, g.s3_off, i, d),
+                                 (g.p2_off, g.s2_off, d, i))]
 
 
-def _rows(layer, x, idx, offset=0):
+def _dequant(layer):
+    return [_expert(layer, e) for e in range(layer.shape.n_experts)]
+
+
+def _rows(layer, x, idx, offset=0, trace=None):
     """contrib [T][k][d] (NaN where the call leaves a row alone); x at offset floats."""
     T, k = idx.shape
     d = layer.shape.hidden
@@ -40,6 +43,8 @@ def _rows(layer, x, idx, offset=0):
     dx.upload(x.astype(np.float32), 4 * offset)
     didx = k3moe.DevBuf.from_array(idx.astype(np.int32))
     dc = k3moe.DevBuf.from_array(np.full(T * k * d, np.nan, np.float32))
+    if trace is not None:
+        k3moe.lib().k3g_ctx_set_trace(ctx.ptr, C.c_void_p(trace.ptr))
     ctx.experts("bf16", L, dx.ptr + 4 * offset, T, didx.ptr, dc.ptr)
     ctx.sync()
     out = dc.download(np.float32, T * k * d).reshape(T, k, d)
@@ -87,18 +92,31 @@ def test_tile_edges(gpu, hidden, inter, bf16):
 
 
 def test_many_tiles_take_the_tall_workgroups(gpu):
-    """Enough column tiles for the 512-row workgroups, 3 and 4 column blocks, ragged rows."""
-    print("case: grouped experts, 300 experts x 40 and 60 pairs, hidden 1760 inter 352", flush=True)
-    shape = k3moe.Shape("tall", 1760, 300, 1, 352, n_shared=0, x_bf16=False, scale_lo=-8, scale_hi=-6)
+    """Enough column tiles for the 512-row workgroups of gate/up and of down, 3 and 4 column blocks,
+    an odd number of feature tiles, the last one ragged; and the workgroups' records: one of every
+    column tile and feature tile (128 features of gate/up, 512 rows of down)."""
+    E, hidden, inter = 300, 1760, 864
+    print(f"case: grouped experts, {E} experts x 40 and 60 pairs, hidden {hidden} inter {inter}", flush=True)
+    nf, nr = -(-inter // 128), -(-hidden // 256)
+    assert nf % 2 and nr % 2 and E * ((nf + 1) // 2) >= 1024 and E * ((nr + 1) // 2) >= 1024
+    shape = k3moe.Shape("tall", hidden, E, 1, inter, n_shared=0, x_bf16=False, scale_lo=-8, scale_hi=-6)
     layer = k3moe.SynthLayer(shape, seed=32, layout="both")
     idx = np.random.default_rng(2).permutation(
-        np.concatenate([np.full(40 + 20 * (e % 2), e) for e in range(300)])).reshape(-1, 1)
-    x = layer.tokens(idx.shape[0])
-    got = _rows(layer, x, idx)
-    w = _dequant(layer)
-    for t in range(0, idx.shape[0], 97):
-        want = _want(w, x[t].astype(np.float64), idx[t, 0])
+        np.concatenate([np.full(40 + 20 * (e % 2), e) for e in range(E)])).reshape(-1, 1)
+    T = idx.shape[0]
+    x = layer.tokens(T)
+    places = 32 * -(-(-(-T // 128) + E) // 32)
+    n0, n1 = places * nf, places * -(-hidden // 512)
+    trace = k3moe.DevBuf.from_array(np.zeros(4 * (n0 + n1), np.uint64))
+    got = _rows(layer, x, idx, trace=trace)
+    for t in range(0, T, 97):
+        want = _want({idx[t, 0]: _expert(layer, idx[t, 0])}, x[t].astype(np.float64), idx[t, 0])
         assert np.linalg.norm(got[t, 0] - want) <= REL * np.linalg.norm(want)
+    rec = trace.download(np.uint64, 4 * (n0 + n1)).reshape(-1, 4)
+    for part, n in ((rec[:n0], nf), (rec[n0:], -(-hidden // 512))):
+        part = part[part[:, 1] != 0]
+        assert (part[:, 0] != 0).all() and (part[:, 0] <= part[:, 1]).all()
+        assert sorted(part[:, 2].tolist()) == [t << 32 | f for t in range(E) for f in range(n)]
 
 
 def test_not_finite_and_unaligned_x(gpu):
