@@ -638,7 +638,6 @@ static int routed_f8(K3gCtx *c, const K3gLayer *L, int T, int lat, int max_tiles
     g.hs = NULL;
     g.out = contrib;
     g.ldo = lat;
-    g.scatter = 1;
     g.nft = (lat + 511) / 512;
     k3g_stage_begin(c, K3G_ST_DOWN, st);
     rc |= k3k_gemm_f8(&g, st);

@@ -49,18 +49,6 @@ __device__ __forceinline__ void gm_dma16(const void *src, uint32_t lds)
                  : "=&s"(keep) : "v"(src), "s"(lds) : "memory");
 }
 
-/* The same DMA with a wave-uniform base in scalar registers and this lane's 32-bit byte
- * offset in one vector register: no per-lane 64-bit address to build or keep. */
-__device__ __forceinline__ void gm_dma16s(const void *sbase, uint32_t voff, uint32_t lds)
-{
-    uint32_t keep;
-    asm volatile("s_mov_b32 %0, m0\n\t"
-                 "s_mov_b32 m0, %3\n\ts_nop 0\n\t"
-                 "global_load_lds_dwordx4 %1, %2\n\t"
-                 "s_mov_b32 m0, %0"
-                 : "=&s"(keep) : "v"(voff), "s"(sbase), "s"(lds) : "memory");
-}
-
 /* 64 lanes x 4 bytes, lane l at lds + 4 l */
 __device__ __forceinline__ void gm_dma4(const void *src, uint32_t lds)
 {

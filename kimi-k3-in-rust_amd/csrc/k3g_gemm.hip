@@ -178,7 +178,6 @@ struct GmTile {
     uint32_t boff[8];          /* element offsets of this lane's DMA rows (+ swizzled slot) */
     uint32_t lds;              /* LDS byte address of the staging buffers */
     uint8_t *ldsp;
-    uint32_t rbb;              /* bytes of one 16-row block of the weight matrix */
 };
 
 /* The tile's GEMM with NB 16-column blocks and NP activation pieces in a workgroup of WV
@@ -376,8 +375,7 @@ __device__ __forceinline__ void gm_tile(const K3kGemm &g, const GmTile &t)
         for (int cb = 0; cb < NB; ++cb) {
             const int col = 16 * cb + col0;
             if (col < t.np) {
-                const int p = t.p0 + col;
-                float *o = g.out + (size_t)(g.scatter ? g.perm[p] : p) * g.ldo + t.orow0 + 4 * t.g4;
+                float *o = g.out + (size_t)(t.p0 + col) * g.ldo + t.orow0 + 4 * t.g4;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     if (t.rv[r]) *(k3v4f *)(o + 16 * r) = acc[r][cb];
@@ -401,9 +399,9 @@ __device__ __forceinline__ bool gm_setup(const K3kGemm &g, GmTile &t, uint8_t *l
     /* dense GEMMs cut into K slices take (column tile, slice) pairs as their tiles; with
      * halves, every column tile is two work items of up to 64 columns, dealt one after
      * the other to the same XCD */
-    const int ks_n = g.tiles ? 1 : max(1, g.ksplit);
-    const int ntl = (g.tiles ? *g.ntiles : (g.dense_rows + GM_COLS - 1) / GM_COLS) * ks_n *
-                    (halves ? 2 : 1);
+    const int ks_n = AF == 0 ? 1 : max(1, g.ksplit);
+    const int ntl = AF == 0 ? *g.ntiles * (halves ? 2 : 1)
+                            : (g.dense_rows + GM_COLS - 1) / GM_COLS * ks_n;
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     int f, tks;
     if (AF == 0) {
@@ -426,7 +424,7 @@ __device__ __forceinline__ bool gm_setup(const K3kGemm &g, GmTile &t, uint8_t *l
     const int tile = tks / ks_n;
     t.ks = tks - tile * ks_n;
     int e = 0;
-    if (g.tiles) {
+    if (AF == 0) {
         const int4 tv = ((const int4 *)g.tiles)[tile];
         e = gm_uniform(tv.x); t.p0 = gm_uniform(tv.y); t.np = gm_uniform(tv.z);
     } else {
@@ -461,7 +459,6 @@ __device__ __forceinline__ bool gm_setup(const K3kGemm &g, GmTile &t, uint8_t *l
     }
     /* bytes per 16-row block */
     const size_t rbb = AF == 0 ? (size_t)((g.K + 511) / 512) * GM_QT : (size_t)(g.K / 32) * 1024;
-    t.rbb = (uint32_t)rbb;
     if (g.mode == 0) {
         t.orow0 = 32 * WV * f + 32 * t.w;
 #pragma unroll
@@ -725,8 +722,7 @@ __device__ __forceinline__ void gm_tile_f8(const K3kGemm &g, const GmTile &t,
         for (int cb = 0; cb < NB; ++cb) {
             const int col = 16 * cb + c0;
             if (col < t.np) {
-                const int p = t.p0 + col;
-                float *o = g.out + (size_t)(g.scatter ? g.perm[p] : p) * g.ldo + t.orow0 + 4 * t.g4;
+                float *o = g.out + (size_t)g.perm[t.p0 + col] * g.ldo + t.orow0 + 4 * t.g4;
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     if (t.rv[r]) *(k3v4f *)(o + 16 * r) = acc[r][cb];
@@ -949,10 +945,8 @@ extern "C" int k3k_gemm_f8(const K3kGemm *g, hipStream_t st)
     if (g->mode == 1 && (g->rows % 16 || g->nft * 512 < g->rows || !g->out || g->ldo < g->rows ||
                          g->ldo % 4))
         return -1;
-    if (g->tiles ? (!g->ntiles || g->max_tiles < 1) : g->dense_rows < 1) return -1;
-    if ((g->scatter || (g->mode == 0 && g->tiles)) && !g->perm) return -1;
-    const long long maxt = g->tiles ? g->max_tiles : (g->dense_rows + GM_COLS - 1) / GM_COLS;
-    const long long grid = 8 * (long long)K3G_TILE_ROUNDS(2 * maxt) * g->nft;   /* halves */
+    if (!g->tiles || !g->ntiles || g->max_tiles < 1 || !g->perm) return -1;
+    const long long grid = 8 * (long long)K3G_TILE_ROUNDS(2LL * g->max_tiles) * g->nft;   /* halves */
     if (grid > 0x7fffffff) return -1;
     hipLaunchKernelGGL(k_gemm_f8, dim3((unsigned)grid), dim3(GM_WAVES * 64), 0, st, *g);
     return hipGetLastError() == hipSuccess ? 0 : -1;
@@ -971,8 +965,7 @@ extern "C" int k3k_gemm(const K3kGemm *g, hipStream_t st)
     if (g->mode == 1 && (g->rows % 16 || g->nft * 512 < g->rows || !g->out || g->ldo < g->rows ||
                          g->ldo % 4))
         return -1;
-    if (!g->wa || (g->mode == 0 && !g->wb) || g->tiles || g->scatter || g->dense_rows < 1)
-        return -1;
+    if (!g->wa || (g->mode == 0 && !g->wb) || g->tiles || g->dense_rows < 1) return -1;
     const int ks_n = g->ksplit > 1 ? g->ksplit : 1;
     if (ks_n > 1 && (!g->part || g->K % GM_KC ||
                      ks_n > g->K / GM_KC || (g->mode == 0 && g->rows % 4)))

@@ -114,8 +114,9 @@ typedef struct {
 #define K3K_HFLAG_DONE 16     /* a separate 64-byte line */
 #define K3K_HFLAG_INTS 32
 
-/* One grouped GEMM on the bf16 matrix cores (k3g_gemm.hip). Columns are (token, slot)
- * pairs grouped by expert (tiles) or all tokens (dense, the shared expert). */
+/* One GEMM of k3g_gemm.hip: dense on the bf16 matrix cores (tiled bf16 weights, all tokens are
+ * columns: shared expert, latent projections), or tiled MXFP4 experts whose columns are (token,
+ * slot) pairs grouped by expert (tiles): FP4 x FP8, or gate/up of bf16-valued x in k_gemm6. */
 typedef struct {
     int mode;                 /* 0: gate/up + activation -> h pieces; 1: down -> fp32 rows */
     int rows;                 /* output rows of one weight matrix: inter (mode 0), hidden (1) */
@@ -137,9 +138,8 @@ typedef struct {
     long long hpiece;
     int ldh;
     float b1, b2;             /* activation caps */
-    float *out;               /* mode 1 out: row per column, stride ldo */
+    float *out;               /* mode 1 out, stride ldo: row column (dense) or perm[column] */
     int ldo;
-    int scatter;              /* mode 1: out row = perm[column] (else the column) */
     int single;               /* tiles of up to 64 pairs, as a rule one an expert (gm_item_of) */
     int nft;                  /* feature tiles: ceil(rows / 256) (mode 0), / 512 (mode 1) */
     /* MXFP8 activations (k3k_gemm_f8, MXFP4 weights only): E4M3 bytes [rows][ldb] and
@@ -147,7 +147,7 @@ typedef struct {
     const uint8_t *bq, *bs;
     uint8_t *hq, *hs;
     int ldhq;                 /* bytes per h row (scales: ldhq / 32) */
-    uint8_t *h6;              /* k3k_gemm with MXFP4 weights: h as FP6 quads (K3kGemm6) */
+    uint8_t *h6;              /* bf16-valued x in k_gemm6: h as FP6 quads (K3kGemm6) */
     size_t hmore;
     uint8_t *hrow;
     int32_t *hwide;
