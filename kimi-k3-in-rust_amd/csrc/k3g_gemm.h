@@ -197,36 +197,48 @@ __device__ __forceinline__ bool gm_bad(const gm_v16f &ev, const gm_v16f &od)
     return bad;
 }
 
-/* How far a block's values lie below its largest: the sum over its 32 values (zeros left out) of
- * the square of the binary orders between, each at most 16. Normally distributed values 243, one
- * block in 100,000 above 790; silu(g) u of such g and u 674, one in 100,000 above 1994; normal
- * values beside one 16 to 31 times as large 992 in the mean, beside one 256 times as large 2790. */
-__device__ __forceinline__ int gm_spread(const gm_v16f &ev, const gm_v16f &od)
+/* Blocks that take eight pieces. Four leave 3e-7 of the block's largest value on every one of its
+ * values; four more 2e-14 beside a value 16 times as large, 1.6e-11 beside 1000, 1.6e-8 beside
+ * 10^6. The rules count the values of 1/8, 1/32 and 1/128 of the largest or more.
+ *
+ * x had been two bf16 pieces, 2.5e-6 of each value: less than four FP6 pieces leave below an eighth
+ * of the largest. Eight where a few values (one and an eighth of those that are not zero) are that
+ * large, or half are 1/32 or three quarters 1/128. What is left then of normally distributed values
+ * beside 1, 4, 8 or 16 that are 16 times as large is 1.5e-6, 1.5e-6, 5e-6 and 9e-6 of them, beside
+ * 100 times as large 7e-7, 6e-8, 0 and 0; and no block of 800,000 normally distributed ones takes
+ * eight. (By the sum of the squared orders below the largest, which leaves more beside
+ * outliers, 4 in a million did, so one in a dozen of full tiles: gate/up of 4,096 fp32 tokens 2.41
+ * ms; four pieces everywhere 2.32, these rules within 1 % of that.)
+ *
+ * h had been a bf16 piece with an MXFP8 remainder, 3.9e-5 of each value: less than four FP6 pieces
+ * leave below 1/130 of the largest. Where gates are large, half of the values of every block lie that
+ * far below the other half (silu of a negative gate), and the block's products are those of the
+ * larger half: eight only where few values are that large. (With the half as well, the down product
+ * of 4,096 tokens of such a layer took nearly every step twice, 1.58 against 1.33 ms.) */
+template <bool X>
+__device__ __forceinline__ bool gm_eight(const gm_v16f &ev, const gm_v16f &od)
 {
     float m = 0.0f;
 #pragma unroll
     for (int i = 0; i < 16; ++i) m = fmaxf(m, fmaxf(fabsf(ev[i]), fabsf(od[i])));
-    const int top = (int)(__float_as_uint(m) >> 23);
-    int sum = 0;
-    auto add = [&](float v) {
-        const int n = min(top - (int)(__float_as_uint(v) << 1 >> 24), 16);
-        sum += v == 0.0f ? 0 : n * n;
+    int n = 0, c3 = 0, c5 = 0, c7 = 0;
+    auto count = [&](float v) {
+        v = fabsf(v);
+        n += v != 0.0f;
+        if (X) {
+            c3 += v >= m * 0x1p-3f;
+            c5 += v >= m * 0x1p-5f;
+        }
+        c7 += v >= m * 0x1p-7f;
     };
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-        add(ev[i]);
-        add(od[i]);
+        count(ev[i]);
+        count(od[i]);
     }
-    return sum;
+    const int few = X ? c3 : c7;
+    return (few <= 1 + n / 8 && few < n) || (X && (2 * c5 <= n || 4 * c7 <= 3 * n));
 }
-
-/* Spreads from which on a block takes eight pieces. Four leave 3e-7 of the block's largest value
- * on every one of its values: less than the two bf16 pieces that x had been (2.5e-6 of each
- * value) down to an eighth of it, and less than the bf16 piece with its MXFP8 remainder that h
- * had been (3.9e-5) down to 1/130. Blocks whose values lie lower get four pieces more: 2e-14
- * beside a value 16 times as large, 1.6e-11 beside 1000, 1.6e-8 beside 10^6. */
-#define GM_WIDE_X 832
-#define GM_WIDE_H 2560
 
 /* One block's four pieces in a quad (k3g_gemm6.h): step j, block q. */
 __device__ __forceinline__ void gm_put_pieces(const uint32_t (&d)[24], uint32_t scales,
@@ -247,15 +259,16 @@ __device__ __forceinline__ uint32_t gm_bytes(const uint8_t (&s)[4])
     return s[0] | (uint32_t)s[1] << 8 | (uint32_t)s[2] << 16 | (uint32_t)s[3] << 24;
 }
 
-/* One block of 32 values into its place in a quad, and where its spread is `at` or more (true) the
- * next four pieces into the same place `more` bytes on; elsewhere that place gets scales of zero.
- * A block with an infinity or NaN gets the NaN scale, so the products are NaN as they were. */
+/* One block of 32 values into its place in a quad and, for a block of eight pieces (true if it is
+ * stored as one), the next four into the same place `more` bytes on; elsewhere that place gets
+ * scales of zero. A block with an infinity or NaN gets the NaN scale, so the products are NaN as
+ * they were. */
 __device__ __forceinline__ bool gm_store_block(gm_v16f ev, gm_v16f od, uint8_t *quad, size_t more,
-                                               int at, int j, int q)
+                                               bool eight, int j, int q)
 {
     uint32_t d[24];
     uint8_t s[4];
-    const bool bad = gm_bad(ev, od), w = !bad && gm_spread(ev, od) >= at;
+    const bool bad = gm_bad(ev, od), w = !bad && eight;
     gm_pieces<4>(ev, od, d, s);
     gm_put_pieces(d, bad ? 0xffffffffu : gm_bytes(s), quad, j, q);
     if (w) {
@@ -331,7 +344,7 @@ __device__ __forceinline__ void gm_store_h(k3v4f (&acc)[RG][NBW], float *wl, int
             }
             const int f = f0 + 32 * b;
             if (gm_store_block(ev, od, h + ((size_t)(p0 + col) * nQh + (f >> 9)) * K3G_P6_QUAD, more,
-                               GM_WIDE_H, (f >> 7) & 3, (f >> 5) & 3)) {
+                               gm_eight<false>(ev, od), (f >> 7) & 3, (f >> 5) & 3)) {
                 wrow[p0 + col] = 1;
                 *wide = 1;
             }

@@ -1,5 +1,5 @@
-"""Activations with values far below their block's largest (32 columns): one value in every block is
-large and meets weights of zero, so that the products are those of the others alone. The expert
+"""Activations with values far below their block's largest (32 columns): some values of every block
+are large and meet weights of zero, so that the products are those of the others alone. The expert
 products through the device API against float64 on the exactly dequantised weights."""
 import numpy as np
 import pytest
@@ -19,10 +19,11 @@ def _zero_columns(codes, rows, cols, at):
 
 
 class _Layer:
-    """Experts whose gate and up take nothing from columns 32 b + 5 and whose down takes nothing from
-    features 32 b + 6; those features' up rows are `big_h` (a power of two) times as large."""
+    """Experts whose gate and up take nothing from columns 32 b + c, c in `big`, and whose down takes
+    nothing from features 32 b + 6; those features' up rows are `big_h` (a power of two) times as
+    large."""
 
-    def __init__(self, hidden, inter, seed, tiled, big_h=1):
+    def __init__(self, hidden, inter, seed, tiled, big_h=1, big=(5,)):
         shape = k3moe.Shape("outlier", hidden, E, 2, inter, n_shared=0, x_bf16=False, scale_lo=-8,
                             scale_hi=-6)
         self.synth = k3moe.SynthLayer(shape, seed=seed, layout="tiled" if tiled else "engine")
@@ -34,12 +35,13 @@ class _Layer:
                                   (3, g.p3_off, g.s3_off, inter, hidden),
                                   (2, g.p2_off, g.s2_off, hidden, inter)):
                 codes, scales = run[p:p + r * c // 2].copy(), run[s:s + r * (c // 32)].copy()
-                _zero_columns(codes, r, c, 6 if m == 2 else 5)
+                for at in (6,) if m == 2 else big:
+                    _zero_columns(codes, r, c, at)
                 if m == 3:
                     scales.reshape(r, c // 32)[6::32] += int(np.log2(big_h))
                 w.append(O.oracle().dequant(codes, scales, r, c // 2).reshape(r, c)
                          .astype(np.float64))
-                assert not w[-1][:, (6 if m == 2 else 5)::32].any()
+                assert not any(w[-1][:, at::32].any() for at in ((6,) if m == 2 else big))
                 if tiled:
                     codes, scales = k3moe.tile_mxfp4_host(codes, scales, r, c), None
                 for v in (codes, scales):
@@ -51,7 +53,7 @@ class _Layer:
         self.table = k3moe.DevBuf.from_array(np.frombuffer(bytes(tab), np.uint8))
         self.L = self.synth.dev
         self.L.experts = self.table.ptr
-        self.kind = "bf16" if tiled else "gemv"
+        self.kind, self.big = "bf16" if tiled else "gemv", big
 
     def want(self, x, e):
         g, u = self.w[e][0] @ x, self.w[e][1] @ x
@@ -78,26 +80,45 @@ def _inputs(m, pairs, scale, every, seed=3):
     T = pairs * E // 2
     idx = np.random.default_rng(seed).permutation(np.repeat(np.arange(E), pairs)[:2 * T]).reshape(T, 2)
     x = m.synth.tokens(T)
-    x[::every, 5::32] *= np.float32(scale)
+    for c in m.big:
+        x[::every, c::32] *= np.float32(scale)
     return x, idx
 
 
 # Four FP6 pieces leave 3e-7 of a block's largest value on each of its values, 8e-5 and 3e-4 of them
 # here; two bf16 pieces 2.5e-6 of each. gate, up and down together: three times that.
 @pytest.mark.parametrize("hidden,inter,pairs", _SIZES)
-@pytest.mark.parametrize("scale,every", [(256, 1), (1000, 1), (1000, 5), (1e5, 1)])
-def test_grouped_x(gpu, hidden, inter, pairs, scale, every):
+@pytest.mark.parametrize("scale,every,big", [(256, 1, 1), (1000, 1, 1), (1000, 5, 1), (1e5, 1, 1),
+                                             (300, 1, 4), (300, 1, 16), (3000, 1, 24)])
+def test_grouped_x(gpu, hidden, inter, pairs, scale, every, big):
+    big = tuple(sorted((5 + 13 * i) % 32 for i in range(big)))
     print(f"case: grouped experts {hidden} x {inter}, {pairs} pairs each, x {scale} times as large in "
-          f"one column of 32, every {every}th token", flush=True)
-    m = _Layer(hidden, inter, 71, True)
+          f"columns {big} of 32, every {every}th token", flush=True)
+    m = _Layer(hidden, inter, 71, True, big=big)
     x, idx = _inputs(m, pairs, scale, every)
     ctx = k3moe.Ctx(m.L, max_tokens=x.shape[0])
     rel = m.error(x, idx, ctx)
-    x[:, 5::32] = 0                       # ordinary blocks on the same context
+    for c in big:                         # ordinary blocks on the same context
+        x[:, c::32] = 0
     plain = m.error(x, idx, ctx)
     ctx.destroy()
     print(f"  rel-L2 {rel:.2e}, without {plain:.2e}", flush=True)
     assert rel <= 7.5e-6 and plain <= 7.5e-6
+
+
+# Where gates are large, half of h's values are next to nothing: four pieces, for the products are
+# those of the others (as for ordinary h).
+@pytest.mark.parametrize("hidden,inter,pairs", _SIZES)
+def test_grouped_h_of_large_gates(gpu, hidden, inter, pairs):
+    print(f"case: grouped experts {hidden} x {inter}, {pairs} pairs each, x 64 times as large", flush=True)
+    m = _Layer(hidden, inter, 74, True)
+    x, idx = _inputs(m, pairs, 1, 1)
+    x *= np.float32(64)
+    ctx = k3moe.Ctx(m.L, max_tokens=x.shape[0])
+    rel = m.error(x, idx, ctx)
+    ctx.destroy()
+    print(f"  rel-L2 {rel:.2e}", flush=True)
+    assert rel <= 1e-5
 
 
 # h had been a bf16 piece and an MXFP8 remainder: 4e-5 of each value
