@@ -17,9 +17,10 @@ import oracle as O
 pytestmark = pytest.mark.gpu
 GOLDEN = os.path.join(os.path.dirname(os.path.abspath(__file__)), "golden")
 REL_L2 = 1e-3
-# the grouped bf16 GEMMs: x and the weights exact in bf16, h as bf16 plus its MXFP8
-# remainder (about 12 significant bits), fp32 accumulation: rel-L2 about 4e-5
-GEMM_REL = 1e-4
+# The grouped GEMMs: weights exact, x exact in bf16 or four FP6 (E2M3) pieces, h four FP6 pieces.
+# Each piece leaves 1/32 of its block's largest value in the mean: 2^-20 after four, over gate, up
+# and down 3e-6; fp32 accumulation below 1e-6 (measured 3e-7 .. 1.5e-6).
+GEMM_REL = 1e-5
 
 
 def rel_l2(a, b):
@@ -481,7 +482,7 @@ def test_layer_k2_fused_consecutive_tokens(k2_layer):
                                      (37, "bf16"), (200, "bf16")])
 def test_layer_tiny_grouped_gemm(gpu, T, xkind):
     say(f"case: k3g_moe tiny layer on the grouped bf16 MFMA GEMMs, {T} tokens, x {xkind} "
-        "(fp32: two activation pieces on 8-wave workgroups; bf16: one piece, 4-wave)")
+        "(fp32: four FP6 activation pieces; bf16: one exact bf16 piece)")
     layer = k3moe.SynthLayer(k3moe.TINY, seed=4321, layout="both")
     x = layer.tokens(T)
     if xkind == "bf16":
@@ -690,17 +691,25 @@ def _run_experts(layer, kind, x, idx):
     return dc.download(np.float32, T * k * d).reshape(T, k, d)
 
 
-def test_grouped_remainder_extremes(gpu):
-    """h's MXFP8 remainder at its edges: tokens of zeros (every remainder block zero, scale
-    byte 0) give rows of exact zeros; tokens scaled by 2^-20 and 2^12 (remainder blocks far
-    from 1, activation caps reached) stay within the grouped tolerance of the oracle."""
-    T = 24
-    say(f"case: grouped bf16 experts, tiny layer, {T} tokens: zero rows, tiny and large rows")
+@pytest.mark.parametrize("xkind", ["bf16", "fp32"])
+def test_grouped_piece_extremes(gpu, xkind):
+    """The FP6 pieces of x (fp32 values) and h at the edges of their block scales: tokens of zeros
+    (every block zero) give rows of exact zeros; tokens scaled by 2^-20, 2^-35 and 2^12 (blocks
+    far from 1, activation caps reached) stay within the grouped tolerance of the oracle; and
+    tokens scaled by 2^-75, whose h is at most the smallest numbers there are and whose pieces meet
+    the smallest scale, give rows next to zero."""
+    T = 30
+    say(f"case: grouped experts, tiny layer, {T} tokens, x {xkind}: zero rows, tiny and large rows")
     layer = k3moe.SynthLayer(k3moe.TINY, seed=4242, layout="both")
     x = layer.tokens(T).copy()
+    if xkind == "fp32":
+        x = (x * np.float32(1.0 + 2.0 ** -12)).astype(np.float32)
+        assert np.any(x.view(np.uint32) & 0xFFFF)
     x[0:4] = 0.0
     x[4:10] *= np.float32(2.0 ** -20)
     x[10:16] *= np.float32(2.0 ** 12)
+    x[16:20] *= np.float32(2.0 ** -35)   # (the oracle's own numbers run out below 2^-40)
+    x[20:24] *= np.float32(2.0 ** -75)
     idx = _random_routing(T, layer.shape.n_experts, layer.shape.topk, seed=5, drop=0.0)
     rows = _run_experts(layer, "bf16", x, idx)
     assert np.all(rows[0:4] == 0.0), "zero tokens must give exact zeros"
@@ -708,11 +717,12 @@ def test_grouped_remainder_extremes(gpu):
     exp = _pair_rows(layer, x, idx, kept)
     got = np.stack([rows[t, j] for t, j in kept])
     assert np.all(np.isfinite(got))
-    for lo, hi in ((4, 10), (10, 16), (16, T)):
+    for lo, hi in ((4, 10), (10, 16), (16, 20), (24, T)):
         sel = [i for i, (t, _) in enumerate(kept) if lo <= t < hi]
         r = rel_l2(got[sel], exp[sel])
         say(f"  tokens {lo}..{hi - 1}: rel-L2 {r:.3e}")
         assert r <= GEMM_REL
+    assert np.abs(rows[20:24]).max() <= 2.0 ** -110
 
 
 @pytest.mark.parametrize("kind,T", [("gemv", 3), ("gemv", 37), ("bf16", 5), ("bf16", 37),
