@@ -43,15 +43,14 @@ B_GATEUP_EXPERT = 2 * (I * D // 2 + I * D // 32)   # w1 + w3 of one expert
 # --pmc runs (FETCH_SIZE x 1.9997 + WRITE_SIZE x 1.0, the factors that make a 256 MiB
 # device-to-device copy read 256 MiB); the run and the numbers are in
 # profiles/k_decode_fused_k2_decode.md. Re-measured whenever the kernel changes.
-TRAFFIC_FUSED = 302055321
-# HBM bytes per launch of the routed gate/up GEMM (k_gemm<0, 4>) of the 4096-token
-# Zipf(0.8) prefill, the same way (FETCH_SIZE x 1.9997 + WRITE_SIZE, mean of 3 launches):
-# 7.666 GB read + 0.204 GB written; profiles/k_gemm_k2_prefill4096.md.
-TRAFFIC_GATEUP_PREFILL = 7869400121
-# the same for the fp32-x sub-leg's routed gate/up (k_gemm<0, 8>: x in two bf16 pieces),
-# mean of its last 6 launches: 8.059 GB read + 0.203 GB written;
-# profiles/k_gemm_k2_prefill4096.md.
-TRAFFIC_GATEUP_PREFILL_FP32 = 8261930315
+TRAFFIC_FUSED = 302318946
+# HBM bytes per launch of the routed gate/up GEMM (k_gemm6<0>) of the 4096-token Zipf(0.8)
+# prefill, the same way (FETCH_SIZE x 1.9997 + WRITE_SIZE, mean of 4 launches): 7.672 GB read +
+# 0.223 GB written; profiles/k_gemm6_k2_k3.md.
+TRAFFIC_GATEUP_PREFILL = 7895430259
+# the same for the fp32-x sub-leg's (x in four FP6 pieces; mean of 5 launches): 10.711 GB read +
+# 0.234 GB written
+TRAFFIC_GATEUP_PREFILL_FP32 = 10944184162
 
 
 def log(msg):
@@ -268,8 +267,8 @@ def batch_decode(a):
             "hbm_frac": round(step_bytes / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4),
             "steps": a.batch_steps, "warmup": a.batch_warmup,
             "workload": "64-token batched decode, same K2 layer, Zipf(1.1) selection-bias "
-                        "skew (alpha 0.025), 2 layers round-robin; grouped bf16 MFMA GEMMs, "
-                        "h's MXFP8 remainder on scaled FP8 MFMA"}
+                        "skew (alpha 0.025), 2 layers round-robin; grouped GEMMs, routed gate/up "
+                        "on bf16 MFMA (every x a bf16 value), down on FP4 x FP6 (h in FP6 pieces)"}
 
 
 def expert_trace(n_steps, n_layers, T, seed, reuse=0.7, zipf_s=1.0, per_step=40):
@@ -513,8 +512,9 @@ def prefill(a):
     ctx.set_fp8(False)
     assert np.isfinite(dout.download(np.float32, T * D)).all()
     # the engine's real prefill input: k3_decoder_layer_inc hands k3_moe_prefill the fp32
-    # hidden state (src/core/k3_ops.c:1015-1024); the same draws, not rounded to bf16, so x
-    # takes two bf16 pieces and the router's second-piece product runs
+    # hidden state (src/core/k3_ops.c:1015-1024); the same draws, not rounded to bf16, so the
+    # routed gate/up takes x in FP6 pieces, the shared expert both bf16 pieces, and the router's
+    # second-piece product runs
     x32 = layer.tokens(T, stream_base=900, bf16=False)
     dx32 = k3moe.DevBuf.from_array(x32)
 
@@ -566,8 +566,8 @@ def prefill(a):
         "achieved_TFLOPs": round(flops / (ms * 1e-3) / 1e12, 1),
         "steps": a.prefill_steps, "warmup": a.prefill_warmup,
         "workload": "4096-token prefill, same K2 layer, Zipf(0.8) selection-bias skew "
-                    "(alpha 0.02), bf16-valued x; bf16 MFMA grouped GEMMs, h's MXFP8 "
-                    "remainder on scaled FP8 MFMA",
+                    "(alpha 0.02), bf16-valued x; grouped GEMMs, routed gate/up on bf16 MFMA "
+                    "(every x a bf16 value), down on FP4 x FP6 (h in FP6 pieces)",
         "routing": {"experts_used": int(len(act)), "max_tokens": int(cnt.max()),
                     "min_tokens": int(act.min()),
                     "p90_over_p10": round(float(np.percentile(act, 90) / max(np.percentile(act, 10), 1)), 2),
@@ -594,19 +594,19 @@ def prefill(a):
                          for s in range(len(names)) if n32_stage[s]},
             "routing_slots_same_as_bf16_x": round(same, 4),
             "what": "the same 4096 tokens as fp32 values (the engine's k3_decoder_layer_inc "
-                    "input, not rounded to bf16): x is two bf16 pieces, so the router adds "
-                    "the second piece's product and the routed and shared gate/up GEMMs "
-                    "multiply both pieces (8-wave workgroups); same layer, same Zipf(0.8) "
-                    "skew",
-            "roofline": {"kernel": "k_gemm<0, 8> routed gate/up on x's two bf16 pieces "
-                                   "(8-wave workgroups)",
+                    "input, not rounded to bf16): the routed gate/up takes x in four FP6 "
+                    "pieces on FP4 x FP6, the router adds the product of x's second bf16 "
+                    "piece and the shared gate/up multiplies both; same layer, same "
+                    "Zipf(0.8) skew",
+            "roofline": {"kernel": "k_gemm6<0> routed gate/up on FP4 x FP6 (x in four FP6 "
+                                   "pieces, SwiGLU epilogue)",
                          "bound": "mfma", "achieved": round(gu32_tf, 1),
                          "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                          "frac": round(gu32_tf / BF16_PEAK_TFLOPS, 4),
                          "traffic": TRAFFIC_GATEUP_PREFILL_FP32,
                          "flop_per_launch": gu_flops, "avg_launch_us": round(gu32_us, 1)}},
-        "roofline": {"kernel": "k_gemm<0> routed gate/up (MXFP4 dequantised to bf16 in "
-                               "registers, bf16 MFMA, SwiGLU epilogue)",
+        "roofline": {"kernel": "k_gemm6<0> routed gate/up (bf16-valued x: MXFP4 dequantised to "
+                               "bf16 in registers, bf16 MFMA, SwiGLU epilogue)",
                      "bound": "mfma", "achieved": round(gu_tf, 1), "peak": BF16_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(gu_tf / BF16_PEAK_TFLOPS, 4),
                      "traffic": TRAFFIC_GATEUP_PREFILL, "flop_per_launch": gu_flops,
