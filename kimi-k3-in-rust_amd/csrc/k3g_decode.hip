@@ -115,8 +115,8 @@ struct K3Geo {
     int lat, L, Dout, nQk;       /* L; D's output rows (L or d); G's K in 512-column quads */
     int nCL, KSLD, KSLU, nLDt, nLUt, nNR, nLD, nLU, oLD, oNR, oLU;
     /* counter lines */
-    int lR, lSD, lD, lTSG, lTG, lRE, lDT, lLD, lLU, lS, lTK, cX, cX16, cR, cSGF, cGF, cZ, cA, cN, eX,
-        eX16, eR, eSEL, eSGF, eGF, eZ, eA, eN, cOD, nlines;
+    int lTSG, lTG, lRE, lDT, lLD, lLU, lS, lTK, cX, cX16, cR, cSGF, cGF, cZ, cA, cN, eX, eX16,
+        eSEL, eSGF, eGF, eZ, eA, eN, cOD, nlines;
 };
 
 __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int SI, int L)
@@ -179,10 +179,7 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.oLU = g.oNR + g.nNR;
     g.total = g.oLU + g.nLU;
     /* counters: one 128-byte line each; events: a counter plus NREP replicated flags */
-    g.lR = 0;
-    g.lSD = g.lR + NSUB;
-    g.lD = g.lSD + NSUB;
-    g.lTSG = g.lD + g.P;
+    g.lTSG = 0;
     g.lTG = g.lTSG + g.nSGt;
     g.lRE = g.lTG + g.P * g.nGt;
     g.lDT = g.lRE + E;
@@ -201,9 +198,11 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.cGF = g.cN + 1 + NSUB;
     g.eX = g.cGF + g.P * (1 + NSUB);
     g.eX16 = g.eX + K3_EVLINES;
-    g.eR = g.eX16 + K3_EVLINES;
-    g.eSEL = g.eR + K3_EVLINES;
-    g.eSGF = g.eSEL + T * K3_EVLINES;
+    /* the tokens' selections, one event each: the copies of one lie between another's (a layer's
+     * counters at 4 tokens must not take more lines than a bank of k3g_moe_noalloc's array has) */
+    g.eSEL = g.eX16 + K3_EVLINES;
+    static_assert(REP_STRIDE >= 4, "a line for each token's selection");
+    g.eSGF = g.eSEL + K3_EVLINES;
     g.eZ = g.eSGF + K3_EVLINES;
     g.eA = g.eZ + K3_EVLINES;
     g.eN = g.eA + K3_EVLINES;
@@ -766,7 +765,8 @@ struct K3Dec {
             const float4 v = k3d_route_score(sv, bv, a.bias ? a.bias[e] : 0.0f, a.d);
             k3d_st4_sc1(rr, (lane * a.E + e) * 16, k3v4f{v.x, v.y, v.z, v.w});
         }
-        k3d_arrive_event2(a.sync, G.cR, a.E, e, G.eR, lane);
+        /* (the selections wait for the sub-counters themselves) */
+        k3d_signal(k3d_line(a.sync, G.cR + 1 + e % NSUB), lane);
     }
 
     /* ----------------------------------------------------------------- S ---- */
@@ -780,7 +780,7 @@ struct K3Dec {
             /* the routing came with the call: publish it once x's pieces exist */
             if (tk) return;
             if (!k3d_wait_event(a.sync, G.eX, 0, a.spin_limit, a.err, lane)) return;
-            for (int i = 0; i < a.T; ++i) k3d_set_event(a.sync, G.eSEL + i * K3_EVLINES, lane);
+            for (int i = 0; i < a.T; ++i) k3d_set_event(a.sync, G.eSEL + i, lane);
             host_routing(a, lane);
             return;
         }
@@ -800,7 +800,7 @@ struct K3Dec {
                          a.renorm, a.routed_scale, a.idx, a.wt, a.force, a.stats, lane,
                          a.trace && t == 0 ? a.trace + 3 * G.total + 2 : nullptr);
         if (a.trace && t == 0 && lane == 0) a.trace[3 * G.total + 1] = wall_clock64();
-        k3d_set_event(a.sync, G.eSEL + t * K3_EVLINES, lane);
+        k3d_set_event(a.sync, G.eSEL + t, lane);
         __builtin_amdgcn_s_setprio(0);
         /* the host's copies, once every token's routing is in */
         if (a.hidx && (a.T == 1 || k3d_arrive(k3d_line(a.sync, G.lS), a.T - 1, lane)))
@@ -977,7 +977,7 @@ struct K3Dec {
         const int gt = rem / G.KSG, ks = rem - gt * G.KSG;
         const int q0 = ks * G.nQk / G.KSG, q1 = (ks + 1) * G.nQk / G.KSG;
         const int t = p / a.k;
-        if (!k3d_wait_event(a.sync, G.eSEL + t * K3_EVLINES, tk, a.spin_limit, a.err, lane)) return next;
+        if (!k3d_wait_event(a.sync, G.eSEL + t, tk, a.spin_limit, a.err, lane)) return next;
         /* the latent layer's routed input is z = down x */
         if (G.lat && !k3d_wait_event(a.sync, G.eZ, tk, a.spin_limit, a.err, lane)) return next;
         k3d_trace_go(a.trace, G.oG + tk, lane);
@@ -1142,8 +1142,7 @@ struct K3Dec {
         const int p = tk / per, rem = tk - p * per;
         const int dt = rem / G.KSDN, ks = rem - dt * G.KSDN;
         const int q0 = ks * G.nQi / G.KSDN, q1 = (ks + 1) * G.nQi / G.KSDN;
-        if (!k3d_wait_event(a.sync, G.eSEL + p / a.k * K3_EVLINES, tk, a.spin_limit, a.err, lane))
-            return next;
+        if (!k3d_wait_event(a.sync, G.eSEL + p / a.k, tk, a.spin_limit, a.err, lane)) return next;
         const int e = k3d_uniform(__hip_atomic_load(&a.idx[p], __ATOMIC_RELAXED,
                                                     __HIP_MEMORY_SCOPE_AGENT));
         k3v4f y0 = {0, 0, 0, 0}, y1 = {0, 0, 0, 0};

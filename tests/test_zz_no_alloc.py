@@ -1,8 +1,8 @@
 """k3g_moe_noalloc (the decode layer with every buffer in a fixed device array, for callers
 that cannot allocate) against k3g_moe on a context (the existing entry point, same fused
 kernel): outputs, routing indices and weights bit-identical, on two calls in a row, the
-second with fewer tokens, on the tiny layer and on the Kimi-K2 layer, and a shape that
-exceeds the array rejected with -1. Called through the C ABI."""
+second with fewer tokens, on the tiny layer and on the Kimi-K2 layer and on one whose counters
+nearly fill a bank, and a shape that exceeds the array rejected with -1. Called through the C ABI."""
 import ctypes as C
 
 import numpy as np
@@ -49,9 +49,14 @@ def _ctx(L, x):
     return res
 
 
-@pytest.mark.parametrize("shape", ["tiny", "k2"])
+# a counter line for each of the 32 pairs' 150 routed gate/up tiles and 3273 others, of a bank's 8192
+_SHAPES = {"tiny": k3moe.TINY, "k2": k3moe.K2,
+           "counters": k3moe.Shape("counters", 512, 16, 8, 4800, n_shared=0, scale_lo=-8, scale_hi=-6)}
+
+
+@pytest.mark.parametrize("shape", list(_SHAPES))
 def test_noalloc_matches_the_context_entry_point(gpu, shape):
-    sh = k3moe.TINY if shape == "tiny" else k3moe.K2
+    sh = _SHAPES[shape]
     say(f"case: k3g_moe_noalloc vs k3g_moe, {sh.name}, T=4 then T=2")
     layer = k3moe.SynthLayer(sh, seed=31, layout="tiled")
     L = layer.dev_tiled
