@@ -810,8 +810,8 @@ static int routed_staged(K3gCtx *c, const K3gLayer *L, const float *z, int lat, 
     const int maxU = P < E ? P : E;
     if (a.fmt == K3K_MXFP4 && lat % 32 == 0 && L->inter % 32 == 0) {
         /* On the matrix cores wherever a row is whole blocks of 32: faster at every size tried
-         * (gate/up and down, us: 1 token of 1024 x 256 32 -> 24, of 7168 x 2048 186 -> 55; 4
-         * tokens of 7168 x 2048 1194 -> 159, 512 tokens 34020 -> 3090). The row-by-row kernels
+         * (gate/up and down, us: 1 token of 1024 x 256 32 -> 24, of 7168 x 2048 186 -> 53; 4
+         * tokens of 7168 x 2048 1194 -> 157, 512 tokens 34020 -> 3200). The row-by-row kernels
          * below take rows that end in half a block. */
         K3kRows r;
         memset(&r, 0, sizeof r);

@@ -19,7 +19,7 @@
  * two intervals ahead, in units swizzled by the row so that the operand reads meet no bank
  * conflict; the rows' scale bytes follow per 512 columns, as the aligned words that hold them.
  * Two workgroups of 4 waves per CU keep 64 KB of weights in flight. Measured, 28 experts of 4
- * tokens (7168 x 2048, 655 MB): gate/up 753 -> 98 us (4.5 TB/s), down 441 -> 61 us (3.6 TB/s)
+ * tokens (7168 x 2048, 655 MB): gate/up 753 -> 95 us (4.6 TB/s), down 441 -> 62 us (3.5 TB/s)
  * against a wave per row tile with fp32 multiply-adds, which decodes every weight once per
  * four tokens; error against 64 bits 3.2e-7 -> 1.6e-7.
  *
@@ -53,33 +53,31 @@ k_rows_x(const float *__restrict__ x, int T, int K, uint8_t *__restrict__ o)
     if (b >= (long long)T * nbk) return;
     const int t = (int)(b / nbk), k = (int)(b - (long long)t * nbk);
     gm_v16f ev = {}, od = {};
-    const float4 *src = (const float4 *)(x + (size_t)t * K + 32 * k);
     if (32 * k < K) {
+        const float4 *src = (const float4 *)(x + (size_t)t * K + 32 * k);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const float4 v = src[i];
             ev[2 * i] = v.x; od[2 * i] = v.y; ev[2 * i + 1] = v.z; od[2 * i + 1] = v.w;
         }
     }
+    const gm_v16f ev0 = ev, od0 = od;
     uint32_t d[6 * RW_NP];
     uint8_t s[RW_NP];
-    bool bad = gm_bad(ev, od);
     gm_pieces<RW_NP>(ev, od, d, s);
     constexpr int LP = 6 * (RW_NP - 1);
     gm_less(ev, od, gm_v6u{d[LP], d[LP + 1], d[LP + 2], d[LP + 3], d[LP + 4], d[LP + 5]}, s[RW_NP - 1]);
-    if (32 * k < K) {
-        int n = 0, left = 0;
-        auto look = [&](float v, float r) {
-            n += v != 0.0f;
-            left += fabsf(r) > 0x1p-22f * fabsf(v);
-        };
+    int n = 0, left = 0;
+    auto look = [&](float v, float r) {
+        n += v != 0.0f;
+        left += fabsf(r) > 0x1p-22f * fabsf(v);
+    };
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float4 v = src[i];
-            look(v.x, ev[2 * i]); look(v.y, od[2 * i]); look(v.z, ev[2 * i + 1]); look(v.w, od[2 * i + 1]);
-        }
-        bad |= left > 0 && left >= n - 1 - n / 8;
+    for (int i = 0; i < 16; ++i) {
+        look(ev0[i], ev[i]);
+        look(od0[i], od[i]);
     }
+    const bool bad = gm_bad(ev0, od0) || (left > 0 && left >= n - 1 - n / 8);
     uint8_t *q = o + ((size_t)t * (nbk / 4) + (k >> 2)) * RW_STEP;
 #pragma unroll
     for (int p = 0; p < RW_NP; ++p) {
