@@ -92,7 +92,8 @@ typedef unsigned int k3v4u __attribute__((ext_vector_type(4)));
 #define K3_EVLINES (NREP * REP_STRIDE)
 /* Ticket counters for T > 1, 64 waves of one XCD each on 4096. Measured, K2 layer, taking the next
  * ticket so and one K slice a routed down ticket: 2 / 3 / 4 tokens 122 / 176 / 220 -> 114 / 159 / 198
- * us. At one token the launch is two and a half tickets a wave, and the count's round trip costs
+ * us. With the selections per token (whole calls, 2 / 3 / 4 tokens): K3 248 / 323 / 384 -> 227 / 294 /
+ * 351, 2048 x 1408 with 64 experts, top 6, 41.2 / 51.2 / 66.8 -> 38.7 / 45.8 / 54.1. At one token the launch is two and a half tickets a wave, and the count's round trip costs
  * what the balance gives (71 -> 72, K3 159 -> 164 us). */
 #define K3_STRIPES 64
 
@@ -146,8 +147,8 @@ __host__ __device__ inline K3Geo k3_geo(int T, int d, int E, int k, int I, int S
     g.KSR = ksr < g.nRc ? ksr : g.nRc;
     /* a routed down ticket takes the whole width where that leaves at least half of the 4096 waves
      * one (K2 and K3 from 2 tokens on, where unsliced is faster, K3_STRIPES); one token's, and few
-     * tokens' of a small layer, are sliced: 2048 x 1408, top 6, at 2 / 3 / 4 tokens unsliced 44.0 /
-     * 55.2 / 65.9 us, sliced 43.1 / 53.0 / 64.1 */
+     * tokens' of a small layer, are sliced: 2048 x 1408, top 6, at 2 / 3 / 4 tokens unsliced 38.7 /
+     * 45.8 / 54.1 us, sliced 38.4 / 44.1 / 53.5 */
     g.KSDN = T > 1 && T * k * (g.Dout / 32) >= 2048 ? 1 : ksdn < g.nQi ? ksdn : g.nQi;
     g.KSLD = g.lat ? (K3G_KS_LD < g.nCd ? K3G_KS_LD : g.nCd) : 0;
     g.KSLU = g.lat ? (K3G_KS_LU < g.nCL ? K3G_KS_LU : g.nCL) : 0;
@@ -1582,8 +1583,8 @@ k_decode_fused(K3kDecode a)
     if (threadIdx.x == 0) rl.count = 0;
     __syncthreads();
     /* (the router's and the selection's use of the workgroup's LDS needs their tickets in the
-     * first round; by the instance, so that one token's tickets carry no count: the engine's call of
-     * a 2048 x 1408 layer at one token 49.5 -> 47.8 us) */
+     * first round; by the instance, so that one token's tickets carry no count: a 2048 x 1408 layer at
+     * one token 33.3 -> 33.2 us, K3 156.2 -> 155.5) */
     const int stripe = w % K3_STRIPES;
     int *count = NT > 1 && W % K3_STRIPES == 0 && G.nX + G.nR + G.nS <= W
                      ? k3d_line(a.sync, G.lTK + stripe) : nullptr;
