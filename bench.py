@@ -43,7 +43,7 @@ B_GATEUP_EXPERT = 2 * (I * D // 2 + I * D // 32)   # w1 + w3 of one expert
 # --pmc runs (FETCH_SIZE x 1.9997 + WRITE_SIZE x 1.0, the factors that make a 256 MiB
 # device-to-device copy read 256 MiB); the run and the numbers are in
 # profiles/k_decode_fused_k2_decode.md. Re-measured whenever the kernel changes.
-TRAFFIC_FUSED = 302318946
+TRAFFIC_FUSED = 302284303
 # HBM bytes per launch of the routed gate/up GEMM (k_gemm6<0>) of the 4096-token Zipf(0.8)
 # prefill, the same way (FETCH_SIZE x 1.9997 + WRITE_SIZE, mean of 4 launches): 7.672 GB read +
 # 0.223 GB written; profiles/k_gemm6_k2_k3.md.
